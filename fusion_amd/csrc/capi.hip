@@ -1274,7 +1274,7 @@ static fu_status run_frame_plain(fu_system* sys, const uint16_t* depth, const ui
                 LAUNCHCHK();
                 HIPCHK(hipMemcpyAsync(&h, t->st, sizeof(h), hipMemcpyDeviceToHost, s));
                 HIPCHK(hipStreamSynchronize(s));
-                float sums[32], rsums[32];
+                float sums[29], rsums[29];
                 memcpy(sums, h.sums, sizeof(sums));
                 memcpy(rsums, h.rgb_sums, sizeof(rsums));
                 const int fin = (l == last_level && j == p.iters[l] - 1);
@@ -1659,11 +1659,11 @@ int batch_layout(BatchLaunch& b, const SessDesc* h, BatchTiling t, int level, in
                 for (int l = 0; l < 3; ++l) cnt += ((d.lc[l] + 15) / 16) * ((d.lr[l] + 15) / 16);
                 gx = cnt;
                 break;
-            case BT_ICP: gx = cnt = d.icp_blocks[level]; break;
+            case BT_ICP: gx = cnt = d.icp_blocks[level] * fixed; break;
             case BT_ONE: gx = cnt = 1; break;
             case BT_FIXED: gx = cnt = fixed; break;
             case BT_ZTILES: gx = cnt = (d.zr.zcols * d.zr.zrows + 255) / 256; break;
-            case BT_ICP_PAIRS: gx = cnt = (d.icp_blocks[level] + 1) / 2; break;
+            case BT_ICP_PAIRS: gx = cnt = (d.icp_blocks[level] + 1) / 2 * fixed; break;
         }
         b.pre[i] = total;
         b.gx[i] = (unsigned short)gx;

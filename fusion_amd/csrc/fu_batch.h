@@ -132,11 +132,11 @@ __device__ __forceinline__ bool slot_first(const BatchLaunch& b, int s) { return
 enum BatchTiling : int {
     BT_TILES = 0,   // 16x16 tiles of the level-`level` image
     BT_PYR3 = 1,    // 16x16 tiles of all three levels, level 0 first
-    BT_ICP = 2,     // icp_blocks[level] work-groups
+    BT_ICP = 2,     // icp_blocks[level] * fixed work-groups
     BT_ONE = 3,     // one work-group per session
     BT_FIXED = 4,   // a fixed number of work-groups per session (grid-stride bodies)
     BT_ZTILES = 5,  // 256-thread groups over the z-range tiles
-    BT_ICP_PAIRS = 7,  // (icp_blocks[level] + 1) / 2 work-groups (kRgbPixels chunks)
+    BT_ICP_PAIRS = 7,  // (icp_blocks[level] + 1) / 2 * fixed work-groups (kRgbPixels chunks)
 };
 // fills b.pre, b.gx and b.uniform for one launch; returns the total work-group count
 int batch_layout(BatchLaunch& b, const SessDesc* h, BatchTiling t, int level, int fixed);

@@ -41,7 +41,9 @@ struct TrackState {
     int count;
     int status;
     int iters_done;
-    float sums[32];
+    float sums[31];
+    // partial rows of the running ICP reduction that are in place (0 between launches)
+    unsigned arrived;
     // photometric term of the last iteration (RGBStep): the weighted-row sums, the residual
     // pass's {count, sum diff^2} and sigma, and sqrt(sum r^2) / count with its count
     float rgb_sums[32];
@@ -152,7 +154,6 @@ struct MeshOut {
     unsigned max_tri;
 };
 
-// work-group sizes of the ICP reduction (one pixel per lane) and of its one-group final sum
 // most work-groups of an ICP reduction (larger frames loop over pixel chunks per lane)
 constexpr int kIcpMaxBlocks = 4096;
 constexpr int kIcpThreads = 1024;
@@ -161,7 +162,6 @@ constexpr int kIcpThreads = 1024;
 constexpr int kIcpLanePixels = 2;
 constexpr int kIcpPixels = kIcpLanePixels * kIcpThreads;
 constexpr int kRgbPixels = 2 * kIcpThreads;
-constexpr int kIcpFinalThreads = 256;
 
 // Inputs of the photometric term at one level (RGBReduction, Reduction.cu:377-407)
 // The pose-independent tests of FindCorresp (Reduction.cu:420-433: the 5-pixel margin, a

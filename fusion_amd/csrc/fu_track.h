@@ -258,6 +258,7 @@ FU_HD void icp_update(TrackState* st, const float* sums, const float* rgb, int m
 // reference's graph-matching Relocalise does).  A tracker that is not lost starts ComputeSE3 (Tracking.cc:305-314): last
 // pose = tracked pose of the previous frame, initial guess = last pose, delta = identity.
 FU_HD void frame_begin(TrackState* st) {
+    st->arrived = 0;
     if (st->sm_state == -1) {
         st->status = st->reloc ? TS_RELOC : TS_LOST;
         FU_UNROLL for (int i = 0; i < 16; ++i) st->next_pose[i] = st->last_pose[i];
