@@ -123,7 +123,7 @@ extern "C" size_t fu_map_bytes(const fu_map_params* p) {
     const size_t ne = (size_t)p->num_buckets + p->num_excess;
     const size_t chunks = (p->num_blocks + 2047) / 2048;
     return ne * sizeof(HEntry) + 64 + (size_t)p->num_blocks * (8 + 4 + 8 + 4) + newset_size(p) * 8ull +
-           (size_t)p->max_new_blocks * 12 + chunks * 4 + occ_bits(p) / 8 +
+           (size_t)p->max_new_blocks * 12 + (3 * chunks + 1) * 4 + occ_bits(p) / 8 +
            (size_t)p->num_blocks * vf_block_bytes((int)p->voxel_format);
 }
 
@@ -177,7 +177,7 @@ extern "C" fu_status fu_map_create(const fu_map_params* p, fu_map** out) {
         (st = dalloc(m, &v.visible, p->num_blocks)) || (st = dalloc(m, &v.visible_key, p->num_blocks)) ||
         (st = dalloc(m, &v.newset, ns)) ||
         (st = dalloc(m, &v.newkeys, p->max_new_blocks)) || (st = dalloc(m, &v.newslot, p->max_new_blocks)) ||
-        (st = dalloc(m, &m->mesh_counts, p->num_blocks)) || (st = dalloc(m, &m->mesh_chunk, chunks)) ||
+        (st = dalloc(m, &m->mesh_counts, p->num_blocks)) || (st = dalloc(m, &m->mesh_chunk, 3 * chunks + 1)) ||
         (st = dalloc(m, &v.occ, occ_bits(p) / 32)) ||
         (st = dalloc(m, &v.pool, (size_t)p->num_blocks * vf_block_bytes((int)p->voxel_format)))) {
         fu_map_destroy(m);

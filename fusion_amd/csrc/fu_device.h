@@ -37,7 +37,7 @@ enum Counter : int {
     C_FLAGS = 4,    // sticky overflow flags (FU_FLAG_*)
     C_RENDER = 5,   // rendering fragments of the last z-range pass
     C_TRI = 6,      // triangles of the last mesh pass
-    C_DONE = 7,     // work-group completion counter (last-group pattern), left at 0
+    C_DONE = 7,     // chunks of the running mesh scan whose sums are in place
     C_OCC = 8,      // occupied blocks seen by the last mesh pass
     C_SPARE = 9,
     C_COUNT = 16
