@@ -106,12 +106,10 @@ extern "C" void fu_map_params_default(fu_map_params* p) {
     p->max_new_blocks = 1u << 18;
 }
 
-// occupancy bitmap: about 8 bits per pool block, 2^20..2^25 bits
-static unsigned occ_bits(const fu_map_params* p) {
-    unsigned n = 1u << 20;
-    while (n < (1u << 25) && (unsigned long long)n < 8ull * p->num_blocks) n <<= 1;
-    return n;
-}
+// cells per axis of the block grid: 2^7 (16 MB) covers a camera's surroundings (5 m at 5 mm
+// voxels) without two blocks in a cell; maps of few blocks take less
+static unsigned grid_bits(const fu_map_params* p) { return p->num_blocks > (1u << 14) ? 7 : p->num_blocks > (1u << 11) ? 6 : 5; }
+static size_t grid_cells(const fu_map_params* p) { return (size_t)1 << (3 * grid_bits(p)); }
 
 static unsigned newset_size(const fu_map_params* p) {
     unsigned n = 1024;
@@ -123,7 +121,7 @@ extern "C" size_t fu_map_bytes(const fu_map_params* p) {
     const size_t ne = (size_t)p->num_buckets + p->num_excess;
     const size_t chunks = (p->num_blocks + 2047) / 2048;
     return ne * sizeof(HEntry) + 64 + (size_t)p->num_blocks * (8 + 4 + 8 + 4) + newset_size(p) * 8ull +
-           (size_t)p->max_new_blocks * 12 + (3 * chunks + 1) * 4 + occ_bits(p) / 8 +
+           (size_t)p->max_new_blocks * 12 + (3 * chunks + 1) * 4 + grid_cells(p) * sizeof(uint2) +
            (size_t)p->num_blocks * vf_block_bytes((int)p->voxel_format);
 }
 
@@ -178,7 +176,7 @@ extern "C" fu_status fu_map_create(const fu_map_params* p, fu_map** out) {
         (st = dalloc(m, &v.newset, ns)) ||
         (st = dalloc(m, &v.newkeys, p->max_new_blocks)) || (st = dalloc(m, &v.newslot, p->max_new_blocks)) ||
         (st = dalloc(m, &m->mesh_counts, p->num_blocks)) || (st = dalloc(m, &m->mesh_chunk, 3 * chunks + 1)) ||
-        (st = dalloc(m, &v.occ, occ_bits(p) / 32)) ||
+        (st = dalloc(m, &v.grid, grid_cells(p))) ||
         (st = dalloc(m, &v.pool, (size_t)p->num_blocks * vf_block_bytes((int)p->voxel_format)))) {
         fu_map_destroy(m);
         return st;
@@ -187,8 +185,7 @@ extern "C" fu_status fu_map_create(const fu_map_params* p, fu_map** out) {
     v.num_excess = p->num_excess;
     v.num_blocks = p->num_blocks;
     v.newset_mask = ns - 1;
-    v.occ_mask = occ_bits(p) - 1;
-    v.occ_shift = 32u - (unsigned)__builtin_ctz(occ_bits(p));
+    v.grid_bits = grid_bits(p);
     v.bucket_mask = (p->num_buckets & (p->num_buckets - 1)) == 0 ? p->num_buckets - 1 : 0u;
     v.max_new = p->max_new_blocks;
     v.max_weight = p->max_weight;

@@ -74,8 +74,8 @@ struct MapView {
     unsigned long long* newkeys;  // [max_new]
     unsigned* newslot;          // [max_new]
     unsigned char* pool;        // voxel blocks
-    unsigned* occ;              // occupancy bitmap, one bit per hash of every allocated key
-    unsigned occ_mask, occ_shift;
+    uint2* grid;                // block grid: (pool index, tag) by the low coordinate bits, see grid_find
+    unsigned grid_bits;         // 2^grid_bits cells per axis
     unsigned bucket_mask;       // num_buckets - 1 when it is a power of two, else 0
     unsigned num_buckets, num_excess, num_blocks, newset_mask, max_new;
     unsigned max_weight;
@@ -166,28 +166,55 @@ FU_HD unsigned long long mix64(unsigned long long k) {
     return k;
 }
 
-// A clear occupancy bit proves the key is not allocated (bits are set for every allocated
-// key; collisions only cost a probe).  The bitmap is small enough to stay in L2, so rays
-// stepping through empty space skip the dependent hash-table load.  Bit index: the top bits
-// of a multiplicative scramble of the 32-bit block hash.
-FU_HD unsigned occ_bit(const MapView& m, uint32_t raw) { return (raw * 0x9E3779B1u) >> m.occ_shift; }
-__device__ __forceinline__ bool maybe_allocated(const MapView& m, uint32_t raw) {
-    const unsigned h = occ_bit(m, raw);
-    return (FU_G(const unsigned, m.occ)[h >> 5] >> (h & 31)) & 1u;
+// ---- block grid --------------------------------------------------------------------------
+// A direct-mapped table of the allocated blocks by the low grid_bits of each block coordinate,
+// beside the hash table: a cell holds the pool index and the ten coordinate bits per axis above
+// those of the first block allocated in it (blocks are never freed between resets).  A lookup is
+// one 8-byte load: an empty cell proves that no block of its congruence class is allocated, an
+// equal tag gives the block, and only another block in the cell (one a whole grid away: 5 m at
+// 5 mm voxels and 2^7 cells) sends the lookup to the hash table, as do coordinates outside
+// +-2^(grid_bits + 9).  Neighbouring blocks along x share cache lines, and the index and tag are
+// shifts where the hash takes three 32-bit multiplications; the rays' and samples' lookups had
+// cost an occupancy bitmap load and then the hash entry's.
+constexpr unsigned kNoBlock = 0xFFFFFFFFu;  // pool index and tag of an empty cell
+FU_HD bool in_grid(const MapView& m, i3 b) {
+    const unsigned half = 512u << m.grid_bits;
+    return ((((unsigned)b.x + half) | ((unsigned)b.y + half) | ((unsigned)b.z + half)) >> (m.grid_bits + 10)) == 0u;
+}
+// the parts of a coordinate: cell index along its axis and tag, shifted into place (axis 0..2)
+FU_HD unsigned grid_cell(const MapView& m, int c, int axis) {
+    return ((unsigned)c & ((1u << m.grid_bits) - 1u)) << (m.grid_bits * axis);
+}
+FU_HD unsigned grid_tag(const MapView& m, int c, int axis) {
+    return (((unsigned)c >> m.grid_bits) & 1023u) << (10 * axis);
+}
+FU_HD unsigned grid_index(const MapView& m, i3 b) { return grid_cell(m, b.x, 0) | grid_cell(m, b.y, 1) | grid_cell(m, b.z, 2); }
+FU_HD unsigned grid_tag3(const MapView& m, i3 b) { return grid_tag(m, b.x, 0) | grid_tag(m, b.y, 1) | grid_tag(m, b.z, 2); }
+// enters block bp (pool index heap) unless its cell is taken; atomic against other inserts
+__device__ __forceinline__ void grid_insert(const MapView& m, i3 bp, unsigned heap) {
+    if (!in_grid(m, bp)) return;
+    const unsigned long long e = (unsigned long long)heap | ((unsigned long long)grid_tag3(m, bp) << 32);
+    atomicCAS(reinterpret_cast<unsigned long long*>(m.grid + grid_index(m, bp)), ~0ull, e);
 }
 
-// heap index of block `bp`, or -1 if it is not allocated
-__device__ __forceinline__ int find_block(const MapView& m, i3 bp) {
+// heap index of block `bp` by the hash table, or -1 if it is not allocated
+__device__ __forceinline__ int hash_find(const MapView& m, i3 bp) {
     if (!key_in_range(bp)) return -1;
-    const uint32_t raw = block_hash_raw(bp);
-    if (!maybe_allocated(m, raw)) return -1;
     const unsigned long long key = pack_key(bp);
-    HEntry h = load_entry(&m.entries[bucket_of(raw, m.num_buckets, m.bucket_mask)]);
+    HEntry h = load_entry(&m.entries[bucket_of(block_hash_raw(bp), m.num_buckets, m.bucket_mask)]);
     while (true) {
         if (h.key == key && h.ptr >= 0) return h.ptr >> 9;
         if (h.next <= 0) return -1;
         h = load_entry(&m.entries[m.num_buckets + h.next - 1]);
     }
+}
+// heap index of block `bp`, or -1 if it is not allocated
+__device__ __forceinline__ int find_block(const MapView& m, i3 bp) {
+    if (in_grid(m, bp)) {
+        const uint2 e = FU_G(const uint2, m.grid)[grid_index(m, bp)];
+        if (e.y == grid_tag3(m, bp) || e.x == kNoBlock) return (int)e.x;
+    }
+    return hash_find(m, bp);
 }
 
 // ---- wave64 helpers -------------------------------------------------------------------

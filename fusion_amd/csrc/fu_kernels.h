@@ -219,6 +219,7 @@ void launch_image_commit(const TrackState* st, const unsigned char* const src[3]
                          const int n[3], hipStream_t s);
 // map.hip
 void launch_reset_map(const MapView& m, hipStream_t s);
+void launch_grid_fill(const MapView& m, unsigned n, hipStream_t s);  // from the first n block keys
 void launch_begin_pass(const MapView& m, int which, hipStream_t s);
 void launch_alloc(const MapView& m, const FuseArgs& a, hipStream_t s);
 void launch_visible(const MapView& m, const VisArgs& v, hipStream_t s);

@@ -48,8 +48,18 @@ void launch_reset_map(const MapView& m, hipStream_t s) {
     hipLaunchKernelGGL(k_reset_entries, dim3(2048), dim3(256), 0, s, m.entries, ne);
     hipLaunchKernelGGL(k_fill_u64, dim3(1024), dim3(256), 0, s, m.block_key, kEmptyKey, m.num_blocks);
     hipLaunchKernelGGL(k_fill_u64, dim3(1024), dim3(256), 0, s, m.newset, kEmptyKey, m.newset_mask + 1);
-    hipLaunchKernelGGL(k_zero_u32, dim3(1024), dim3(256), 0, s, m.occ, (m.occ_mask + 1) / 32);
+    hipLaunchKernelGGL(k_fill_u64, dim3(1024), dim3(256), 0, s, reinterpret_cast<unsigned long long*>(m.grid), ~0ull,
+                       1u << (3 * m.grid_bits));
     hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, s, m.ctr, (unsigned)C_COUNT);
+}
+
+// the block grid of a map whose keys came from a snapshot (the grid cleared)
+__global__ __launch_bounds__(256) void k_grid_fill(MapView m, unsigned n) {
+    for (unsigned i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+        if (m.block_key[i] != kEmptyKey) grid_insert(m, unpack_key(m.block_key[i]), i);
+}
+void launch_grid_fill(const MapView& m, unsigned n, hipStream_t s) {
+    hipLaunchKernelGGL(k_grid_fill, dim3(1024), dim3(256), 0, s, m, n);
 }
 
 // per-frame counters: the new-key count and the visible count start at zero
@@ -245,10 +255,7 @@ __device__ __forceinline__ void alloc_b_body(WG g, const MapView& m, const Track
                     }
                 }
                 m.block_key[heap] = ok ? key : kEmptyKey;
-                if (ok) {
-                    const unsigned hb = occ_bit(m, block_hash_raw(bp));
-                    atomicOr(&m.occ[hb >> 5], 1u << (hb & 31));
-                }
+                if (ok) grid_insert(m, bp, (unsigned)heap);
             }
         }
         heap = __shfl(heap, 0);

@@ -288,17 +288,11 @@ fu_status parse_map(const fu_map_params& p, In& in, MapImage& img) {
     return FU_OK;
 }
 
-// the checked image onto the device: entries, keys, the occupancy bitmap (a function of the
-// keys), the pool (read again from the file) and the map-wide counters; the per-frame
+// the checked image onto the device: entries, keys, the block grid (a function of the keys),
+// the pool (read again from the file) and the map-wide counters; the per-frame
 // counters start at zero as after a reset
 fu_status commit_map(fu_map* m, FILE* f, const MapImage& img, hipStream_t s) {
     MapView& v = m->v;
-    std::vector<unsigned> occ((v.occ_mask + 1) / 32, 0u);
-    for (unsigned long long key : img.keys)
-        if (key != kEmptyKey) {
-            const unsigned hb = occ_bit(v, block_hash_raw(unpack_key(key)));
-            occ[hb >> 5] |= 1u << (hb & 31);
-        }
     Pinned buf;
     HIPOK(hipHostMalloc(&buf.p, kChunk, hipHostMallocDefault));
     if (fseeko(f, img.pool_off, SEEK_SET) != 0) return snapshot_error("cannot re-read the pool");
@@ -307,7 +301,11 @@ fu_status commit_map(fu_map* m, FILE* f, const MapImage& img, hipStream_t s) {
     HIPOK(hipStreamSynchronize(s));
     HIPOK(hipMemcpy(v.entries, img.ent.data(), img.ent.size() * sizeof(HEntry), hipMemcpyHostToDevice));
     if (img.n_alloc) HIPOK(hipMemcpy(v.block_key, img.keys.data(), img.n_alloc * 8ull, hipMemcpyHostToDevice));
-    HIPOK(hipMemcpy(v.occ, occ.data(), occ.size() * 4, hipMemcpyHostToDevice));
+    if (img.n_alloc) {
+        launch_grid_fill(v, img.n_alloc, s);
+        HIPOK(hipGetLastError());
+        HIPOK(hipStreamSynchronize(s));
+    }
     In in;
     in.f = f;
     if (!file_to_dev(in, v.pool, img.pool_bytes, buf)) {
