@@ -357,7 +357,6 @@ extern "C" fu_status fu_create_rendering_blocks(fu_map* m, float* zrange_min, fl
     int ov = n_visible == 0xffffffffu ? -1 : (int)(n_visible < m->p.num_blocks ? n_visible : m->p.num_blocks);
     const ZRangeArgs a =
         make_zr(m, zrange_min, zrange_max, zcols, zrows, depth_max, depth_min, posef_from(pose), nullptr, ov, fx, fy, cx, cy);
-    launch_begin_pass(m->v, 4, S(s));
     launch_zrange(m->v, a, S(s));
     LAUNCHCHK();
     if (n_fragments || rendered) {
@@ -1186,7 +1185,7 @@ static void queue_fuse_raycast(fu_system* sys, const uint8_t* rgb, hipStream_t s
     a.px = sys->fuse_px;
     a.prgb = sys->fuse_rgb;
     const VisArgs v = make_vis(m, dummy, st, p.cols, p.rows, p.fx, p.fy, p.cx, p.cy, m->p.depth_min, m->p.depth_max);
-    launch_begin_pass(m->v, 7, s);
+    launch_begin_pass(m->v, 3, s);
     launch_fuse_pack(a, s);
     launch_alloc(m->v, a, s);
     mark(sys, FU_STAGE_ALLOC + 1, s);
@@ -1296,7 +1295,7 @@ static fu_status run_frame_plain(fu_system* sys, const uint16_t* depth, const ui
     a.px = sys->fuse_px;
     a.prgb = sys->fuse_rgb;
     const VisArgs v = make_vis(m, dummy, t->st, p.cols, p.rows, p.fx, p.fy, p.cx, p.cy, m->p.depth_min, m->p.depth_max);
-    launch_begin_pass(m->v, 7, s);
+    launch_begin_pass(m->v, 3, s);
     if (fuse) {
         launch_fuse_pack(a, s);
         launch_alloc(m->v, a, s);
@@ -1491,7 +1490,6 @@ static fu_status render_at(fu_system* sys, const double P[16], unsigned min_vis,
     if (nvis > 0) {
         const ZRangeArgs z = make_zr(m, b.zrange_min, b.zrange_max, b.zcols, b.zrows, m->p.depth_max, m->p.depth_min,
                                      pose, nullptr, -1, p.fx, p.fy, p.cx, p.cy);
-        launch_begin_pass(m->v, 4, s);
         launch_zrange(m->v, z, s);
         LAUNCHCHK();
         nfrag = read_ctr(m, C_RENDER, s, &st);

@@ -67,7 +67,6 @@ __device__ __forceinline__ void begin_pass_body(unsigned* ctr, int which) {
     if (threadIdx.x == 0) {
         if (which & 1) ctr[C_NEW] = 0;
         if (which & 2) ctr[C_VISIBLE] = 0;
-        if (which & 4) ctr[C_RENDER] = 0;
     }
 }
 __global__ void k_begin_pass(unsigned* ctr, int which) { begin_pass_body(ctr, which); }
@@ -118,81 +117,132 @@ __device__ __forceinline__ void claim_block(const MapView& m, bool want, unsigne
 // the group's rays share is probed and claimed once, by the lanes that scan the set
 // afterwards.  A block that finds no free LDS slot within kAllocProbes is probed and claimed
 // at once by its lane; the global per-pass set de-duplicates across lanes and groups.
-constexpr int kAllocSlots = 512;  // a 16x16 tile holds a few dozen blocks
+//
+// Bound by instruction issue: rays of a wave enter blocks at different steps, so the march only
+// queues them (at most kAllocQueue per lane, a word each) and the lanes then insert their first,
+// second, ... together.  A block is one word, its offset from the camera's block in ten bits per
+// axis (rays that leave +-500 blocks claim as they go); slots are an 8x8x8 neighbourhood, more
+// than a tile's rays span, and a lane reads a slot before it swaps, as lanes that swap at one
+// address wait for each other.  640x480 at 5 mm: 13.0 -> 10.5 us; eleven served sessions 82 -> 63 us.
+constexpr int kAllocSlots = 512;
 constexpr int kAllocProbes = 8;
 constexpr int kAllocThreads = 256;  // 16x16 pixels per group
+constexpr int kAllocQueue = 4;      // a band as long as a block enters at most four
+constexpr unsigned kNoOffset = 0xFFFFFFFFu;
 static_assert(kAllocSlots % kAllocThreads == 0, "whole slot rows per lane");
 __device__ __forceinline__ void alloc_a_body(WG g, const MapView& m, const FuseArgs& p) {
-    __shared__ unsigned long long set[kAllocSlots];
+    __shared__ unsigned set[kAllocSlots];
+    __shared__ unsigned queue[kAllocQueue][kAllocThreads];
+    __shared__ unsigned nkeys;
     PoseF pose = p.pose;
     if (p.st && !(frame_fuses(p.st) && pose_from_state(p.st, pose))) return;  // uniform: the frame does not fuse
-    for (int i = threadIdx.x; i < kAllocSlots; i += blockDim.x) set[i] = kEmptyKey;
-    __syncthreads();
     const auto depth = FU_G(const float, p.depth);
     const int x = g.x * 16 + (threadIdx.x & 15);
     const int y = g.y * 16 + (threadIdx.x >> 4);
-    bool live = x < p.cols && y < p.rows;
+    const bool live = x < p.cols && y < p.rows;
+    const float z = live ? depth[y * p.cols + x] : fnan();
+    for (int i = threadIdx.x; i < kAllocSlots; i += kAllocThreads) set[i] = kNoOffset;
+    if (threadIdx.x == 0) nkeys = 0;
+    __syncthreads();
+    // offsets count from 512 blocks below the camera's
+    const i3 cam = voxel_to_block(f2i3(mul(pose.t, m.voxel_inv)));
+    const i3 base = mki3(cam.x - 512, cam.y - 512, cam.z - 512);
     f3 pt = mk3(0.f, 0.f, 0.f), dir = mk3(0.f, 0.f, 0.f);
     int nsteps = 0;
-    if (live) {
-        const float z = depth[y * p.cols + x];
-        if (!(isnanf_(z) || z < m.depth_min || z > m.depth_max)) {
-            const float thresh = m.trunc / 2.0f;
-            const float z_near = fminf(m.depth_max, z - thresh);
-            const float z_far = fminf(m.depth_max, z + thresh);
-            if (z_near < z_far) {
-                // unproject: Rview * (z(x-cx)/fx, z(y-cy)/fy, z) + tview, then to voxel units
-                f3 a = mk3(z_near * ((float)x - p.cx) * p.invfx, z_near * ((float)y - p.cy) * p.invfy, z_near);
-                f3 b = mk3(z_far * ((float)x - p.cx) * p.invfx, z_far * ((float)y - p.cy) * p.invfy, z_far);
-                a = mul(add(mv(pose.R, a), pose.t), m.voxel_inv);
-                b = mul(add(mv(pose.R, b), pose.t), m.voxel_inv);
-                dir = sub(b, a);
-                const float len = norm(dir);
-                nsteps = d2i(ceil(2.0 * (double)len));
-                dir = divs(dir, (float)(nsteps - 1));
-                pt = a;
+    bool near = false;  // the whole band lies within the offsets' range
+    if (!(isnanf_(z) || z < m.depth_min || z > m.depth_max)) {
+        const float thresh = m.trunc / 2.0f;
+        const float z_near = fminf(m.depth_max, z - thresh);
+        const float z_far = fminf(m.depth_max, z + thresh);
+        if (z_near < z_far) {
+            // unproject: Rview * (z(x-cx)/fx, z(y-cy)/fy, z) + tview, then to voxel units
+            f3 a = mk3(z_near * ((float)x - p.cx) * p.invfx, z_near * ((float)y - p.cy) * p.invfy, z_near);
+            f3 b = mk3(z_far * ((float)x - p.cx) * p.invfx, z_far * ((float)y - p.cy) * p.invfy, z_far);
+            a = mul(add(mv(pose.R, a), pose.t), m.voxel_inv);
+            b = mul(add(mv(pose.R, b), pose.t), m.voxel_inv);
+            dir = sub(b, a);
+            const float len = norm(dir);
+            nsteps = d2i(ceil(2.0 * (double)len));
+            dir = divs(dir, (float)(nsteps - 1));
+            pt = a;
+            // steps lie between the ends, but for rounding far below a block
+            auto inside = [&](f3 q) {
+                const i3 c = voxel_to_block(f2i3(q));
+                return (unsigned)(c.x - base.x - 12) < 1000u && (unsigned)(c.y - base.y - 12) < 1000u &&
+                       (unsigned)(c.z - base.z - 12) < 1000u;
+            };
+            near = inside(a) && inside(b);
+        }
+    }
+    if (!near) {
+        // one block after the other, claimed at once
+        i3 prev = mki3(0x7fffffff, 0, 0);
+        for (int i = 0; i < nsteps; ++i) {
+            const i3 b = voxel_to_block(f2i3(pt));
+            pt = add(pt, dir);
+            if (eqi(b, prev)) continue;
+            prev = b;
+            if (key_in_range(b))
+                claim_block(m, true, pack_key(b), b);
+            else
+                atomicOr(&m.ctr[C_FLAGS], (unsigned)FLAG_COORD_RANGE);
+        }
+        nsteps = 0;
+    }
+    auto unpack = [&](unsigned o) {
+        return mki3(base.x + (int)(o & 1023u), base.y + (int)((o >> 10) & 1023u), base.z + (int)(o >> 20));
+    };
+    unsigned prev = kNoOffset;
+    for (int i = 0; __any(i < nsteps);) {
+        int n = 0;
+        for (; i < nsteps && n < kAllocQueue; ++i) {
+            const i3 b = voxel_to_block(f2i3(pt));
+            pt = add(pt, dir);
+            const unsigned o = (unsigned)(b.x - base.x) | (unsigned)(b.y - base.y) << 10 | (unsigned)(b.z - base.z) << 20;
+            if (o == prev) continue;
+            prev = o;
+            queue[n++][threadIdx.x] = o;
+        }
+#pragma unroll 1
+        for (int k = 0; __any(k < n); ++k) {
+            if (k >= n) continue;
+            const unsigned o = queue[k][threadIdx.x];
+            unsigned h = (o & 7u) | ((o >> 10) & 7u) << 3 | ((o >> 20) & 7u) << 6;
+            bool done = false;
+            for (int probe = 0; probe < kAllocProbes && !done; ++probe) {
+                unsigned cur = *(volatile unsigned*)&set[h];
+                if (cur == kNoOffset) {
+                    cur = atomicCAS(&set[h], kNoOffset, o);
+                    done = cur == kNoOffset;
+                }
+                done = done || cur == o;
+                h = (h + 1) & (kAllocSlots - 1);
+            }
+            if (!done) {
+                const i3 b = unpack(o);
+                if (key_in_range(b)) claim_block(m, true, pack_key(b), b);
             }
         }
     }
-    i3 prev = mki3(0x7fffffff, 0, 0);
-    for (int i = 0; i < nsteps; ++i) {
-        const i3 b = voxel_to_block(f2i3(pt));
-        pt = add(pt, dir);
-        if (eqi(b, prev)) continue;
-        prev = b;
-        if (!key_in_range(b)) {
-            atomicOr(&m.ctr[C_FLAGS], (unsigned)FLAG_COORD_RANGE);
-            continue;
-        }
-        const unsigned long long key = pack_key(b);
-        unsigned h = (unsigned)mix64(key) & (kAllocSlots - 1);
-        bool done = false;
-        for (int probe = 0; probe < kAllocProbes && !done; ++probe) {
-            const unsigned long long old = atomicCAS(&set[h], kEmptyKey, key);
-            done = old == kEmptyKey || old == key;
-            h = (h + 1) & (kAllocSlots - 1);
-        }
-        if (!done) claim_block(m, true, key, b);
-    }
     __syncthreads();
-    // the group's keys (a few dozen in a 16x16 tile) move to the front of the set, so the
-    // table probes and claims run in as few wave passes as there are keys, not one per
+    // the group's blocks (a few dozen in a 16x16 tile) move to the front of the set, so the
+    // table probes and claims run in as few wave passes as there are blocks, not one per
     // occupied 64-slot row; the order of the claims does not matter
-    __shared__ unsigned nkeys;
-    unsigned long long held[kAllocSlots / kAllocThreads];
+    unsigned held[kAllocSlots / kAllocThreads];
 #pragma unroll
     for (int k = 0; k < kAllocSlots / kAllocThreads; ++k) held[k] = set[threadIdx.x + k * kAllocThreads];
-    if (threadIdx.x == 0) nkeys = 0;
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < kAllocSlots / kAllocThreads; ++k)
-        if (held[k] != kEmptyKey) set[atomicAdd(&nkeys, 1u)] = held[k];
+        if (held[k] != kNoOffset) set[atomicAdd(&nkeys, 1u)] = held[k];
     __syncthreads();
     const int n = (int)nkeys;  // uniform: every lane runs the same passes
-    for (int base = 0; base < n; base += kAllocThreads) {
-        const int i = base + (int)threadIdx.x;
-        const unsigned long long key = i < n ? set[i] : kEmptyKey;
-        claim_block(m, key != kEmptyKey, key, unpack_key(key));
+    for (int first = 0; first < n; first += kAllocThreads) {
+        const int i = first + (int)threadIdx.x;
+        const i3 b = unpack(i < n ? set[i] : 0u);
+        const bool in = key_in_range(b);
+        if (i < n && !in) atomicOr(&m.ctr[C_FLAGS], (unsigned)FLAG_COORD_RANGE);
+        claim_block(m, i < n && in, pack_key(b), b);
     }
 }
 __global__ __launch_bounds__(kAllocThreads) void k_alloc_pass_a(MapView m, FuseArgs p) { alloc_a_body(hw_wg(), m, p); }
@@ -555,7 +605,7 @@ void launch_integrate(const MapView& m, const FuseArgs& a, unsigned grid, hipStr
 // ------------------------------------------------------------------ batched launches
 // FuseMapColor for every session of a step: counters, allocation (both passes), visible
 // list and integration, each stage one launch over all sessions.
-__global__ void kb_begin_pass(BatchLaunch b) { begin_pass_body(b.desc[b.sess[blockIdx.x]].m.ctr, 7); }
+__global__ void kb_begin_pass(BatchLaunch b) { begin_pass_body(b.desc[b.sess[blockIdx.x]].m.ctr, 3); }
 
 __device__ __forceinline__ FuseArgs slot_fuse(const BatchLaunch& b, const SessDesc& d, int s) {
     FuseArgs a = d.fuse;

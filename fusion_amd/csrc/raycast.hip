@@ -18,7 +18,10 @@
 
 namespace fu {
 
-__device__ __forceinline__ void zrange_init_body(WG g, const TrackState* st, unsigned* zmin, unsigned* zmax, int n) {
+// the tile maps and the fragment counter at the start of a pass
+__device__ __forceinline__ void zrange_init_body(WG g, unsigned* ctr, const TrackState* st, unsigned* zmin, unsigned* zmax,
+                                                 int n) {
+    if (g.x == 0 && threadIdx.x == 0) FU_G(unsigned, ctr)[C_RENDER] = 0;
     if (st && !(FU_G(const TrackState, st)->gates & GATE_RENDER)) return;
     const unsigned hundred = __float_as_uint(100.0f);
     for (int i = g.x * blockDim.x + threadIdx.x; i < n; i += g.nx * blockDim.x) {
@@ -26,8 +29,8 @@ __device__ __forceinline__ void zrange_init_body(WG g, const TrackState* st, uns
         zmax[i] = 0u;
     }
 }
-__global__ void k_zrange_init(const TrackState* st, unsigned* zmin, unsigned* zmax, int n) {
-    zrange_init_body(hw_wg(), st, zmin, zmax, n);
+__global__ void k_zrange_init(unsigned* ctr, const TrackState* st, unsigned* zmin, unsigned* zmax, int n) {
+    zrange_init_body(hw_wg(), ctr, st, zmin, zmax, n);
 }
 
 // exclusive prefix sum of `v` over the lanes of a wave, and the wave total in `total`
@@ -47,7 +50,10 @@ __device__ __forceinline__ unsigned wave_exclusive_scan(unsigned v, unsigned& to
 // which is flushed into the global maps once, only where it changed.  Min and max are exact
 // and order-free, so the maps are the same as with direct global atomics.
 constexpr int kZTilesLds = 6144;  // 48 KB of LDS for both maps; 640x480 needs 4800 tiles
-constexpr int kProjectGroups = 16;  // work-groups per session with LDS tile maps
+// work-groups per session with LDS tile maps, and their lanes: clearing and flushing the maps is
+// most of a group's time, so it has many lanes (16 groups of 256 took 13.0 us at 640x480)
+constexpr int kProjectGroups = 16;
+constexpr int kProjectLanes = 1024;
 
 template <bool kLds>
 __device__ __forceinline__ void project_body(WG g, const MapView& m, const ZRangeArgs& a) {
@@ -146,15 +152,15 @@ __device__ __forceinline__ void project_body(WG g, const MapView& m, const ZRang
     }
 }
 template <bool kLds>
-__global__ __launch_bounds__(256) void k_project_blocks(MapView m, ZRangeArgs a) {
+__global__ __launch_bounds__(kLds ? kProjectLanes : 256) void k_project_blocks(MapView m, ZRangeArgs a) {
     project_body<kLds>(hw_wg(), m, a);
 }
 
 void launch_zrange(const MapView& m, const ZRangeArgs& a, hipStream_t s) {
     const int n = a.zcols * a.zrows;
-    hipLaunchKernelGGL(k_zrange_init, dim3((n + 255) / 256), dim3(256), 0, s, a.st, a.zmin, a.zmax, n);
+    hipLaunchKernelGGL(k_zrange_init, dim3((n + 255) / 256), dim3(256), 0, s, m.ctr, a.st, a.zmin, a.zmax, n);
     if (n <= kZTilesLds)
-        hipLaunchKernelGGL(k_project_blocks<true>, dim3(kProjectGroups), dim3(256), 0, s, m, a);
+        hipLaunchKernelGGL(k_project_blocks<true>, dim3(kProjectGroups), dim3(kProjectLanes), 0, s, m, a);
     else
         hipLaunchKernelGGL(k_project_blocks<false>, dim3(512), dim3(256), 0, s, m, a);
 }
@@ -481,10 +487,10 @@ __global__ void kb_zrange_init(BatchLaunch b) {
     WG g;
     const int s = batch_slot(b, blockIdx.x, g);
     const SessDesc& d = b.desc[b.sess[s]];
-    zrange_init_body(g, d.st, d.zr.zmin, d.zr.zmax, d.zr.zcols * d.zr.zrows);
+    zrange_init_body(g, d.m.ctr, d.st, d.zr.zmin, d.zr.zmax, d.zr.zcols * d.zr.zrows);
 }
 template <bool kLds>
-__global__ __launch_bounds__(256) void kb_project(BatchLaunch b) {
+__global__ __launch_bounds__(kLds ? kProjectLanes : 256) void kb_project(BatchLaunch b) {
     WG g;
     const int s = batch_slot(b, blockIdx.x, g);
     const SessDesc& d = b.desc[b.sess[s]];
@@ -505,7 +511,7 @@ void launch_b_zrange(BatchLaunch& b, const SessDesc* h, hipStream_t s) {
     for (int i = 0; i < b.n; ++i) lds = lds && h[b.sess[i]].zr.zcols * h[b.sess[i]].zr.zrows <= kZTilesLds;
     if (lds) {
         grid = batch_layout(b, h, BT_FIXED, 0, kProjectGroups);
-        hipLaunchKernelGGL(kb_project<true>, dim3(grid), dim3(256), 0, s, b);
+        hipLaunchKernelGGL(kb_project<true>, dim3(grid), dim3(kProjectLanes), 0, s, b);
     } else {
         const int per = b.n > 0 ? 4096 / b.n : 64;
         grid = batch_layout(b, h, BT_FIXED, 0, per < 32 ? 32 : (per > 512 ? 512 : per));

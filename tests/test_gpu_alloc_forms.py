@@ -1,0 +1,56 @@
+"""Allocation's two ways of naming a ray's blocks (offsets from the camera's block, and whole keys
+for rays that leave their range) and its per-lane queue: the block set is the oracle's for bands of
+one to many blocks, near and beyond the offsets' range, and coordinates past the key range are
+flagged."""
+import numpy as np
+import pytest
+import torch
+
+from fusion_amd import api as A
+from oracle import binding as O
+from tests.helpers import rows_set
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("voxel,trunc,shift", [
+    (0.02, 3.0, 0.0),      # one or two blocks per ray
+    (0.005, 8.0, 0.0),     # a band as long as a block
+    (0.002, 100.0, 0.0),   # more blocks per ray than the queue holds
+    (0.0005, 40.0, 0.0),   # 500 blocks are 2 m: depths on both sides
+    (0.02, 3.0, -3000.0),  # negative block coordinates far from the origin
+])
+def test_block_set(gpu, voxel, trunc, shift):
+    cols, rows = 61, 47
+    K = (60.0, 60.0, 30.0, 23.0)
+    print("alloc: voxel %g trunc %g shift %g" % (voxel, trunc, shift), flush=True)
+    rng = np.random.default_rng(1)
+    depth = rng.uniform(0.5, 2.9, (rows // 4 + 1, cols // 4 + 1)).repeat(4, 0).repeat(4, 1)[:rows, :cols].astype(np.float32)
+    depth[rng.random(depth.shape) < 0.1] = np.nan
+    rgb = np.zeros((rows, cols, 3), np.uint8)
+    nm = np.full((rows, cols, 4), np.nan, np.float32)
+    pose = np.eye(4)
+    pose[:3, 3] = (shift, 0.3, -shift)
+    p = dict(num_buckets=1 << 17, num_excess=1 << 17, num_blocks=1 << 17, voxel_size=float(np.float32(voxel)),
+             trunc_dist=float(np.float32(voxel) * np.float32(trunc)))
+    o = O.Map(**p)
+    o.fuse_map_color(depth, rgb, nm, pose, K)
+    g = A.Mapping(**p, max_new_blocks=1 << 17)
+    g.FuseMapColor(torch.from_numpy(depth).cuda(), torch.from_numpy(rgb).cuda(), torch.from_numpy(nm).cuda(), pose, K)
+    ob = o.export_blocks()
+    assert len(ob) > 50 and rows_set(g.export_blocks()) == rows_set(ob)
+    assert g.stats()["flags"] == 0
+
+
+@pytest.mark.parametrize("blocks_from_limit", [2, -600])
+def test_key_range_is_flagged(gpu, blocks_from_limit):
+    """a camera at the key range's end (2^20 blocks): blocks past it are skipped and flagged, by
+    rays within the offsets' range and beyond it"""
+    voxel = 0.01
+    d = torch.full((16, 16), 1.0, dtype=torch.float32, device="cuda")
+    pose = np.eye(4)
+    pose[2, 3] = ((1 << 20) - blocks_from_limit) * 8 * voxel
+    g = A.Mapping(num_buckets=64, num_excess=64, num_blocks=64, voxel_size=voxel, trunc_dist=0.03, max_new_blocks=64)
+    g.FuseMapColor(d, torch.zeros((16, 16, 3), dtype=torch.uint8, device="cuda"),
+                   torch.full((16, 16, 4), float("nan"), device="cuda"), pose, (20.0, 20.0, 8.0, 8.0))
+    assert g.stats()["flags"] & 8 and g.stats()["n_allocated"] == 0
