@@ -27,11 +27,12 @@ def _addr(t):
 
 
 def _p(t):
-    return C.c_void_p(_addr(t)) if t is not None else None
+    return _addr(t) if t is not None else None
 
 
 def _s():
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """the current stream's handle (torch's raw getter: a Stream object costs more than a launch)"""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _dev():
@@ -43,14 +44,11 @@ def _dev():
 def pose_f(pose):
     """Frame::GpuRotation/GpuInvRotation/GpuTranslation (Core/Frame.cc:275-294)."""
     pose = np.asarray(pose, dtype=np.float64).reshape(4, 4)
-    p = N.PoseF()
-    R = pose[:3, :3]
-    for i in range(9):
-        p.R[i] = float(np.float32(R.flat[i]))
-        p.Rinv[i] = float(np.float32(R.T.flat[i]))
-    for i in range(3):
-        p.t[i] = float(np.float32(pose[i, 3]))
-    return p
+    v = np.empty(21, np.float32)  # R, its transpose, t, each rounded to float32
+    v[:9].reshape(3, 3)[:] = pose[:3, :3]
+    v[9:18].reshape(3, 3)[:] = pose[:3, :3].T
+    v[18:] = pose[:3, 3]
+    return N.PoseF.from_buffer_copy(v)
 
 
 def level_k(K, level):
@@ -109,7 +107,7 @@ def ICPStep(next_vmap, last_vmap, next_nmap, last_nmap, pose_curr, pose_last, K)
     check(N.lib().fu_icp_step(_p(next_vmap), _p(last_vmap), _p(next_nmap), _p(last_nmap), cols, rows,
                               pc.R, pc.t, pl.R, pl.Rinv, pl.t, K[0], K[1], K[2], K[3], res, A, b, _s()),
           "fu_icp_step")
-    return np.array(A[:]).reshape(6, 6), np.array(b[:]), np.array(res[:], dtype=np.float32)
+    return np.frombuffer(A).reshape(6, 6), np.frombuffer(b), np.frombuffer(res, dtype=np.float32)
 
 
 # --------------------------------------------------------------------- photometric term
@@ -151,7 +149,7 @@ def RGBStep(next_image, last_image, next_vmap, last_vmap, dIdx, dIdy, pose_curr,
     check(N.lib().fu_rgb_step(_p(next_image), _p(last_image), _p(next_vmap), _p(last_vmap), _p(dIdx), _p(dIdy),
                               cols, rows, pc.R, pc.Rinv, pl.R, pl.Rinv, pc.t, pl.t, K[0], K[1], K[2], K[3], res, A, b,
                               corr, _s()), "fu_rgb_step")
-    return (np.array(A[:]).reshape(6, 6), np.array(b[:]), np.array(res[:], dtype=np.float32),
+    return (np.frombuffer(A).reshape(6, 6), np.frombuffer(b), np.frombuffer(res, dtype=np.float32),
             (int(corr[0]), int(corr[1])))
 
 
@@ -339,10 +337,15 @@ class Tracker:
     def result(self):
         r = N.TrackResult()
         check(N.lib().fu_tracker_result(self.handle, C.byref(r), _s()), "fu_tracker_result")
-        return {"pose": np.array(r.pose[:]).reshape(4, 4), "last_pose": np.array(r.last_pose[:]).reshape(4, 4),
-                "x": np.array(r.x[:]), "A": np.array(r.A[:]).reshape(6, 6), "b": np.array(r.b[:]),
-                "icp_error": r.icp_error, "count": r.count, "status": r.status, "iterations": r.iterations,
-                "rgb_error": r.rgb_error, "rgb_count": r.rgb_count}
+        return _track_result(r)
+
+
+def _track_result(r):
+    """the fields of a fu_track_result, its arrays as views of the record"""
+    f = lambda a, *shape: np.frombuffer(a).reshape(shape)
+    return {"pose": f(r.pose, 4, 4), "last_pose": f(r.last_pose, 4, 4), "x": f(r.x, 6), "A": f(r.A, 6, 6), "b": f(r.b, 6),
+            "icp_error": r.icp_error, "count": r.count, "status": r.status, "iterations": r.iterations,
+            "rgb_error": r.rgb_error, "rgb_count": r.rgb_count}
 
 
 class IcpBatch:
@@ -371,7 +374,9 @@ class IcpBatch:
                                            arr(next_vmaps), arr(next_nmaps), arr(last_vmaps), arr(last_nmaps), Kf,
                                            (C.c_int32 * 3)(*iters), (C.c_int32 * 3)(*min_count), thresh, _s()),
               "fu_compute_se3_batch")
-        return [t.result() for t in trackers]
+        out = (N.TrackResult * n)()
+        check(N.lib().fu_icp_batch_results(self.handle, n, out, _s()), "fu_icp_batch_results")
+        return [_track_result(r) for r in out]
 
 
 # --------------------------------------------------------------------- system
@@ -439,7 +444,7 @@ class System:
                     raise N.FusionError("GrabImageHost: contiguous host tensors expected")
             elif not (isinstance(a, np.ndarray) and a.flags.c_contiguous):
                 raise N.FusionError("GrabImageHost: contiguous host arrays expected")
-        ptr = lambda a: C.c_void_p(a.data_ptr() if isinstance(a, torch.Tensor) else a.ctypes.data)
+        ptr = lambda a: a.data_ptr() if isinstance(a, torch.Tensor) else a.ctypes.data
         check(N.lib().fu_system_grab_image_host(self.handle, ptr(depth), ptr(rgb), _s()), "fu_system_grab_image_host")
 
     def relocalise(self, pose):
@@ -489,7 +494,7 @@ class System:
         r = N.FrameResult()
         check(N.lib().fu_system_result(self.handle, C.byref(r), _s()), "fu_system_result")
         d = {f: getattr(r, f) for f, _ in N.FrameResult._fields_ if f != "pose"}
-        d["pose"] = np.array(r.pose[:]).reshape(4, 4)
+        d["pose"] = np.frombuffer(r.pose).reshape(4, 4)
         return d
 
     def save(self, path):

@@ -16,6 +16,7 @@
 #include "fu_batch.h"
 #include "mc_tables.h"
 #include "fu_api.h"
+#include "fu_mail.h"
 
 using namespace fu;
 
@@ -166,6 +167,7 @@ extern "C" fu_status fu_map_create(const fu_map_params* p, fu_map** out) {
     if (st) return st;
     if ((st = ensure_tables())) return st;
     fu_map* m = new fu_map();
+    m->dev = current_device();
     m->p = *p;
     MapView& v = m->v;
     const unsigned ns = newset_size(p);
@@ -220,8 +222,7 @@ extern "C" fu_status fu_reset_map(fu_map* m, fu_stream s) {
 extern "C" fu_status fu_map_stats_get(fu_map* m, fu_map_stats* out, fu_stream s) {
     if (!m || !out) return set_err(FU_ERR_ARG, "null argument");
     unsigned c[C_COUNT];
-    HIPCHK(hipMemcpyAsync(c, m->v.ctr, sizeof(c), hipMemcpyDeviceToHost, S(s)));
-    HIPCHK(hipStreamSynchronize(S(s)));
+    HIPCHK(mail_read(m->dev, c, m->v.ctr, sizeof(c), S(s)));
     out->n_allocated = c[C_ALLOC] < m->p.num_blocks ? c[C_ALLOC] : m->p.num_blocks;
     out->n_excess = c[C_EXCESS] < m->p.num_excess ? c[C_EXCESS] : m->p.num_excess;
     out->n_visible = c[C_VISIBLE];
@@ -235,9 +236,7 @@ extern "C" fu_status fu_map_stats_get(fu_map* m, fu_map_stats* out, fu_stream s)
 
 static unsigned read_ctr(fu_map* m, int which, hipStream_t s, fu_status* st) {
     unsigned v = 0;
-    if (hipMemcpyAsync(&v, m->v.ctr + which, 4, hipMemcpyDeviceToHost, s) != hipSuccess ||
-        hipStreamSynchronize(s) != hipSuccess)
-        *st = set_err(FU_ERR_HIP, "counter read failed");
+    if (mail_read(m->dev, &v, m->v.ctr + which, 4, s) != hipSuccess) *st = set_err(FU_ERR_HIP, "counter read failed");
     return v;
 }
 
@@ -417,9 +416,9 @@ extern "C" fu_status fu_mesh_scene(fu_map* m, float* vertex, float* normal, uint
     o.max_tri = max_triangles;
     launch_mesh(m->v, o, m->mesh_counts, m->mesh_chunk, S(s));
     LAUNCHCHK();
-    fu_status st = FU_OK;
-    const unsigned tot = read_ctr(m, C_TRI, S(s), &st);
-    if (st) return st;
+    unsigned c[C_COUNT];
+    HIPCHK(mail_read(m->dev, c, m->v.ctr, sizeof(c), S(s)));
+    const unsigned tot = c[C_TRI];
     if (tot > max_triangles) {
         unsigned f = FU_FLAG_TRI_FULL;
         HIPCHK(hipMemcpy(&f, m->v.ctr + C_FLAGS, 4, hipMemcpyDeviceToHost));
@@ -427,8 +426,8 @@ extern "C" fu_status fu_mesh_scene(fu_map* m, float* vertex, float* normal, uint
         HIPCHK(hipMemcpy(m->v.ctr + C_FLAGS, &f, 4, hipMemcpyHostToDevice));
     }
     if (n_triangles) *n_triangles = tot < max_triangles ? tot : max_triangles;
-    if (n_occupied) *n_occupied = read_ctr(m, C_OCC, S(s), &st);
-    return st;
+    if (n_occupied) *n_occupied = c[C_OCC];
+    return FU_OK;
 }
 
 // ---- inspection
@@ -634,6 +633,7 @@ extern "C" fu_status fu_tracker_create(int cols, int rows, fu_tracker** out) {
     *out = nullptr;
     if (cols < 4 || rows < 4) return set_err(FU_ERR_ARG, "tracker size %dx%d too small", cols, rows);
     fu_tracker* t = new fu_tracker();
+    t->dev = current_device();
     t->cols = cols;
     t->rows = rows;
     size_t nlist = 0;
@@ -814,10 +814,47 @@ static void fill_result(const TrackState& h, fu_track_result* out) {
 extern "C" fu_status fu_tracker_result(fu_tracker* t, fu_track_result* out, fu_stream s) {
     if (!t || !out) return set_err(FU_ERR_ARG, "null argument");
     TrackState h;
-    HIPCHK(hipMemcpyAsync(&h, t->st, sizeof(h), hipMemcpyDeviceToHost, S(s)));
-    HIPCHK(hipStreamSynchronize(S(s)));
+    HIPCHK(mail_read(t->dev, &h, t->st, sizeof(h), S(s)));
     fill_result(h, out);
     return FU_OK;
+}
+
+// CreateMatrix<6,7> (Reduction.cu:6-16) and the residual of 29 sums
+static void icp_step_outputs(const float* sums, float residual[2], double A[36], double b[6]) {
+    int shift = 0;
+    for (int i = 0; i < 6; ++i)
+        for (int j = i; j < 7; ++j) {
+            const double v = (double)sums[shift++];
+            if (j == 6) {
+                if (b) b[i] = v;
+            } else if (A) {
+                A[j * 6 + i] = A[i * 6 + j] = v;
+            }
+        }
+    if (residual) {
+        residual[0] = sums[27];
+        residual[1] = sums[28];
+    }
+}
+static IcpArgs icp_step_args(TrackState* st, float* partials, const float* next_vmap, const float* last_vmap,
+                             const float* next_nmap, const float* last_nmap, int cols, int rows, float fx, float fy,
+                             float cx, float cy) {
+    IcpArgs a;
+    memset(&a, 0, sizeof(a));
+    a.vcurr = (const f4*)next_vmap;
+    a.ncurr = (const f4*)next_nmap;
+    a.vlast = (const f4*)last_vmap;
+    a.nlast = (const f4*)last_nmap;
+    a.cols = cols;
+    a.rows = rows;
+    a.fx = fx;
+    a.fy = fy;
+    a.cx = cx;
+    a.cy = cy;
+    a.st = st;
+    a.partials = partials;
+    a.mode = 0;
+    return a;
 }
 
 // ICPStep's body on a caller-given state and partial-row buffer (kIcpMaxBlocks rows of 64
@@ -836,40 +873,12 @@ fu_status fu::icp_step_on(TrackState* st, float* partials, const float* next_vma
     memcpy(h.tlast, tlast, 12);
     h.status = TS_RUNNING;
     HIPCHK(hipMemcpyAsync(st, &h, sizeof(h), hipMemcpyHostToDevice, s));
-    IcpArgs a;
-    memset(&a, 0, sizeof(a));
-    a.vcurr = (const f4*)next_vmap;
-    a.ncurr = (const f4*)next_nmap;
-    a.vlast = (const f4*)last_vmap;
-    a.nlast = (const f4*)last_nmap;
-    a.cols = cols;
-    a.rows = rows;
-    a.fx = fx;
-    a.fy = fy;
-    a.cx = cx;
-    a.cy = cy;
-    a.st = st;
-    a.partials = partials;
-    a.mode = 0;
+    const IcpArgs a = icp_step_args(st, partials, next_vmap, last_vmap, next_nmap, last_nmap, cols, rows, fx, fy, cx, cy);
     launch_icp(a, icp_groups(cols * rows), s);
     LAUNCHCHK();
     HIPCHK(hipMemcpyAsync(&h, st, sizeof(h), hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
-    // CreateMatrix<6,7> (Reduction.cu:6-16)
-    int shift = 0;
-    for (int i = 0; i < 6; ++i)
-        for (int j = i; j < 7; ++j) {
-            const double v = (double)h.sums[shift++];
-            if (j == 6) {
-                if (b) b[i] = v;
-            } else if (A) {
-                A[j * 6 + i] = A[i * 6 + j] = v;
-            }
-        }
-    if (residual) {
-        residual[0] = h.sums[27];
-        residual[1] = h.sums[28];
-    }
+    icp_step_outputs(h.sums, residual, A, b);
     return FU_OK;
 }
 
@@ -887,8 +896,23 @@ extern "C" fu_status fu_icp_step(const float* next_vmap, const float* last_vmap,
         fu_status st = fu_tracker_create(8, 8, &scratch);
         if (st) return st;
     }
-    return icp_step_on(scratch->st, scratch->partials, next_vmap, last_vmap, next_nmap, last_nmap, cols, rows, Rcurr,
-                       tcurr, Rlast, RlastInv, tlast, fx, fy, cx, cy, residual, A, b, S(s));
+    Mail mail;
+    if (!mail.dev)
+        return icp_step_on(scratch->st, scratch->partials, next_vmap, last_vmap, next_nmap, last_nmap, cols, rows, Rcurr,
+                           tcurr, Rlast, RlastInv, tlast, fx, fy, cx, cy, residual, A, b, S(s));
+    // one launch: the poses are arguments, the sums land in host memory
+    launch_icp_step(icp_step_args(scratch->st, scratch->partials, next_vmap, last_vmap, next_nmap, last_nmap, cols, rows, fx,
+                                  fy, cx, cy),
+                    icp_groups(cols * rows), Rcurr, tcurr, Rlast, RlastInv, tlast, (float*)mail.dev, S(s));
+    const hipError_t le = hipGetLastError();
+    if (le != hipSuccess) {
+        mail.done();
+        return set_err(FU_ERR_HIP, "kernel launch: %s", hipGetErrorString(le));
+    }
+    HIPCHK(hipStreamSynchronize(S(s)));
+    mail.done();
+    icp_step_outputs((const float*)mail.host, residual, A, b);
+    return FU_OK;
 }
 
 // RGBStep (Reduction.h:74-84, Reduction.cu:537-627): the photometric reduction of one level.
@@ -946,8 +970,7 @@ extern "C" fu_status fu_rgb_step(const uint8_t* next_image, const uint8_t* last_
     launch_rgb_lists(&a, &nb, 1, S(s));
     launch_icp(a, nb, S(s));
     LAUNCHCHK();
-    HIPCHK(hipMemcpyAsync(&h, scratch->st, sizeof(h), hipMemcpyDeviceToHost, S(s)));
-    HIPCHK(hipStreamSynchronize(S(s)));
+    HIPCHK(mail_read(scratch->dev, &h, scratch->st, sizeof(h), S(s)));
     double Ah[36], bh[6];
     unpack_sums29(h.rgb_sums, Ah, bh);
     if (A) memcpy(A, Ah, sizeof(Ah));
@@ -1620,9 +1643,7 @@ extern "C" fu_status fu_system_result(fu_system* sys, fu_frame_result* out, fu_s
     if (!sys || !out) return set_err(FU_ERR_ARG, "null argument");
     TrackState h;
     unsigned c[C_COUNT];
-    HIPCHK(hipMemcpyAsync(&h, sys->trk->st, sizeof(h), hipMemcpyDeviceToHost, S(s)));
-    HIPCHK(hipMemcpyAsync(c, sys->map->v.ctr, sizeof(c), hipMemcpyDeviceToHost, S(s)));
-    HIPCHK(hipStreamSynchronize(S(s)));
+    HIPCHK(mail_read(sys->trk->dev, &h, sys->trk->st, sizeof(h), c, sys->map->v.ctr, sizeof(c), S(s)));
     memcpy(out->pose, h.next_pose, sizeof(out->pose));
     out->track_status = h.status;
     out->fused = (h.gates & GATE_FUSE) ? 1 : 0;
@@ -2106,6 +2127,9 @@ struct fu_icp_batch {
     int cap = 0;
     SessDesc* d_desc = nullptr;
     std::vector<SessDesc> h_desc;
+    int ran = 0;                 // pairs of the last call
+    TrackState* h_res = nullptr;  // pinned: their states (fu_icp_batch_results), cap of them
+    void* d_res = nullptr;       // its device address
 };
 
 extern "C" fu_status fu_icp_batch_create(int capacity, fu_icp_batch** out) {
@@ -2127,7 +2151,32 @@ extern "C" fu_status fu_icp_batch_create(int capacity, fu_icp_batch** out) {
 extern "C" fu_status fu_icp_batch_destroy(fu_icp_batch* b) {
     if (!b) return FU_OK;
     (void)hipFree(b->d_desc);
+    if (b->h_res) (void)hipHostFree(b->h_res);
     delete b;
+    return FU_OK;
+}
+
+// the results of every tracker of the last fu_compute_se3_batch call: their states gathered into
+// pinned memory by one launch, one synchronisation for all of them
+extern "C" fu_status fu_icp_batch_results(fu_icp_batch* b, int n, fu_track_result* out, fu_stream s) {
+    if (!b || !out) return set_err(FU_ERR_ARG, "fu_icp_batch_results: null argument");
+    if (n < 1 || n != b->ran) return set_err(FU_ERR_STATE, "fu_icp_batch_results: %d results of a call with %d pairs", n, b->ran);
+    if (!b->h_res) {
+        void* p = nullptr;
+        if (hipHostMalloc(&p, sizeof(TrackState) * b->cap, hipHostMallocMapped) != hipSuccess) {
+            (void)hipGetLastError();
+            return set_err(FU_ERR_NOMEM, "fu_icp_batch_results: pinned memory");
+        }
+        if (hipHostGetDevicePointer(&b->d_res, p, 0) != hipSuccess) {
+            (void)hipHostFree(p);
+            return set_err(FU_ERR_HIP, "fu_icp_batch_results: pinned memory is not mapped");
+        }
+        b->h_res = (TrackState*)p;
+    }
+    launch_states(b->d_desc, n, b->d_res, S(s));
+    LAUNCHCHK();
+    HIPCHK(hipStreamSynchronize(S(s)));
+    for (int i = 0; i < n; ++i) fill_result(b->h_res[i], &out[i]);
     return FU_OK;
 }
 
@@ -2168,6 +2217,7 @@ extern "C" fu_status fu_compute_se3_batch(fu_icp_batch* ib, int n, fu_tracker* c
         }
     }
     hipStream_t hs = S(s);
+    ib->ran = 0;
     // the descriptors of this call; copied before any kernel of the call reads them
     HIPCHK(hipMemcpyAsync(ib->d_desc, ib->h_desc.data(), sizeof(SessDesc) * n, hipMemcpyHostToDevice, hs));
     HIPCHK(hipStreamSynchronize(hs));
@@ -2183,5 +2233,6 @@ extern "C" fu_status fu_compute_se3_batch(fu_icp_batch* ib, int n, fu_tracker* c
             for (int j = 0; j < iters[l]; ++j) launch_b_icp(b, h, l, j, hs);
     }
     LAUNCHCHK();
+    ib->ran = n;
     return FU_OK;
 }

@@ -15,9 +15,11 @@ struct fu_map {
     unsigned* mesh_counts = nullptr;
     unsigned* mesh_chunk = nullptr;
     std::vector<void*> allocs;
+    int dev = -1;  // the device the map was created on
 };
 
 struct fu_tracker {
+    int dev = -1;  // the device the tracker was created on
     int cols, rows;
     fu::TrackState* st = nullptr;
     float* partials = nullptr;  // 64 floats per ICP work-group

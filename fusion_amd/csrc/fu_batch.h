@@ -172,6 +172,7 @@ void launch_b_icp(BatchLaunch& b, const SessDesc* h, int level, int iter, hipStr
 void launch_b_rgb_lists(BatchLaunch& b, const SessDesc* h, hipStream_t s);  // once per frame
 void launch_b_track_commit(BatchLaunch& b, const SessDesc* h, hipStream_t s);
 void launch_b_results(BatchLaunch& b, FrameBrief* out, hipStream_t s);
+void launch_states(const SessDesc* desc, int n, void* out, hipStream_t s);  // n whole TrackStates
 // map.hip
 void launch_b_alloc(BatchLaunch& b, const SessDesc* h, hipStream_t s);
 void launch_b_visible(BatchLaunch& b, const SessDesc* h, hipStream_t s);

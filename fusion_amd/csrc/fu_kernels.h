@@ -233,6 +233,10 @@ void upload_mc_tables();
 void launch_mesh(const MapView& m, const MeshOut& o, unsigned* counts, unsigned* chunk, hipStream_t s);
 // icp.hip
 void launch_icp(const IcpArgs& a, int nblocks, hipStream_t s);  // with a.use_rgb: RGBStep too
+// one ICP-only reduction at a pose of its own, its 29 sums into `out` (pinned host memory); a.st
+// and a.partials are scratch (a.st->arrived zero)
+void launch_icp_step(const IcpArgs& a, int nblocks, const float Rcurr[9], const float tcurr[3], const float Rlast[9],
+                     const float RlastInv[9], const float tlast[3], float* out, hipStream_t s);
 // the list of eligible pixels of the photometric term for up to three levels (a[l].use_rgb)
 void launch_rgb_lists(const IcpArgs* a, const int* nblocks, int nlevels, hipStream_t s);
 void launch_track_begin(TrackState* st, hipStream_t s);

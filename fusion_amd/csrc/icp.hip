@@ -487,8 +487,13 @@ __device__ __forceinline__ void icp_update_wave(const IcpArgs& a, const float* t
 
 // the last stage of an ICP-only iteration, by a work-group of NW waves
 template <int NW>
-__device__ __forceinline__ void icp_last(const IcpArgs& a, int chunks) {
+__device__ __forceinline__ void icp_last(const IcpArgs& a, int chunks, float* out = nullptr) {
     __shared__ float total[32];
+    if (out) {
+        sum_rows32<NW>(a.partials, chunks, total);
+        if (threadIdx.x < 29) out[threadIdx.x] = total[threadIdx.x];  // the lane's own total
+        return;
+    }
     __shared__ double sm[64];
     const UpdateIn in = load_update(a.st);
     sum_rows32<NW>(a.partials, chunks, total);
@@ -508,8 +513,14 @@ __device__ __forceinline__ void icp_last(const IcpArgs& a, int chunks) {
 // than kLastGroups chunks, where a second launch does (kTicket).
 enum IcpForm : int { kLoop, kChunk, kQuarter };
 
+// `step`: a single reduction (ICPStep) at the pose given there, whose 29 sums go to step->out; the
+// tracking state only counts the rows.
+struct IcpStep {
+    IcpPose pose;
+    float* out;  // pinned host memory
+};
 template <int FORM, bool kTicket>
-__device__ __forceinline__ void icp_body(WG g, const IcpArgs& a) {
+__device__ __forceinline__ void icp_body(WG g, const IcpArgs& a, const IcpStep* step = nullptr) {
     constexpr int NT = FORM == kQuarter ? 256 : kIcpThreads, NW = NT / 64;
     static_assert(kIcpLanePixels == 2, "a lane's pixels are loaded as a pair");
     const int N = a.cols * a.rows;
@@ -523,7 +534,7 @@ __device__ __forceinline__ void icp_body(WG g, const IcpArgs& a) {
     icp_load(a, i0 + kIcpThreads, i0 + kIcpThreads < N, q);
     const auto st = FU_G(const TrackState, a.st);
     if (a.mode != 0 && st->status != TS_RUNNING) return;  // uniform: a failed frame skips
-    const IcpPose P = icp_pose(a.st);
+    const IcpPose P = step ? step->pose : icp_pose(a.st);
     __shared__ float wsum[NW][32];
     float v[32];
     v[29] = v[30] = v[31] = 0.f;
@@ -560,12 +571,16 @@ __device__ __forceinline__ void icp_body(WG g, const IcpArgs& a) {
     }
     block_rows29(v, wsum, a.partials + g.x * 32);
     if constexpr (kTicket) {
-        if (last_to_arrive(a.st, g.nx)) icp_last<NW>(a, FORM == kQuarter ? g.nx >> 2 : g.nx);
+        if (last_to_arrive(a.st, g.nx)) icp_last<NW>(a, FORM == kQuarter ? g.nx >> 2 : g.nx, step ? step->out : nullptr);
     }
 }
 template <int FORM>
 __global__ __launch_bounds__(FORM == kQuarter ? 256 : kIcpThreads) void k_icp(IcpArgs a) {
     icp_body<FORM, true>(hw_wg(), a);
+}
+template <int FORM>
+__global__ __launch_bounds__(FORM == kQuarter ? 256 : kIcpThreads) void k_icp_step(IcpArgs a, IcpStep step) {
+    icp_body<FORM, true>(hw_wg(), a, &step);
 }
 
 // ------------------------------------------------------------------ photometric term
@@ -984,6 +999,20 @@ constexpr int kQuarterChunks = 128;
 // microsecond for its row and its count holds up the next: the rows are summed by a second launch.
 constexpr int kLastGroups = 4096;
 
+void launch_icp_step(const IcpArgs& a, int nblocks, const float Rcurr[9], const float tcurr[3], const float Rlast[9],
+                     const float RlastInv[9], const float tlast[3], float* out, hipStream_t s) {
+    auto m = [](const float* r) { return m3{mk3(r[0], r[1], r[2]), mk3(r[3], r[4], r[5]), mk3(r[6], r[7], r[8])}; };
+    const IcpStep step{IcpPose{m(Rcurr), m(Rlast), m(RlastInv), mk3(tcurr[0], tcurr[1], tcurr[2]),
+                               mk3(tlast[0], tlast[1], tlast[2])},
+                       out};
+    if ((long long)nblocks * kIcpPixels < (long long)a.cols * a.rows)
+        hipLaunchKernelGGL(k_icp_step<kLoop>, dim3(nblocks), dim3(kIcpThreads), 0, s, a, step);
+    else if (nblocks <= kQuarterChunks)
+        hipLaunchKernelGGL(k_icp_step<kQuarter>, dim3(nblocks * 4), dim3(256), 0, s, a, step);
+    else
+        hipLaunchKernelGGL(k_icp_step<kChunk>, dim3(nblocks), dim3(kIcpThreads), 0, s, a, step);
+}
+
 void launch_icp(const IcpArgs& a, int nblocks, hipStream_t s) {
     if (a.use_rgb) {  // one pixel per lane (the caller sizes nblocks to cover the level)
         hipLaunchKernelGGL(k_rgb_resid, dim3(nblocks), dim3(kIcpThreads), 0, s, a);
@@ -1115,6 +1144,15 @@ __global__ void kb_results(BatchLaunch b, FrameBrief* out) {
     if (t == 20) o->n_alloc = min(d.m.ctr[C_ALLOC], d.m.num_blocks);
     if (t == 21) o->flags = d.m.ctr[C_FLAGS];
     if (t == 22) o->rgb_count = d.use_rgb ? st->rgb_count : 0;
+}
+// the states of the first n sessions, one after the other
+__global__ __launch_bounds__(256) void k_states(const SessDesc* desc, unsigned* out) {
+    const auto src = FU_G(const unsigned, reinterpret_cast<const unsigned*>(desc[blockIdx.x].st));
+    constexpr int n = (int)(sizeof(TrackState) / 4);
+    for (int i = threadIdx.x; i < n; i += 256) out[blockIdx.x * n + i] = src[i];
+}
+void launch_states(const SessDesc* desc, int n, void* out, hipStream_t s) {
+    hipLaunchKernelGGL(k_states, dim3(n), dim3(256), 0, s, desc, (unsigned*)out);
 }
 void launch_b_results(BatchLaunch& b, FrameBrief* out, hipStream_t s) {
     hipLaunchKernelGGL(kb_results, dim3(b.n), dim3(64), 0, s, b, out);

@@ -178,6 +178,7 @@ SIGNATURES = {
     "fu_icp_batch_destroy": (I, [P]),
     "fu_compute_se3_batch": (I, [P, I, C.POINTER(P), C.POINTER(P), C.POINTER(P), C.POINTER(P), C.POINTER(P), FP,
                                  C.POINTER(C.c_int32), C.POINTER(C.c_int32), C.c_float, P]),
+    "fu_icp_batch_results": (I, [P, I, C.POINTER(TrackResult), P]),
     "fu_batch_create": (I, [I, C.POINTER(P)]),
     "fu_batch_destroy": (I, [P]),
     "fu_batch_attach": (I, [P, P]),
