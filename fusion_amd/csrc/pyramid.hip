@@ -79,11 +79,26 @@ __global__ __launch_bounds__(256) void k_filter_depth(const uint16_t* __restrict
     filter_depth_body(hw_wg(), depth, raw, filt, cols, rows, scale_inv, cutoff);
 }
 
-// binomial [1 4 6 4 1] outer product, indexed (ty-cy-1)*5 + (tx-cx-1) as in Pyrdown.cu:151,
-// which mirrors the weights at the right/bottom border
-__constant__ float c_gauss[25] = {1, 4, 6, 4, 1, 4, 16, 24, 16, 4, 6, 24, 36, 24, 6, 4, 16, 24, 16, 4, 1, 4, 6, 4, 1};
+// binomial [1 4 6 4 1] outer product, indexed (ty-cy-1)*5 + (tx-cx-1) as in Pyrdown.cu:151, where
+// tx and ty end the window: clipped at the right or bottom border by s samples, its weights shift
+// by s (tap q of an axis takes entry 4 - s - q)
 constexpr float kGauss[25] = {1, 4, 6, 4, 1, 4, 16, 24, 16, 4, 6, 24, 36, 24, 6, 4, 16, 24, 16, 4, 1, 4, 6, 4, 1};
+// the weights of an axis' five taps for s = 0, 1, 2 samples clipped
+__device__ __forceinline__ void axis_weights(int s, float (&w)[5]) {
+    constexpr float g[7] = {1, 4, 6, 4, 1, 0, 0};
+#pragma unroll
+    for (int q = 0; q < 5; ++q) w[q] = s == 0 ? g[q] : s == 1 ? g[q + 1] : g[q + 2];
+}
+// destination pixel (x, y) whose whole 5x5 window lies in the source: its right and bottom ends
+// are not clipped either
+__device__ __forceinline__ bool whole_window(int x, int y, int scols, int srows) {
+    return x >= 1 && y >= 1 && 2 * x + 3 < scols && 2 * y + 3 < srows;
+}
 
+// Every wave loads its windows' 25 samples together: as they are, or, where a lane's window is
+// clipped, from clamped places with the weights above and a test per tap.  Bound by one trip to
+// memory and the launch.  One tap after the other, a clipped window took 5 of a launch's 8 us:
+// 320x240 -> 160x120 7.9 -> 3.6 us, 1280x720 -> 640x360 8.1 -> 4.3 us.
 __device__ __forceinline__ void pyrdown_body(WG g, const float* __restrict__ src_, int scols, int srows,
                                              float* __restrict__ dst_, int dcols, int drows,
                                              VertexOut vo = VertexOut{}, float cutoff = 0.f) {
@@ -92,12 +107,8 @@ __device__ __forceinline__ void pyrdown_body(WG g, const float* __restrict__ src
     if (x >= dcols || y >= drows) return;
     const auto src = FU_G(const float, src_);
     const auto dst = FU_G(float, dst_);
-    const int tx = min(2 * x + 3, scols - 1);
-    const int ty = min(2 * y + 3, srows - 1);
-    float sum = 0.f;
-    int count = 0;
-    if (x >= 1 && y >= 1 && 2 * x + 3 < scols && 2 * y + 3 < srows) {
-        // the whole 5x5 window: its loads issue together; NaN samples are skipped as below
+    float sum = 0.f, count = 0.f;  // whole numbers up to 256
+    if (__all(whole_window(x, y, scols, srows))) {
         const auto p = src + (2 * y - 2) * scols + (2 * x - 2);
         float v[25];
 #pragma unroll
@@ -107,21 +118,30 @@ __device__ __forceinline__ void pyrdown_body(WG g, const float* __restrict__ src
             const float g = kGauss[(4 - q / 5) * 5 + (4 - q % 5)];
             const bool ok = !isnanf_(v[q]);
             sum = ok ? sum + v[q] * g : sum;
-            count += ok ? (int)g : 0;
+            count += ok ? g : 0.f;
         }
     } else {
-        for (int cy = max(0, 2 * y - 2); cy < ty; ++cy) {
-            for (int cx = max(0, 2 * x - 2); cx < tx; ++cx) {
-                const float v = src[cy * scols + cx];
-                if (!isnanf_(v)) {
-                    const float g = c_gauss[(ty - cy - 1) * 5 + (tx - cx - 1)];
-                    sum += v * g;
-                    count += (int)g;
-                }
-            }
+        const int tx = min(2 * x + 3, scols - 1), ty = min(2 * y + 3, srows - 1);
+        float wx[5], wy[5];
+        axis_weights(2 * x + 3 - tx, wx);
+        axis_weights(2 * y + 3 - ty, wy);
+        float v[25];
+#pragma unroll
+        for (int q = 0; q < 25; ++q) {
+            const int cx = 2 * x - 2 + q % 5, cy = 2 * y - 2 + q / 5;
+            const bool in = cx >= 0 && cy >= 0 && cx < tx && cy < ty;
+            const float t = src[in ? cy * scols + cx : 0];
+            v[q] = in ? t : fnan();
+        }
+#pragma unroll
+        for (int q = 0; q < 25; ++q) {
+            const float g = wx[q % 5] * wy[q / 5];
+            const bool ok = !isnanf_(v[q]);
+            sum = ok ? sum + v[q] * g : sum;
+            count += ok ? g : 0.f;
         }
     }
-    const float z = sum / (float)count;
+    const float z = sum / count;
     dst[y * dcols + x] = z;
     if (vo.vmap) FU_G(f4, vo.vmap)[y * dcols + x] = vertex_of(z, x, y, vo.invfx, vo.invfy, vo.cx, vo.cy, cutoff);
 }
@@ -222,9 +242,17 @@ __global__ __launch_bounds__(256) void k_intensity(const unsigned char* __restri
     intensity_body(hw_wg(), rgb, img, cols, rows);
 }
 
+// four bytes at any address
+__device__ __forceinline__ unsigned load4(FU_GPTR(const unsigned char) p) {
+    typedef unsigned __attribute__((aligned(1))) U1;
+    return *(FU_GPTR(const U1))p;
+}
+
 // PyrDownGaussKernel<uchar, uchar> (Pyrdown.cu:133-158): the float kernel's window and
 // mirrored weights over bytes (no byte is NaN), the float mean truncated to a byte.  Every
-// product and partial sum is an integer below 2^24, so the float sums are exact.
+// product and partial sum is an integer below 2^24, so the float sums are exact and a whole
+// window's mean is its integer sum / 256: a row is one 4-byte load, a byte and a dot product
+// (1280x720 -> 640x360: 5.5 -> 3.6 us).
 __device__ __forceinline__ void pyrdown_u8_body(WG g, const unsigned char* __restrict__ src_, int scols, int srows,
                                                 unsigned char* __restrict__ dst_, int dcols, int drows) {
     const int x = g.x * 16 + (threadIdx.x & 15);
@@ -232,33 +260,38 @@ __device__ __forceinline__ void pyrdown_u8_body(WG g, const unsigned char* __res
     if (x >= dcols || y >= drows) return;
     const auto src = FU_G(const unsigned char, src_);
     const auto dst = FU_G(unsigned char, dst_);
-    const int tx = min(2 * x + 3, scols - 1);
-    const int ty = min(2 * y + 3, srows - 1);
-    float sum = 0.f;
-    int count = 0;
-    if (x >= 1 && y >= 1 && 2 * x + 3 < scols && 2 * y + 3 < srows) {
-        // the whole 5x5 window: its loads issue together, the same products and sums in the
-        // same order as the clipped loop below
+    if (__all(whole_window(x, y, scols, srows))) {
         const auto p = src + (2 * y - 2) * scols + (2 * x - 2);
-        float v[25];
+        unsigned r[5], e[5];
 #pragma unroll
-        for (int q = 0; q < 25; ++q) v[q] = (float)p[(q / 5) * scols + q % 5];
+        for (int q = 0; q < 5; ++q) {
+            r[q] = load4(p + q * scols);
+            e[q] = p[q * scols + 4];
+        }
 #pragma unroll
-        for (int q = 0; q < 25; ++q) {
-            const float g = kGauss[(4 - q / 5) * 5 + (4 - q % 5)];
-            sum += v[q] * g;
-            count += (int)g;
-        }
-    } else {
-        for (int cy = max(0, 2 * y - 2); cy < ty; ++cy) {
-            for (int cx = max(0, 2 * x - 2); cx < tx; ++cx) {
-                const float g = c_gauss[(ty - cy - 1) * 5 + (tx - cx - 1)];
-                sum += (float)src[cy * scols + cx] * g;
-                count += (int)g;
-            }
-        }
+        for (int q = 0; q < 5; ++q) r[q] = __builtin_amdgcn_udot4(r[q], 0x04060401u, e[q], false);
+        dst[y * dcols + x] = (unsigned char)((r[0] + 4u * r[1] + 6u * r[2] + 4u * r[3] + r[4]) >> 8);
+        return;
     }
-    dst[y * dcols + x] = (unsigned char)f2i(sum / (float)count);
+    const int tx = min(2 * x + 3, scols - 1), ty = min(2 * y + 3, srows - 1);
+    float wx[5], wy[5];
+    axis_weights(2 * x + 3 - tx, wx);
+    axis_weights(2 * y + 3 - ty, wy);
+    float v[25], w[25];
+#pragma unroll
+    for (int q = 0; q < 25; ++q) {
+        const int cx = 2 * x - 2 + q % 5, cy = 2 * y - 2 + q / 5;
+        const bool in = cx >= 0 && cy >= 0 && cx < tx && cy < ty;
+        v[q] = (float)src[in ? cy * scols + cx : 0];
+        w[q] = in ? wx[q % 5] * wy[q / 5] : 0.f;
+    }
+    float sum = 0.f, count = 0.f;
+#pragma unroll
+    for (int q = 0; q < 25; ++q) {
+        sum += v[q] * w[q];
+        count += w[q];
+    }
+    dst[y * dcols + x] = (unsigned char)f2i(sum / count);
 }
 __global__ __launch_bounds__(256) void k_pyrdown_u8(const unsigned char* __restrict__ src, int scols, int srows,
                                                    unsigned char* __restrict__ dst, int dcols, int drows) {
@@ -268,42 +301,35 @@ __global__ __launch_bounds__(256) void k_pyrdown_u8(const unsigned char* __restr
 // ComputeDerivativeImageKernel (Pyrdown.cu:210-236): 3x3 Sobel over the window clipped to
 // the image, the weight index counting down from 8 across the clipped window (at the border
 // the weights shift), float sums stored as shorts
-__constant__ float c_sobel_x[9] = {1, 0, -1, 2, 0, -2, 1, 0, -1};
-__constant__ float c_sobel_y[9] = {1, 2, 1, 0, 0, 0, -1, -2, -1};
+__constant__ int c_sobel_x[9] = {1, 0, -1, 2, 0, -2, 1, 0, -1};
+__constant__ int c_sobel_y[9] = {1, 2, 1, 0, 0, 0, -1, -2, -1};
 __device__ __forceinline__ void derivative_body(WG g, const unsigned char* __restrict__ img_, short* __restrict__ dx_,
                                                 short* __restrict__ dy_, int cols, int rows) {
     const int x = g.x * 16 + (threadIdx.x & 15);
     const int y = g.y * 16 + (threadIdx.x >> 4);
     if (x >= cols || y >= rows) return;
     const auto img = FU_G(const unsigned char, img_);
-    float a = 0.f, b = 0.f;
-    if (x >= 1 && y >= 1 && x + 1 < cols && y + 1 < rows) {
-        // the whole 3x3 window: its nine loads issue together, the same products and sums in
-        // the same order as the clipped loop below (k = 8 .. 0)
-        constexpr float sx[9] = {1, 0, -1, 2, 0, -2, 1, 0, -1};
-        constexpr float sy[9] = {1, 2, 1, 0, 0, 0, -1, -2, -1};
+    int a = 0, b = 0;  // the float sums are of small integers: exact
+    if (x >= 1 && y >= 1 && x + 2 < cols && y + 1 < rows) {
+        // the whole 3x3 window, a 4-byte load per row (its last byte not used)
         const auto p = img + (y - 1) * cols + (x - 1);
-        float v[9];
-#pragma unroll
-        for (int q = 0; q < 9; ++q) v[q] = (float)p[(q / 3) * cols + q % 3];
-#pragma unroll
-        for (int q = 0; q < 9; ++q) {
-            a += v[q] * sx[8 - q];
-            b += v[q] * sy[8 - q];
-        }
+        const unsigned r0 = load4(p), r1 = load4(p + cols), r2 = load4(p + 2 * cols);
+        auto at = [](unsigned r, int k) { return (int)((r >> (8 * k)) & 255u); };
+        a = (at(r0, 2) - at(r0, 0)) + 2 * (at(r1, 2) - at(r1, 0)) + (at(r2, 2) - at(r2, 0));
+        b = (at(r2, 0) + 2 * at(r2, 1) + at(r2, 2)) - (at(r0, 0) + 2 * at(r0, 1) + at(r0, 2));
     } else {
         int k = 8;
         for (int j = max(y - 1, 0); j <= min(y + 1, rows - 1); ++j) {
             for (int i = max(x - 1, 0); i <= min(x + 1, cols - 1); ++i) {
-                const float v = (float)img[j * cols + i];
+                const int v = img[j * cols + i];
                 a += v * c_sobel_x[k];
                 b += v * c_sobel_y[k];
                 --k;
             }
         }
     }
-    FU_G(short, dx_)[y * cols + x] = (short)f2i(a);
-    FU_G(short, dy_)[y * cols + x] = (short)f2i(b);
+    FU_G(short, dx_)[y * cols + x] = (short)a;
+    FU_G(short, dy_)[y * cols + x] = (short)b;
 }
 __global__ __launch_bounds__(256) void k_derivative(const unsigned char* __restrict__ img, short* __restrict__ dx,
                                                    short* __restrict__ dy, int cols, int rows) {
