@@ -116,19 +116,29 @@ __global__ void k_lift_keys(LiftArgs a) {
 // ---------------------------------------------------------------------------- matching
 // The two nearest train descriptors of every query descriptor by L2 distance (sqrt of the sum
 // of the 64 squared differences, in dimension order); ties go to the lower train index.
-// Work-group: 256 queries, one per lane (its descriptor in registers), against a chunk of
-// train descriptors staged through LDS kTile at a time (every lane reads the same record: LDS
-// broadcast).  Each (query, chunk) pair leaves its best two; a second pass merges the chunks.
-// The chunk length is chosen per call so that the grid holds about kTargetGroups work-groups
-// (a few hundred queries against tens of thousands of keys would otherwise fill a dozen CUs).
-// Both passes keep the two smallest (distance, index) pairs in lexicographic order, a total
-// order over the candidates (NaN and +inf distances never enter), so the result is the same for
-// every chunking and merge order: that of one lane scanning the train set in index order with
-// strict comparisons.
+// Few of the pairs need that exact sum.  k_match_bound prices every pair on the matrix cores
+// (|t|^2 - 2 q.t, FP32) and keeps, per query and chunk of train descriptors, the least lower and
+// the least upper bound; k_match_scan, a wave per query, takes the second least upper bound and
+// evaluates the chunks whose lower bound does not exceed it, a lane per train descriptor, with
+// the sum's own operations and order.  It keeps the two smallest (distance, index) pairs in
+// lexicographic order, a total order over the candidates (NaN and +inf distances never enter), so
+// the result is that of one lane scanning the train set in index order with strict comparisons.
+//
+// The bounds.  u = 2^-24, Q = |q|^2, T = |t|^2: the price errs by at most 64 u (Q + T) (the dot
+// product, doubled, with 2 |q||t| <= Q + T) + 64 u T + 4 u (Q + 3 T) from |q - t|^2 - Q, and the
+// exact sum by 67 u |q - t|^2 <= 134 u (Q + T), its root's rounding (ties) by another 8 u (Q + T).
+// kSlack = 512 u times (2 T + Q) covers twice that; kTiny covers sums that round towards zero
+// below the normal range.  The chunk of a T that is not below kHuge (or not a number: products may
+// overflow) is always evaluated, a query with such a Q evaluates all of them.
+//
+// 900 queries against 20,000: all pairs by the exact sum, bound by VALU issue (192 operations a
+// pair), took 153 us; the two passes take 43 + 14.  The first is bound by its matrix instructions
+// (17 us) and the loads under them: with a quarter of the instructions it still takes 28 us.
 constexpr int kDesc = 64;
-constexpr int kTile = 128;
-constexpr int kChunk = 8192;
+constexpr int kChunkMin = 128, kChunkMax = 8192;  // train descriptors
 constexpr int kTargetGroups = 4096;
+constexpr int kScanAll = 512;  // up to so many train descriptors are all evaluated: no first pass
+constexpr float kSlack = 0x1p-15f, kTiny = 0x1p-100f, kHuge = 1e37f;
 
 struct Best2 {
     float d0, d1;
@@ -151,45 +161,149 @@ __device__ __forceinline__ void push2(Best2& b, float d, int i) {
     }
 }
 
-__global__ __launch_bounds__(256) void k_match_chunk(const float* q, int nq, const float* t, int nt, int chunk,
-                                                     Best2* part) {
-    __shared__ float tile[kTile * kDesc];
-    const int qi = blockIdx.x * 256 + threadIdx.x;
-    const int c0 = blockIdx.y * chunk, c1 = min(nt, c0 + chunk);
-    float mine[kDesc];
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef v4f v4f_word __attribute__((aligned(4)));  // descriptors are aligned as floats are
+
+// A wave: 32 queries (its A operand: lane l holds of query l & 31 the four dimensions of every
+// eight from 4 (l >> 5) on, in both operands, so that a load takes 32-byte pieces; the sum's order
+// is free) against its chunk, 32 train
+// descriptors at a time.  Four waves a SIMD hide each other's loads better than the next
+// descriptors loaded ahead, which leave registers for three (44 and 50 us); a chunk's work-groups
+// share an XCD's L2 (43 us).
+// bound[chunk * nq + query] = {lower, upper}, without the query's own share.
+__global__ __launch_bounds__(256, 4) void k_match_bound(const float* q, int nq, const float* t, int nt, int chunk,
+                                                        float2* bound) {
+    const int lane = threadIdx.x & 63, n = lane & 31, half = lane >> 5;
+    // work-groups go to the eight XCDs in turn: each XCD takes every eighth chunk, all its queries
+    const int groups = (nq + 127) / 128, slot = blockIdx.x >> 3;
+    const int c = slot / groups * 8 + (blockIdx.x & 7);
+    const int q0 = (slot % groups * 4 + (threadIdx.x >> 6)) * 32;
+    const int c0 = c * chunk, c1 = min(nt, c0 + chunk);
+    if (q0 >= nq || c0 >= nt) return;  // uniform
+    auto fetch = [&](const float* base, int row, v4f (&x)[8]) {
+        const auto p = FU_G(const v4f_word, base + (size_t)row * kDesc + half * 4);
 #pragma unroll
-    for (int j = 0; j < kDesc; ++j) mine[j] = qi < nq ? q[(size_t)qi * kDesc + j] : 0.f;
-    Best2 b{INFINITY, INFINITY, -1, -1};
-    for (int base = c0; base < c1; base += kTile) {
-        const int cnt = min(kTile, c1 - base);
-        __syncthreads();
-        for (int k = threadIdx.x; k < cnt * kDesc; k += 256) tile[k] = t[(size_t)base * kDesc + k];
-        __syncthreads();
-        for (int r = 0; r < cnt; ++r) {
-            float s = 0.f;
+        for (int k = 0; k < 8; ++k) x[k] = p[2 * k];
+    };
+    v4f a[8], cur[8];
+    fetch(q, min(q0 + n, nq - 1), a);
+    float lo[16], hi[16];
 #pragma unroll
-            for (int j = 0; j < kDesc; ++j) {
-                const float dj = mine[j] - tile[r * kDesc + j];
-                s = s + dj * dj;
+    for (int r = 0; r < 16; ++r) lo[r] = hi[r] = INFINITY;
+    bool bad = false;
+#pragma unroll 1
+    for (int base = c0; base < c1; base += 32) {
+        fetch(t, min(base + n, nt - 1), cur);
+        v16f acc = {0.f};
+        float T = 0.f;
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[k][e], cur[k][e], acc, 0, 0, 0);
+                T = fmaf(cur[k][e], cur[k][e], T);
             }
-            const float d = sqrtf(s);
-            if (d < b.d1) push2(b, d, base + r);  // indices rise within the chunk: d < d1 is the test
+        T += __shfl_xor(T, 32);
+        const bool in = base + n < c1, sane = T < kHuge;
+        bad = bad || (in && !sane);
+        const float tl = in && sane ? fmaf(T, -2.f * kSlack, T) : INFINITY;
+        const float th = in && sane ? fmaf(T, 2.f * kSlack, T) : INFINITY;
+        // an infinite price or NaN (columns outside, or whose chunk is evaluated anyway) is no bound
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            lo[r] = fminf(lo[r], fmaf(-2.f, acc[r], tl));
+            hi[r] = fminf(hi[r], fmaf(-2.f, acc[r], th));
         }
     }
-    if (qi < nq) part[(size_t)blockIdx.y * nq + qi] = b;
+    // the least over the 32 columns: halves of the rows are exchanged, so that lane n ends with
+    // row n >> 1 of its 16
+    if (bad)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) lo[r] = -INFINITY;
+#pragma unroll
+    for (int h = 8; h >= 1; h >>= 1) {
+        const int off = 2 * h;
+        const bool up = (n & off) != 0;
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+            if (r >= h) break;
+            const float gl = up ? lo[r] : lo[r + h], gh = up ? hi[r] : hi[r + h];
+            const float kl = up ? lo[r + h] : lo[r], kh = up ? hi[r + h] : hi[r];
+            lo[r] = fminf(kl, __shfl_xor(gl, off));
+            hi[r] = fminf(kh, __shfl_xor(gh, off));
+        }
+    }
+    const float l = fminf(lo[0], __shfl_xor(lo[0], 1)), h = fminf(hi[0], __shfl_xor(hi[0], 1));
+    const int r = n >> 1;                                 // the row, of query:
+    const int qi = q0 + 8 * (r >> 2) + 4 * half + (r & 3);
+    if (!(n & 1) && qi < nq) bound[(size_t)c * nq + qi] = make_float2(l, h);
 }
 
-// one wave per query: lane l merges chunks l, l + 64, ..., then the lanes' best two are merged
-// across the wave
-__global__ __launch_bounds__(256) void k_match_merge(const Best2* part, int nq, int nchunks, int* idx, float* dist) {
-    const int qi = blockIdx.x * 4 + (threadIdx.x >> 6);
+// distance of train descriptor p to the wave's query
+template <class Q>
+__device__ __forceinline__ float exact_dist(const Q& q, FU_GPTR(const v4f_word) p) {
+    v4f x[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) x[k] = p[k];
+    float s = 0.f;
+#pragma unroll
+    for (int k = 0; k < 16; ++k)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float d = q[4 * k + e] - x[k][e];
+            s = s + d * d;
+        }
+    return sqrtf(s);
+}
+
+// a wave per query; without bounds (null) every chunk is evaluated
+__global__ __launch_bounds__(256) void k_match_scan(const float* q, int nq, const float* t, int nt, int chunk, int nchunks,
+                                                    const float2* bound, int* idx, float* dist) {
+    const int qi = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
     const int lane = threadIdx.x & 63;
-    if (qi >= nq) return;
+    if (qi >= nq) return;  // uniform
+    typedef const __attribute__((address_space(4))) float CF;
+    CF* qc = (CF*)(q + (size_t)qi * kDesc);
+    float limit = INFINITY;  // NaN or +inf: all chunks
+    if (bound) {
+        const float mine = q[(size_t)qi * kDesc + lane];
+        float Q = mine * mine;
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) Q += __shfl_xor(Q, off);
+        // the two least upper bounds
+        float h0 = INFINITY, h1 = INFINITY;
+        for (int c = lane; c < nchunks; c += 64) {
+            const float h = bound[(size_t)c * nq + qi].y;
+            h1 = fminf(h1, fmaxf(h0, h));
+            h0 = fminf(h0, h);
+        }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            const float g0 = __shfl_xor(h0, off), g1 = __shfl_xor(h1, off);
+            h1 = fminf(fminf(h1, g1), fmaxf(h0, g0));
+            h0 = fminf(h0, g0);
+        }
+        limit = Q < kHuge ? h1 + 2.f * fmaf(Q, kSlack, kTiny) : INFINITY;
+    }
     Best2 b{INFINITY, INFINITY, -1, -1};
-    for (int c = lane; c < nchunks; c += 64) {
-        const Best2 p = part[(size_t)c * nq + qi];
-        if (p.i0 >= 0) push2(b, p.d0, p.i0);
-        if (p.i1 >= 0) push2(b, p.d1, p.i1);
+    for (int base = 0; base < nchunks; base += 64) {
+        const int c = base + lane;
+        bool take = c < nchunks;
+        if (bound && take) take = !(bound[(size_t)c * nq + qi].x > limit);
+        unsigned long long m = __ballot(take);
+        while (m) {
+            const int k = base + __builtin_ctzll(m);
+            m &= m - 1;
+            const int c0 = k * chunk, c1 = min(nt, c0 + chunk);
+            for (int r = c0 + lane; r < c1; r += 128) {
+                const int r2 = min(r + 64, nt - 1);
+                const float d = exact_dist(qc, FU_G(const v4f_word, t + (size_t)r * kDesc));
+                const float e = exact_dist(qc, FU_G(const v4f_word, t + (size_t)r2 * kDesc));
+                push2(b, d, r);
+                if (r + 64 < c1) push2(b, e, r + 64);
+            }
+        }
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
@@ -206,13 +320,13 @@ __global__ __launch_bounds__(256) void k_match_merge(const Best2* part, int nq, 
     }
 }
 
-// train records per chunk: about kTargetGroups work-groups in all, at least one LDS tile and at
-// most kChunk records each, a whole number of tiles
+// train descriptors per chunk: about kTargetGroups chunks of 256 queries in all, at least
+// kChunkMin and at most kChunkMax, a whole number of kChunkMin
 static int match_chunk_len(int nq, int nt) {
     const long long qgroups = (nq + 255) / 256;
     long long want = ((long long)nt * qgroups + kTargetGroups - 1) / kTargetGroups;
-    want = (want + kTile - 1) / kTile * kTile;
-    return (int)std::min<long long>(kChunk, std::max<long long>(kTile, want));
+    want = (want + kChunkMin - 1) / kChunkMin * kChunkMin;
+    return (int)std::min<long long>(kChunkMax, std::max<long long>(kChunkMin, want));
 }
 
 // ---------------------------------------------------------------------------- graph selection
@@ -547,19 +661,23 @@ extern "C" fu_status fu_match_knn2(const float* query, int32_t nq, const float* 
         return api_error(FU_ERR_ARG, "fu_match_knn2: %d x %d descriptors (at most 2^25 each)", nq, nt);
     hipStream_t hs = (hipStream_t)s;
     const int chunk = match_chunk_len(nq, nt);
-    const int nchunks = nt > 0 ? (nt + chunk - 1) / chunk : 1;
-    Best2* part = nullptr;
-    if (hipMallocAsync((void**)&part, sizeof(Best2) * (size_t)nchunks * nq, hs) != hipSuccess) {
-        (void)hipGetLastError();
-        return api_error(FU_ERR_NOMEM, "fu_match_knn2: %d partial lists", nchunks);
+    const int nchunks = (nt + chunk - 1) / chunk;
+    float2* bound = nullptr;
+    if (nt > kScanAll) {
+        if (hipMallocAsync((void**)&bound, sizeof(float2) * (size_t)nchunks * nq, hs) != hipSuccess) {
+            (void)hipGetLastError();
+            return api_error(FU_ERR_NOMEM, "fu_match_knn2: %d partial lists", nchunks);
+        }
+        hipLaunchKernelGGL(k_match_bound, dim3((nq + 127) / 128 * ((nchunks + 7) / 8 * 8)), dim3(256), 0, hs, query, nq, train, nt, chunk,
+                           bound);
     }
-    if (nt > 0)
-        hipLaunchKernelGGL(k_match_chunk, dim3((nq + 255) / 256, nchunks), dim3(256), 0, hs, query, nq, train, nt, chunk,
-                           part);
-    hipLaunchKernelGGL(k_match_merge, dim3((nq + 3) / 4), dim3(256), 0, hs, part, nq, nt > 0 ? nchunks : 0, idx,
-                       dist);
+    hipLaunchKernelGGL(k_match_scan, dim3((nq + 3) / 4), dim3(256), 0, hs, query, nq, train, nt, chunk, nchunks, bound,
+                       idx, dist);
     hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = hipFreeAsync(part, hs);
+    if (bound) {
+        const hipError_t ef = hipFreeAsync(bound, hs);
+        if (e == hipSuccess) e = ef;
+    }
     if (e != hipSuccess) return api_error(FU_ERR_HIP, "fu_match_knn2: %s", hipGetErrorString(e));
     return FU_OK;
 }
