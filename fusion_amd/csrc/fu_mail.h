@@ -12,7 +12,7 @@ namespace fu {
 // A pinned, device-mapped slot of kMailBytes, taken from a process-wide pool for one call at a
 // time (any thread, any stream, any device) and given back when the call has synchronised.  The
 // pool keeps at most kMailSlots; `dev` is null when no slot could be had.
-constexpr size_t kMailBytes = 8192;
+constexpr size_t kMailBytes = 16384;
 constexpr size_t kMailSlots = 16;
 class Mail {
 public:

@@ -11,9 +11,12 @@
 // per-bucket try-lock drops a key that meets another in its bucket in the same launch.
 #include <hip/hip_runtime.h>
 #include <limits.h>
+#include <stddef.h>
 #include <string.h>
 
 #include "fu_api.h"
+#include "fu_keys.h"
+#include "fu_mail.h"
 
 using namespace fu;
 
@@ -27,6 +30,8 @@ struct alignas(16) Surf {  // fu_surf / SURF: valid, pos, normal, descriptor (28
     float desc[64];
 };
 static_assert(sizeof(Surf) == sizeof(fu_surf) && sizeof(Surf) == 288, "SURF layout");
+constexpr int kSurfHeads = kSlotHeads;
+static_assert(sizeof(Surf) % sizeof(SurfHead) == 0, "records are whole heads apart");
 
 // KeyMap::Hash (DeviceMap.cu:206-214): the signed remainder of the wrapped products' xor
 __device__ __forceinline__ int key_hash(i3 p, int max_keys) {
@@ -101,31 +106,54 @@ __global__ void k_insert_apply(KeyArgs a, Surf* in, int* index, unsigned char* d
 }
 
 // CollectKeys (FuseMap.cu:384-406) in slot order: valid key j (0-based over the slots) goes to
-// out[j] when 0 < j < cap (the reference copies only at offsets > 0).  Three passes: valid
-// counts per 1024-slot group, their exclusive prefix (one group), the scatter.
+// out[j] when 0 < j < cap (the reference copies only at offsets > 0).  k_collect_count leaves a
+// word of valid bits per 64 slots and the count of each 1024-slot group, and its last group to
+// end turns the counts into their exclusive prefix (16 us in all, as with a launch for the prefix,
+// without the gap between the two).  It is bound by the records' first lines (500,000 slots: 32 MB,
+// 11 us); the copies that follow read only the bits and the valid records (20,000 of 500,000 slots,
+// a lane per record behind its slot's flag: 20 us, now 6).
 constexpr int kCollect = 1024;
-__global__ void k_collect_count(const Surf* keys, int n, unsigned* counts) {
-    __shared__ unsigned c;
-    if (threadIdx.x == 0) c = 0;
-    __syncthreads();
-    const int i = blockIdx.x * kCollect + threadIdx.x;
-    const bool v = i < n && keys[i].valid;
-    const unsigned long long m = __ballot(v);
-    if ((threadIdx.x & 63) == 0 && m) atomicAdd(&c, (unsigned)__popcll(m));
-    __syncthreads();
-    if (threadIdx.x == 0) counts[blockIdx.x] = c;
+struct CollectArgs {
+    const Surf* keys;
+    int n, groups;
+    unsigned* counts;          // per group; then its exclusive prefix
+    unsigned* total;
+    unsigned* arrived;         // groups that have counted; 0 between calls
+    unsigned long long* bits;  // 16 words per group
+};
+// between work-groups of a launch: through the memory that all XCDs share
+__device__ __forceinline__ void store_shared(unsigned* p, unsigned v) {
+    __hip_atomic_store(FU_G(unsigned, p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// the exclusive prefix of the group counts, in place, and their total: one work-group of
-// kPrefixLanes lanes, lane t owning a run of consecutive counts, the runs' sums scanned across
-// the work-group (integer sums: the same as one lane walking the counts in order)
-constexpr int kPrefixLanes = 1024;
-__global__ __launch_bounds__(kPrefixLanes) void k_collect_prefix(unsigned* counts, int groups, unsigned* total) {
-    __shared__ unsigned wsum[kPrefixLanes / 64];
-    const int per = (groups + kPrefixLanes - 1) / kPrefixLanes;
-    const int b = min(groups, (int)threadIdx.x * per), e = min(groups, b + per);
+__device__ __forceinline__ unsigned load_shared(const unsigned* p) {
+    return __hip_atomic_load(FU_G(const unsigned, p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__global__ __launch_bounds__(kCollect) void k_collect_count(CollectArgs a) {
+    __shared__ unsigned wsum[kCollect / 64];
+    __shared__ int last;
+    const int i = blockIdx.x * kCollect + threadIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const unsigned long long m = __ballot(i < a.n && a.keys[i].valid);
+    if (lane == 0) {
+        a.bits[blockIdx.x * (kCollect / 64) + w] = m;
+        wsum[w] = (unsigned)__popcll(m);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned c = 0;
+        for (int k = 0; k < kCollect / 64; ++k) c += wsum[k];
+        store_shared(&a.counts[blockIdx.x], c);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the count is in place
+        last = __hip_atomic_fetch_add(FU_G(unsigned, a.arrived), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+               (unsigned)a.groups - 1u;
+    }
+    __syncthreads();
+    if (!last) return;  // uniform
+    // lane t owns a run of consecutive counts; the runs' sums are scanned across the work-group
+    // (integer sums: the same as one lane walking the counts in order)
+    const int per = (a.groups + kCollect - 1) / kCollect;
+    const int b = min(a.groups, (int)threadIdx.x * per), e = min(a.groups, b + per);
     unsigned own = 0;
-    for (int g = b; g < e; ++g) own += counts[g];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    for (int g = b; g < e; ++g) own += load_shared(&a.counts[g]);
     unsigned x = own;  // inclusive scan over the wave
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
@@ -136,43 +164,59 @@ __global__ __launch_bounds__(kPrefixLanes) void k_collect_prefix(unsigned* count
     __syncthreads();
     unsigned before = 0, all = 0;
 #pragma unroll
-    for (int k = 0; k < kPrefixLanes / 64; ++k) {
+    for (int k = 0; k < kCollect / 64; ++k) {
         const unsigned c = wsum[k];
         before += k < w ? c : 0u;
         all += c;
     }
     unsigned run = before + x - own;
     for (int g = b; g < e; ++g) {
-        const unsigned c = counts[g];
-        counts[g] = run;
+        const unsigned c = load_shared(&a.counts[g]);
+        a.counts[g] = run;
         run += c;
     }
-    if (threadIdx.x == 0) *total = all;
-}
-__global__ void k_collect_scatter(const Surf* keys, int n, const unsigned* base, Surf* out, unsigned cap) {
-    __shared__ unsigned wave_base[kCollect / 64];
-    const int i = blockIdx.x * kCollect + threadIdx.x;
-    const bool v = i < n && keys[i].valid;
-    const unsigned long long m = __ballot(v);
-    const int w = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) wave_base[w] = (unsigned)__popcll(m);
-    __syncthreads();
     if (threadIdx.x == 0) {
-        unsigned s = 0;
-        for (int k = 0; k < kCollect / 64; ++k) {
-            const unsigned c = wave_base[k];
-            wave_base[k] = s;
-            s += c;
-        }
+        *a.total = all;
+        *a.arrived = 0u;
     }
-    __syncthreads();
-    if (!v) return;
-    const unsigned below = __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-    const unsigned j = base[blockIdx.x] + wave_base[w] + below;
-    if (j > 0 && j < cap) {
-        const uint4* src = reinterpret_cast<const uint4*>(&keys[i]);
-        uint4* dst = reinterpret_cast<uint4*>(&out[j]);
-        for (int q = 0; q < (int)(sizeof(Surf) / 16); ++q) dst[q] = src[q];
+}
+// A wave per word of bits, 16 lanes per record, four records at a time.  kPack: the descriptors
+// alone, packed for the matcher, and each one's slot (record 0 as the zeros that CollectKeys
+// leaves there, slot -1); else whole records into `out`, where they are below `cap`.
+template <bool kPack>
+__global__ __launch_bounds__(256) void k_collect_copy(CollectArgs a, Surf* out, float* desc, int* slot, unsigned cap) {
+    const int word = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    constexpr int kWords = kCollect / 64;
+    if (word >= a.groups * kWords) return;  // uniform
+    unsigned long long m = a.bits[word];
+    if (!m) return;  // uniform
+    const int w = word % kWords;
+    // valid records of the group's words before this one
+    unsigned before = 0;
+    if (lane < w) before = (unsigned)__popcll(a.bits[word - w + lane]);
+#pragma unroll
+    for (int d = 1; d < kWords; d <<= 1) before += __shfl_xor(before, d);
+    before = (unsigned)__builtin_amdgcn_readfirstlane((int)before);
+    const unsigned j0 = a.counts[word / kWords] + before;
+    const int sub = lane >> 4, q = lane & 15, n = __popcll(m);
+    for (int k = 0; k < sub; ++k) m &= m - 1;
+    for (int r = sub; r < n; r += 4) {
+        const int i = word * 64 + __builtin_ctzll(m);
+        const unsigned j = j0 + r;
+        const uint4* src = reinterpret_cast<const uint4*>(&a.keys[i]);
+        if constexpr (kPack) {
+            static_assert(offsetof(Surf, desc) == 32, "two 16-byte words ahead of the descriptor");
+            uint4 v = src[2 + q];
+            if (j == 0) v = make_uint4(0u, 0u, 0u, 0u);
+            reinterpret_cast<uint4*>(desc)[(size_t)j * 16 + q] = v;
+            if (q == 0) slot[j] = j == 0 ? -1 : i;
+        } else if (j > 0 && j < cap) {
+            uint4* dst = reinterpret_cast<uint4*>(&out[j]);
+            dst[q] = src[q];
+            if (q < 2) dst[16 + q] = src[16 + q];
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) m &= m - 1;
     }
 }
 
@@ -181,12 +225,13 @@ __device__ __forceinline__ float clamp1(float a) {  // KeyPoints.cu:6-10
     a = a < 1.f ? a : 1.f;
     return a;
 }
-__device__ __forceinline__ f3 spos(const Surf& s) { return mk3(s.pos[0], s.pos[1], s.pos[2]); }
-__device__ __forceinline__ f4 snrm(const Surf& s) { return mk4(s.normal[0], s.normal[1], s.normal[2], s.normal[3]); }
+__device__ __forceinline__ f3 spos(const SurfHead& s) { return mk3(s.pos[0], s.pos[1], s.pos[2]); }
+__device__ __forceinline__ f4 snrm(const SurfHead& s) { return mk4(s.normal[0], s.normal[1], s.normal[2], s.normal[3]); }
 __device__ __forceinline__ float dot4f(f4 a, f4 b) { return a.x * b.x + a.y * b.y + a.z * b.z + a.w * b.w; }
 
-// BuildAdjecencyMatrixKernel (KeyPoints.cu:12-57), one lane per entry of the n x n matrix
-__global__ void k_adjacency(const Surf* frame, const Surf* map, const float* dist, int n, float* out) {
+// BuildAdjecencyMatrixKernel (KeyPoints.cu:12-57), one lane per entry of the n x n matrix; the
+// records' heads, `stride` heads apart
+__global__ void k_adjacency(const SurfHead* frame, const SurfHead* map, int stride, const float* dist, int n, float* out) {
     const int x = blockIdx.x * 16 + (threadIdx.x & 15);
     const int y = blockIdx.y * 16 + (threadIdx.x >> 4);
     if (x >= n || y >= n) return;
@@ -194,7 +239,7 @@ __global__ void k_adjacency(const Surf* frame, const Surf* map, const float* dis
     if (x == y) {
         score = expf(-dist[x]);
     } else {
-        const Surf &m0 = map[x], &m1 = map[y], &f0 = frame[x], &f1 = frame[y];
+        const SurfHead &m0 = map[x * stride], &m1 = map[y * stride], &f0 = frame[x * stride], &f1 = frame[y * stride];
         const float d00 = norm(sub(spos(f0), spos(f1)));
         const float d01 = norm(sub(spos(m0), spos(m1)));
         const f3 e10 = normalised(sub(spos(f0), spos(f1)));
@@ -222,7 +267,9 @@ __global__ void k_adjacency(const Surf* frame, const Surf* map, const float* dis
 struct fu_keymap {
     fu_keymap_params p;
     KeyArgs a;
-    unsigned* aux = nullptr;    // [0] keys left in a round, [1] collect total, then group counts
+    unsigned* aux = nullptr;    // [0] keys left in a round, [1] collect total, [2] groups counted,
+                                // from [4] a 64-slot word of valid bits each, then group counts
+    int dev = -1;               // the device the map was created on
     unsigned char* done = nullptr;  // per key of an insert call, grown on demand
     int* bucket = nullptr;
     int cap = 0;
@@ -255,6 +302,12 @@ extern "C" fu_status fu_keymap_destroy(fu_keymap* k) {
 
 static int n_slots(const fu_keymap* k) { return k->a.max_keys * k->a.nbuckets; }
 static int n_groups(const fu_keymap* k) { return (n_slots(k) + kCollect - 1) / kCollect; }
+static CollectArgs collect_args(const fu_keymap* k) {
+    const int g = n_groups(k);
+    unsigned* bits = k->aux + 4;
+    return CollectArgs{k->a.keys, n_slots(k),         g, bits + (size_t)g * (2 * kCollect / 64), k->aux + 1,
+                       k->aux + 2, (unsigned long long*)bits};
+}
 
 extern "C" fu_status fu_keymap_create(const fu_keymap_params* p, fu_keymap** out) {
     if (!p || !out) return api_error(FU_ERR_ARG, "fu_keymap_create: null argument");
@@ -270,14 +323,15 @@ extern "C" fu_status fu_keymap_create(const fu_keymap_params* p, fu_keymap** out
     const size_t n = (size_t)n_slots(k);
     if (hipMalloc(&k->a.keys, n * sizeof(Surf)) != hipSuccess || hipMalloc(&k->a.mutex, n * 4) != hipSuccess ||
         hipMalloc(&k->a.owner, (size_t)p->max_keys * 4) != hipSuccess ||
-        hipMalloc(&k->aux, (2 + (size_t)n_groups(k)) * 4) != hipSuccess) {
+        hipMalloc(&k->aux, (4 + (size_t)n_groups(k) * (2 * kCollect / 64 + 1)) * 4) != hipSuccess) {
         (void)hipGetLastError();
         fu_keymap_destroy(k);
         return api_error(FU_ERR_NOMEM, "fu_keymap_create: allocation failed");
     }
     // records start zeroed (ResetKeys clears only the valid flags, so a record's other bytes
     // keep what the last key there left)
-    if (hipMemset(k->a.keys, 0, n * sizeof(Surf)) != hipSuccess) {
+    k->dev = current_device();
+    if (hipMemset(k->a.keys, 0, n * sizeof(Surf)) != hipSuccess || hipMemset(k->aux, 0, 16) != hipSuccess) {
         (void)hipGetLastError();
         fu_keymap_destroy(k);
         return api_error(FU_ERR_HIP, "fu_keymap_create: clearing the records failed");
@@ -341,16 +395,40 @@ extern "C" fu_status fu_insert_key_points(fu_keymap* k, fu_surf* keys, int32_t* 
 extern "C" fu_status fu_collect_key_points(fu_keymap* k, fu_surf* out, uint32_t cap, uint32_t* n_keys, fu_stream s) {
     if (!k || !n_keys || (cap && !out)) return api_error(FU_ERR_ARG, "fu_collect_key_points: null argument");
     hipStream_t hs = (hipStream_t)s;
-    const int n = n_slots(k), g = n_groups(k);
-    hipLaunchKernelGGL(k_collect_count, dim3(g), dim3(kCollect), 0, hs, (const Surf*)k->a.keys, n, k->aux + 2);
-    hipLaunchKernelGGL(k_collect_prefix, dim3(1), dim3(kPrefixLanes), 0, hs, k->aux + 2, g, k->aux + 1);
-    if (cap) hipLaunchKernelGGL(k_collect_scatter, dim3(g), dim3(kCollect), 0, hs, (const Surf*)k->a.keys, n, k->aux + 2,
-                                (Surf*)out, cap);
+    const CollectArgs a = collect_args(k);
+    hipLaunchKernelGGL(k_collect_count, dim3(a.groups), dim3(kCollect), 0, hs, a);
+    if (cap)
+        hipLaunchKernelGGL(k_collect_copy<false>, dim3(a.groups * (kCollect / 256)), dim3(256), 0, hs, a, (Surf*)out,
+                           nullptr, nullptr, cap);
     KM_HIP(hipGetLastError());
-    KM_HIP(hipMemcpyAsync(n_keys, k->aux + 1, 4, hipMemcpyDeviceToHost, hs));
-    KM_HIP(hipStreamSynchronize(hs));
+    KM_HIP(mail_read(k->dev, n_keys, a.total, 4, hs));
     return FU_OK;
 }
+
+namespace fu {
+// the number of valid keys; synchronises the stream
+fu_status keymap_count(fu_keymap* k, uint32_t* n_keys, hipStream_t s) {
+    return fu_collect_key_points(k, nullptr, 0, n_keys, (fu_stream)s);
+}
+// after keymap_count with nothing inserted since, for its n keys: their descriptors (n x 64,
+// 16-byte aligned) and slots, key 0 as zeros and slot -1
+fu_status keymap_pack(fu_keymap* k, float* desc, int32_t* slot, hipStream_t s) {
+    const CollectArgs a = collect_args(k);
+    hipLaunchKernelGGL(k_collect_copy<true>, dim3(a.groups * (kCollect / 256)), dim3(256), 0, s, a, nullptr, desc, slot, 0u);
+    KM_HIP(hipGetLastError());
+    return FU_OK;
+}
+const SurfHead* keymap_heads(const fu_keymap* k) { return (const SurfHead*)k->a.keys; }
+int keymap_device(const fu_keymap* k) { return k->dev; }
+// fu_build_adjacency_matrix on the records' heads alone
+fu_status build_adjacency(const SurfHead* frame, const SurfHead* map, int stride, const float* dist, int n, float* matrix,
+                          hipStream_t s) {
+    const dim3 grid((n + 15) / 16, (n + 15) / 16);
+    hipLaunchKernelGGL(k_adjacency, grid, dim3(256), 0, s, frame, map, stride, dist, n, matrix);
+    KM_HIP(hipGetLastError());
+    return FU_OK;
+}
+}  // namespace fu
 
 extern "C" fu_status fu_keymap_read(fu_keymap* k, fu_surf* host, fu_stream s) {
     if (!k || !host) return api_error(FU_ERR_ARG, "fu_keymap_read: null argument");
@@ -365,9 +443,6 @@ extern "C" fu_status fu_build_adjacency_matrix(const fu_surf* frame_keys, const 
         return api_error(FU_ERR_ARG, "fu_build_adjacency_matrix: null argument or negative size");
     if (n > 46340) return api_error(FU_ERR_ARG, "fu_build_adjacency_matrix: %d pairs (the matrix index is 32-bit)", n);
     if (n == 0) return FU_OK;
-    const dim3 grid((n + 15) / 16, (n + 15) / 16);
-    hipLaunchKernelGGL(k_adjacency, grid, dim3(256), 0, (hipStream_t)s, (const Surf*)frame_keys, (const Surf*)map_keys,
-                       dist, n, matrix);
-    KM_HIP(hipGetLastError());
-    return FU_OK;
+    return build_adjacency((const SurfHead*)frame_keys, (const SurfHead*)map_keys, kSurfHeads, dist, n, matrix,
+                           (hipStream_t)s);
 }

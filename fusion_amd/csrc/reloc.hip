@@ -8,15 +8,14 @@
 #include <math.h>
 #include <stddef.h>
 #include <stdint.h>
-#include <string.h>
 
 #include <algorithm>
 #include <cmath>
-#include <system_error>
-#include <thread>
 #include <vector>
 
 #include "fu_api.h"
+#include "fu_keys.h"
+#include "fu_mail.h"
 
 using namespace fu;
 
@@ -335,38 +334,44 @@ static int match_chunk_len(int nq, int nt) {
 // matrix back to the host as the reference does:
 //   k_rank_sums   the column sums (cv::cuda::reduce over rows): each column's rows in order,
 //                 summed in double and rounded to float (OpenCV's order is its own).  A
-//                 work-group takes 64 columns: all its lanes stage tiles of kSumRows rows in
-//                 LDS, and one wave adds them, a lane per column;
+//                 work-group takes 16 columns: all its lanes stage tiles of kSumRows rows in
+//                 LDS, and 16 lanes add them, one per column;
 //   k_rank_order  the pairs by rank, largest first (cv::sortIdx descending): a pair's position
 //                 is the number of ranks above its own, ties going to the lower index
 //                 (std::sort leaves them in no fixed order), counted against LDS tiles of the
-//                 ranks by four waves a quarter each and added; a NaN rank counts as -inf, so
+//                 ranks by sixteen waves a part each and added; a NaN rank counts as -inf, so
 //                 the positions are a permutation;
-//   k_subgraphs   one 1024-lane work-group per list: the head and the pairs ranked after it
+//   k_select      one 1024-lane work-group per list: the head and the pairs ranked after it
 //                 with C[head][pair] > min_score, kept in rank order by a block-wide ballot
-//                 prefix until max_sel are selected; then the refinement test of each selected
-//                 pair against every later pair of the list, one wave per pair, its lanes
-//                 over the later pairs (the test is an "any", so their order is free).
+//                 prefix until max_sel are selected;
+//   k_refine      the refinement test of each selected pair against every later pair of the list,
+//                 one wave per pair, its lanes over the later pairs (the test is an "any", so
+//                 their order is free).  Bound by the latency of its gathers: the ten work-groups
+//                 of k_select took 89 us for both parts of ten lists of 400, most CUs idle, the
+//                 two launches take 19 us.
 constexpr int kSelLanes = 1024;
 constexpr int kMaxSelect = 1024;
 
-constexpr int kSumRows = 128;  // rows per LDS tile of k_rank_sums (32 KB)
+constexpr int kSumCols = 16, kSumRows = 512;  // columns and rows per LDS tile of k_rank_sums (32 KB)
 
-// launch: ceil(n / 64) work-groups of 256 lanes.  Lane t loads columns 4 (t & 15) .. +3 of
-// rows t >> 4, (t >> 4) + 16, ... of a tile (eight 16-byte loads when the row is whole and
-// aligned), the next tile's loads issued before wave 0 adds the current one from LDS.
+// launch: ceil(n / kSumCols) work-groups of 256 lanes.  Lane t loads columns 4 (t & 3) .. +3 of
+// rows t >> 2, (t >> 2) + 64, ... of a tile (eight 16-byte loads when the row is whole and
+// aligned), the next tile's loads issued before the current one is added from LDS.  Bound by the
+// columns' serial sums; with 64 columns and 128 rows a tile the trips for the tiles came to more:
+// n = 1125, 20 -> 14 us.
 __global__ __launch_bounds__(256) void k_rank_sums(const float* C, int n, float* rank) {
-    __shared__ __align__(16) float tile[kSumRows][64];  // written as 16-byte words
-    const int tid = threadIdx.x, col = tid & 63;
-    const int c0 = blockIdx.x * 64;
-    const int q = (tid & 15) * 4, r_lane = tid >> 4;
+    __shared__ __align__(16) float tile[kSumRows][kSumCols];  // written as 16-byte words
+    const int tid = threadIdx.x, col = tid & (kSumCols - 1);
+    const int c0 = blockIdx.x * kSumCols;
+    constexpr int kLoad = 256 / (kSumCols / 4);  // rows loaded at once
+    const int q = tid % (kSumCols / 4) * 4, r_lane = tid / (kSumCols / 4);
     // whole 16-byte words: an aligned matrix and n a multiple of 4 keep every row start aligned
     const bool vec = ((uintptr_t)C & 15) == 0 && (n & 3) == 0 && c0 + q + 3 < n;
-    float4 buf[kSumRows / 16];
+    float4 buf[kSumRows / kLoad];
     auto fetch = [&](int r0) {
 #pragma unroll
-        for (int k = 0; k < kSumRows / 16; ++k) {
-            const int r = r0 + r_lane + 16 * k;
+        for (int k = 0; k < kSumRows / kLoad; ++k) {
+            const int r = r0 + r_lane + kLoad * k;
             float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
             if (r < n) {
                 const float* row = C + (size_t)r * n + c0 + q;
@@ -382,31 +387,33 @@ __global__ __launch_bounds__(256) void k_rank_sums(const float* C, int n, float*
             buf[k] = v;
         }
     };
-    double s = 0;  // wave 0: column c0 + col
+    double s = 0;  // the first lanes: column c0 + col
     fetch(0);
     for (int r0 = 0; r0 < n; r0 += kSumRows) {
         __syncthreads();  // the previous tile is summed
 #pragma unroll
-        for (int k = 0; k < kSumRows / 16; ++k) *reinterpret_cast<float4*>(&tile[r_lane + 16 * k][q]) = buf[k];
+        for (int k = 0; k < kSumRows / kLoad; ++k) *reinterpret_cast<float4*>(&tile[r_lane + kLoad * k][q]) = buf[k];
         __syncthreads();
         if (r0 + kSumRows < n) fetch(r0 + kSumRows);
         // rows past n hold +0, which leaves the sum as it is (it starts at +0 and so is never
-        // -0), so every tile is summed whole
-        if (tid < 64) {
+        // -0), so the last tile is summed to a multiple of 16 rows
+        if (tid < kSumCols) {
+            const int rows = min(kSumRows, (n - r0 + 15) & ~15);
 #pragma unroll 16
-            for (int r = 0; r < kSumRows; ++r) s += (double)tile[r][col];
+            for (int r = 0; r < rows; ++r) s += (double)tile[r][col];
         }
     }
-    if (tid < 64 && c0 + col < n) rank[c0 + col] = (float)s;
+    if (tid < kSumCols && c0 + col < n) rank[c0 + col] = (float)s;
 }
 
 __device__ __forceinline__ float rank_key(float v) { return isnan(v) ? -INFINITY : v; }
 
-// launch: ceil(n / 64) work-groups of 256 lanes; lane (w, l) counts for pair 64 * group + l
-// against entries w * 256 .. w * 256 + 255 of every 1024-rank tile
-__global__ __launch_bounds__(256) void k_rank_order(const float* rank, int n, int* order) {
+// launch: ceil(n / 64) work-groups of 1024 lanes; lane (w, l) counts for pair 64 * group + l
+// against entries w * 64 .. w * 64 + 63 of every 1024-rank tile (with four waves a tile's 256
+// entries a lane were 20 us at n = 1125, now 7)
+__global__ __launch_bounds__(1024) void k_rank_order(const float* rank, int n, int* order) {
     __shared__ float tile[1024];
-    __shared__ int part[4][64];
+    __shared__ int part[16][64];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int x = blockIdx.x * 64 + lane;
     const float kx = x < n ? rank_key(rank[x]) : 0.f;
@@ -415,18 +422,24 @@ __global__ __launch_bounds__(256) void k_rank_order(const float* rank, int n, in
         __syncthreads();
         // slots past n hold -inf: never above a rank, and equal to one only with an index
         // above it, so they never count
-        for (int k = threadIdx.x; k < 1024; k += 256) tile[k] = base + k < n ? rank_key(rank[base + k]) : -INFINITY;
+        const int k0 = base + threadIdx.x;
+        tile[threadIdx.x] = k0 < n ? rank_key(rank[k0]) : -INFINITY;
         __syncthreads();
-        const int lo = w * 256;
+        const int lo = w * 64;
 #pragma unroll 16
-        for (int k = lo; k < lo + 256; ++k) {
+        for (int k = lo; k < lo + 64; ++k) {
             const float ky = tile[k];
             pos += (ky > kx) || (ky == kx && base + k < x);
         }
     }
     part[w][lane] = pos;
     __syncthreads();
-    if (w == 0 && x < n) order[part[0][lane] + part[1][lane] + part[2][lane] + part[3][lane]] = x;
+    if (w == 0 && x < n) {
+        int p = 0;
+#pragma unroll
+        for (int k = 0; k < 16; ++k) p += part[k][lane];
+        order[p] = x;
+    }
 }
 
 struct SelArgs {
@@ -435,8 +448,8 @@ struct SelArgs {
     int n, max_sel;
     float min_score;
     int* n_selected;  // per list
-    int* n_refined;   // per list
-    int* refined;     // max_sel per list
+    int* n_refined;   // per list; k_refine's count of ended work-groups until the last ends
+    int* refined;     // max_sel per list; the selected pairs until then, the kept ones marked
 };
 
 // the exclusive prefix of `flag` over the work-group (lanes in order) and the total
@@ -457,91 +470,120 @@ __device__ __forceinline__ int block_prefix(bool flag, int* wsum, int& total) {
     return before + in_wave;
 }
 
-__global__ __launch_bounds__(kSelLanes) void k_subgraphs(SelArgs a) {
-    __shared__ int sel[kMaxSelect];
-    __shared__ float hs[kMaxSelect];  // C[head][sel[k]]
+__global__ __launch_bounds__(kSelLanes) void k_select(SelArgs a) {
     __shared__ int wsum[kSelLanes / 64];
     const int i = blockIdx.x, tid = threadIdx.x;
+    if (tid == 0) a.n_refined[i] = 0;
     if (i >= a.n) {  // no pairs from this rank on (Tracking.cc:538)
-        if (tid == 0) a.n_selected[i] = a.n_refined[i] = 0;
+        if (tid == 0) a.n_selected[i] = 0;
         return;
     }
     const int head = a.order[i];
     const float* Ch = a.C + (size_t)head * a.n;
+    int* sel = a.refined + (size_t)i * a.max_sel;
     int count = 1;  // the head is always taken (:544-548)
-    if (tid == 0) {
-        sel[0] = head;
-        hs[0] = Ch[head];
-    }
+    if (tid == 0) sel[0] = head;
     for (int base = i + 1; base < a.n && count < a.max_sel; base += kSelLanes) {
         const int j = base + tid;
         int idx = 0;
-        float sc = 0.f;
         bool f = false;
         if (j < a.n) {
             idx = a.order[j];
-            sc = Ch[idx];
-            f = sc > a.min_score;  // :551-555
+            f = Ch[idx] > a.min_score;  // :551-555
         }
         int total;
         const int slot = count + block_prefix(f, wsum, total);
-        if (f && slot < a.max_sel) {
-            sel[slot] = idx;
-            hs[slot] = sc;
-        }
+        if (f && slot < a.max_sel) sel[slot] = idx;
         count = min(count + total, a.max_sel);  // the same in every lane
     }
-    __syncthreads();
     if (tid == 0) a.n_selected[i] = count;
-    if (count < 3) {  // no PoseEstimate from fewer than three (:565)
-        if (tid == 0) a.n_refined[i] = 0;
-        return;
-    }
+}
+
+// launch: (ceil((max_sel - 1) / 4), lists) work-groups of 256 lanes.  The work-group that ends last
+// of a list's (counted in its n_refined, the marks written through to the memory that all XCDs
+// share) moves the marked pairs together.
+constexpr int kMark = (int)0x80000000u;  // pair indices are below 46340
+__global__ __launch_bounds__(256) void k_refine(SelArgs a) {
+    __shared__ int last, wsum[4];
+    const int i = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    const int count = a.n_selected[i];
+    if (count < 3) return;  // no PoseEstimate from fewer than three (:565)
+    const int groups = (count + 2) / 4;
+    if ((int)blockIdx.x >= groups) return;
+    int* sel = a.refined + (size_t)i * a.max_sel;
+    const float* Ch = a.C + (size_t)(sel[0] & ~kMark) * a.n;
     // the t-th pair is kept unless a later one is nearly exclusive with it and scores higher
-    // with the head (:567-582); the head (t = 0) is never kept.  Wave w tests pairs w + 1,
-    // w + 17, ..., its lanes over the later pairs 64 at a time.
-    __shared__ unsigned char kept[kMaxSelect];
-    const int lane = tid & 63, wid = tid >> 6;
-    for (int t = 1 + wid; t < count; t += kSelLanes / 64) {
-        const int av = sel[t];
-        const float ha = hs[t];
+    // with the head (:567-582); the head (t = 0) is never kept
+    const int t = 1 + blockIdx.x * 4 + wid;
+    if (t < count) {
+        const int av = sel[t] & ~kMark;
+        const float ha = Ch[av];
         const float* Ca = a.C + (size_t)av * a.n;
         bool drop = false;
 #pragma unroll 4
         for (int l = t + 1 + lane; l < count; l += 64) {
-            const int b = sel[l];
+            const int b = sel[l] & ~kMark;
             const bool x = Ca[b] < 5e-3f || a.C[(size_t)b * a.n + av] < 5e-3f;
-            drop = drop || (hs[l] > ha && x);
+            drop = drop || (Ch[b] > ha && x);
         }
-        if (lane == 0) kept[t] = 0;
-        if (__ballot(drop) == 0ull && lane == 0) kept[t] = 1;
+        if (__ballot(drop) == 0ull && lane == 0)
+            __hip_atomic_store(FU_G(int, sel + t), av | kMark, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the wave's mark is in place
     __syncthreads();
-    const bool keep = tid >= 1 && tid < count && kept[tid];
-    int total;
-    const int slot = block_prefix(keep, wsum, total);
-    if (keep) a.refined[(size_t)i * a.max_sel + slot] = sel[tid];
+    if (tid == 0)
+        last = __hip_atomic_fetch_add(FU_G(int, a.n_refined + i), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == groups - 1;
+    __syncthreads();
+    if (!last) return;  // uniform
+    int v[kMaxSelect / 256];
+#pragma unroll
+    for (int k = 0; k < kMaxSelect / 256; ++k) {
+        const int p = k * 256 + tid;
+        v[k] = p < count ? __hip_atomic_load(FU_G(int, sel + p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+    }
+    unsigned long long m[kMaxSelect / 256];
+#pragma unroll
+    for (int k = 0; k < kMaxSelect / 256; ++k) m[k] = __ballot((v[k] & kMark) != 0);  // every pair has been read
+    int total = 0;
+#pragma unroll
+    for (int k = 0; k < kMaxSelect / 256; ++k) {
+        __syncthreads();  // by every wave; the previous sums are read
+        if (lane == 0) wsum[wid] = __popcll(m[k]);
+        __syncthreads();
+        int at = total + __popcll(m[k] & ((1ull << lane) - 1ull));
+        for (int w = 0; w < 4; ++w) {
+            at += w < wid ? wsum[w] : 0;
+            total += wsum[w];
+        }
+        if ((v[k] & kMark) != 0) sel[at] = v[k] & ~kMark;
+    }
     if (tid == 0) a.n_refined[i] = total;
 }
 
 // ---------------------------------------------------------------------------- pose
-// 3x3 helpers in double, row-major
+// PoseEstimate (Optimization/Solver.cc:6-183) in double.  A hypothesis is a function of its draw
+// alone, so the device counts the inliers of many at once (k_hypotheses) and the host walks the
+// counts as the reference walks its iterations.  Both sides run the functions below, every
+// operation of which is an IEEE one: the same counts and the same pose, whichever side counts.
+#define FU_HD __host__ __device__ __forceinline__
+
+// 3x3 helpers, row-major
 struct M3d {
     double a[9];
 };
-M3d mul(const M3d& x, const M3d& y) {
+FU_HD M3d mul(const M3d& x, const M3d& y) {
     M3d r;
     for (int i = 0; i < 3; ++i)
         for (int j = 0; j < 3; ++j) r.a[i * 3 + j] = x.a[i * 3] * y.a[j] + x.a[i * 3 + 1] * y.a[3 + j] + x.a[i * 3 + 2] * y.a[6 + j];
     return r;
 }
-M3d transpose(const M3d& x) {
+FU_HD M3d transpose(const M3d& x) {
     M3d r;
     for (int i = 0; i < 3; ++i)
         for (int j = 0; j < 3; ++j) r.a[i * 3 + j] = x.a[j * 3 + i];
     return r;
 }
-double det(const M3d& m) {
+FU_HD double det(const M3d& m) {
     const double* a = m.a;
     return a[0] * (a[4] * a[8] - a[5] * a[7]) - a[1] * (a[3] * a[8] - a[5] * a[6]) + a[2] * (a[3] * a[7] - a[4] * a[6]);
 }
@@ -550,13 +592,14 @@ double det(const M3d& m) {
 // Jacobi on the columns of Ab gives Ab V = U S; a singular vector of a zero singular value
 // (three points of a sample span a plane) is completed as the cross product of the other two,
 // on both sides, so such a sample yields the proper rotation.
-M3d kabsch(const M3d& Ab) {
+FU_HD M3d kabsch(const M3d& Ab) {
     double A[9], V[9] = {1, 0, 0, 0, 1, 0, 0, 0, 1};
-    memcpy(A, Ab.a, sizeof(A));
+    for (int k = 0; k < 9; ++k) A[k] = Ab.a[k];
     for (int sweep = 0; sweep < 40; ++sweep) {
         double off = 0;
-        for (int p = 0; p < 2; ++p)
-            for (int q = p + 1; q < 3; ++q) {
+#pragma unroll
+        for (int pq = 0; pq < 3; ++pq) {
+                const int p = pq < 2 ? 0 : 1, q = pq < 1 ? 1 : 2;
                 double al = 0, be = 0, ga = 0;
                 for (int i = 0; i < 3; ++i) {
                     al += A[i * 3 + p] * A[i * 3 + p];
@@ -579,19 +622,38 @@ M3d kabsch(const M3d& Ab) {
             }
         if (off < 1e-15) break;
     }
-    // singular values (column norms), largest first
+    // singular values (column norms), largest first: the columns in order, a later one ahead of an
+    // earlier where it is strictly larger
     double sv[3];
-    int ord[3] = {0, 1, 2};
     for (int k = 0; k < 3; ++k) sv[k] = sqrt(A[k] * A[k] + A[3 + k] * A[3 + k] + A[6 + k] * A[6 + k]);
-    std::sort(ord, ord + 3, [&](int x, int y) { return sv[x] > sv[y]; });
+    auto exchange = [&](int x, int y) {
+        auto swap = [](double& u, double& v) {
+            const double w = u;
+            u = v;
+            v = w;
+        };
+        swap(sv[x], sv[y]);
+        for (int i = 0; i < 3; ++i) {
+            swap(A[i * 3 + x], A[i * 3 + y]);
+            swap(V[i * 3 + x], V[i * 3 + y]);
+        }
+    };
+    if (sv[1] > sv[0]) exchange(0, 1);
+    if (sv[2] > sv[0]) {
+        exchange(1, 2);
+        exchange(0, 1);
+    } else if (sv[2] > sv[1]) {
+        exchange(1, 2);
+    }
     double U[9], W[9];
     for (int c = 0; c < 3; ++c) {
-        const int k = ord[c];
-        for (int i = 0; i < 3; ++i) W[i * 3 + c] = V[i * 3 + k];
-        const double inv = sv[k] > 0 ? 1 / sv[k] : 0;
-        for (int i = 0; i < 3; ++i) U[i * 3 + c] = A[i * 3 + k] * inv;
+        const double inv = sv[c] > 0 ? 1 / sv[c] : 0;
+        for (int i = 0; i < 3; ++i) {
+            W[i * 3 + c] = V[i * 3 + c];
+            U[i * 3 + c] = A[i * 3 + c] * inv;
+        }
     }
-    if (sv[ord[2]] <= 1e-12 * fmax(sv[ord[0]], 1e-300)) {
+    if (sv[2] <= 1e-12 * fmax(sv[0], 1e-300)) {
         // rank <= 2: third columns as cross products of the first two
         U[2] = U[3] * U[7] - U[6] * U[4];
         U[5] = U[6] * U[1] - U[0] * U[7];
@@ -601,40 +663,238 @@ M3d kabsch(const M3d& Ab) {
         W[8] = W[0] * W[4] - W[3] * W[1];
     }
     M3d u, w;
-    memcpy(u.a, U, sizeof(U));
-    memcpy(w.a, W, sizeof(W));
+    for (int k = 0; k < 9; ++k) {
+        u.a[k] = U[k];
+        w.a[k] = W[k];
+    }
     return mul(u, transpose(w));
 }
 
 struct V3d {
     double x, y, z;
 };
-V3d operator-(V3d a, V3d b) { return {a.x - b.x, a.y - b.y, a.z - b.z}; }
-V3d operator+(V3d a, V3d b) { return {a.x + b.x, a.y + b.y, a.z + b.z}; }
-V3d operator/(V3d a, double s) { return {a.x / s, a.y / s, a.z / s}; }
-V3d rot(const M3d& R, V3d v) {
+FU_HD V3d operator-(V3d a, V3d b) { return {a.x - b.x, a.y - b.y, a.z - b.z}; }
+FU_HD V3d operator+(V3d a, V3d b) { return {a.x + b.x, a.y + b.y, a.z + b.z}; }
+FU_HD V3d operator/(V3d a, double s) { return {a.x / s, a.y / s, a.z / s}; }
+FU_HD V3d rot(const M3d& R, V3d v) {
     return {R.a[0] * v.x + R.a[1] * v.y + R.a[2] * v.z, R.a[3] * v.x + R.a[4] * v.y + R.a[5] * v.z,
             R.a[6] * v.x + R.a[7] * v.y + R.a[8] * v.z};
 }
-double vnorm(V3d v) { return sqrt(v.x * v.x + v.y * v.y + v.z * v.z); }
-V3d vcross(V3d a, V3d b) { return {a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x}; }
-void outer_add(M3d& m, V3d a, V3d b) {
+FU_HD double vnorm(V3d v) { return sqrt(v.x * v.x + v.y * v.y + v.z * v.z); }
+FU_HD V3d vcross(V3d a, V3d b) { return {a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x}; }
+FU_HD void outer_add(M3d& m, V3d a, V3d b) {
     const double av[3] = {a.x, a.y, a.z}, bv[3] = {b.x, b.y, b.z};
     for (int i = 0; i < 3; ++i)
         for (int j = 0; j < 3; ++j) m.a[i * 3 + j] += av[i] * bv[j];
 }
 
-// the sample generator: splitmix64 in place of the reference's srand(clock) / rand()
-struct Rng {
-    uint64_t s;
-    uint32_t next(uint32_t n) {
-        uint64_t z = (s += 0x9E3779B97F4A7C15ull);
-        z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-        z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
-        z ^= z >> 31;
-        return (uint32_t)((z >> 32) % n);
+// number k (from 0) of the sample generator, below n: splitmix64 in place of the reference's
+// srand(clock) / rand(), whose state is seed + (k + 1) times a constant
+FU_HD int sample(uint64_t seed, uint64_t k, uint32_t n) {
+    uint64_t z = seed + (k + 1) * 0x9E3779B97F4A7C15ull;
+    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+    z ^= z >> 31;
+    return (int)((uint32_t)((z >> 32) % n));
+}
+
+// src = R * ref + t
+struct Model {
+    M3d R;
+    V3d t;
+};
+FU_HD bool inlier(const Model& m, V3d s, V3d r) {
+    const float thresh_inlier = 0.05f;
+    return vnorm(s - (rot(m.R, r) + m.t)) <= thresh_inlier;
+}
+
+// The model of draw d, three samples of the n pairs p.s(i) / p.r(i): false where the draw gives
+// none, with its verdict: kNoModel, or kReflected, after which the iteration is not counted.
+enum { kNoModel = -1, kReflected = -2 };
+template <class P>
+FU_HD bool draw_model(const P& p, int n, uint64_t seed, long long d, Model& m, int& verdict) {
+    verdict = kNoModel;
+    const int i = sample(seed, 3 * (uint64_t)d, (uint32_t)n), j = sample(seed, 3 * (uint64_t)d + 1, (uint32_t)n),
+              k = sample(seed, 3 * (uint64_t)d + 2, (uint32_t)n);
+    const bool bad = i == j || j == k || k == i;
+    const V3d sa = p.s(i), sb = p.s(j), sc = p.s(k);
+    const V3d ra = p.r(i), rb = p.r(j), rc = p.r(k);
+    const float sd = (float)vnorm(vcross(sb - sa, sa - sc));  // stored in floats (Solver.cc:52-53)
+    const float rd = (float)vnorm(vcross(rb - ra, ra - rc));
+    if (bad || (double)sd < 1e-6 || (double)rd < 1e-6) return false;
+    const V3d sm = (sa + sb + sc) / 3, rm = (ra + rb + rc) / 3;
+    M3d Ab{{0, 0, 0, 0, 0, 0, 0, 0, 0}};
+    outer_add(Ab, sa - sm, ra - rm);
+    outer_add(Ab, sb - sm, rb - rm);
+    outer_add(Ab, sc - sm, rc - rm);
+    m.R = kabsch(Ab);
+    if (det(m.R) < 0) {  // as Solver.cc:82: a new sample
+        verdict = kReflected;
+        return false;
+    }
+    m.t = sm - rot(m.R, rm);
+    return true;
+}
+
+// The pairs on the device: those of the ratio test (a frame point by its index, the map's point) ...
+struct RatioPair {
+    int query;
+    float pos[3];
+};
+struct RatioPoints {
+    const int* count;
+    const RatioPair* pair;
+    const double* frame;
+    __device__ int begin() { return *count; }
+    __device__ V3d s(int i) const {
+        const double* f = frame + 3 * (size_t)pair[i].query;
+        return V3d{f[0], f[1], f[2]};
+    }
+    __device__ V3d r(int i) const {
+        const RatioPair& k = pair[i];
+        return V3d{(double)k.pos[0], (double)k.pos[1], (double)k.pos[2]};
     }
 };
+// ... or the refined pairs of the first list that selected three or more
+struct ListPoints {
+    const int* n_selected;
+    const int* n_refined;
+    const int* list;
+    int lists, max_sel;
+    const SurfHead* frame;
+    const SurfHead* map;
+    __device__ int begin() {
+        for (int i = 0; i < lists; ++i)
+            if (n_selected[i] >= 3) {
+                list += (size_t)i * max_sel;
+                return n_refined[i];
+            }
+        return 0;
+    }
+    __device__ V3d s(int i) const {
+        const float* f = frame[list[i]].pos;
+        return V3d{(double)f[0], (double)f[1], (double)f[2]};
+    }
+    __device__ V3d r(int i) const {
+        const float* f = map[list[i]].pos;
+        return V3d{(double)f[0], (double)f[1], (double)f[2]};
+    }
+};
+
+// The inliers of draws first .. first + gridDim.x - 1 of call blockIdx.y (which draws from seed +
+// blockIdx.y), a wave each: its lanes run the serial model side by side, then take the pairs 64 at
+// a time.  Bound by the model's chain of divisions and roots.  100 draws of five calls over 380
+// pairs took a host thread per call 500 us, here 14 us.
+template <class P>
+__global__ __launch_bounds__(64) void k_hypotheses(P p, uint64_t seed, long long first, int stride, int* verdict) {
+    const int n = p.begin();
+    if (n < 3) return;  // uniform
+    Model m;
+    int v;
+    if (draw_model(p, n, seed + blockIdx.y, first + blockIdx.x, m, v)) {
+        v = 0;
+        for (int i = threadIdx.x; i - (int)threadIdx.x < n; i += 64) {
+            const bool in = i < n && inlier(m, p.s(min(i, n - 1)), p.r(min(i, n - 1)));
+            v += __popcll(__ballot(in));
+        }
+    }
+    if (threadIdx.x == 0) verdict[blockIdx.y * stride + blockIdx.x] = v;
+}
+
+// the pairs on the host
+struct HostPoints {
+    const double* src;
+    const double* ref;
+    FU_HD V3d s(int i) const { return V3d{src[3 * i], src[3 * i + 1], src[3 * i + 2]}; }
+    FU_HD V3d r(int i) const { return V3d{ref[3 * i], ref[3 * i + 1], ref[3 * i + 2]}; }
+};
+
+// Solver::PoseEstimate (Optimization/Solver.cc:6-183), checkAngle = false, over the verdicts of its
+// draws: verdict(d, v) gives draw d's kNoModel, kReflected or count of inliers.  Only the last
+// accepted hypothesis' refined model and the last evaluated one's outliers reach the result, so
+// only those two are worked out here.
+template <class V>
+fu_status pose_estimate(const HostPoints& p, int n, int iterations, uint64_t seed, V&& verdict, double T[16],
+                        uint8_t* inliers, int32_t* ok) {
+    *ok = 0;
+    for (int k = 0; k < 16; ++k) T[k] = (k % 5 == 0) ? 1.0 : 0.0;
+    if (n < 3) return FU_OK;
+    const float thresh_confidence = 0.95f;
+    const int min_iter = 20;
+    int inliers_best = 0, it = 0;
+    long long best = -1, evaluated = -1;
+    // a reflection re-draws without counting the iteration (as the reference); a three-point
+    // sample spans at most a plane and its completed bases are right-handed, so that does not
+    // repeat, but the draws are bounded all the same
+    long long draws = 0;
+    const long long max_draws = 64ll * (iterations > 0 ? iterations : 1);
+    while (it < iterations && draws < max_draws) {
+        const long long d = draws++;
+        int nin = 0;
+        const fu_status st = verdict(d, nin);
+        if (st) return st;
+        if (nin == kReflected) continue;
+        if (nin >= 0) evaluated = d;
+        if (nin > inliers_best) {
+            best = d;
+            inliers_best = nin;
+            const float ratio = (float)nin / (float)n;
+            // pow of a float and an int is the double pow (Solver.cc:124)
+            const float confidence = (float)(1 - pow(1 - pow((double)ratio, 3), (double)(it + 1)));
+            if (it >= min_iter && confidence >= thresh_confidence) break;
+        }
+        ++it;
+    }
+    if (evaluated < 0) return FU_OK;  // no hypothesis was evaluated
+    std::vector<char> outlier(n);
+    auto mark = [&](long long d) {  // the outliers of draw d's model (Solver.cc:84-93)
+        Model m;
+        int v;
+        (void)draw_model(p, n, seed, d, m, v);
+        for (int i = 0; i < n; ++i) outlier[i] = !inlier(m, p.s(i), p.r(i));
+    };
+    // the model of the pairs that are not outliers: false if there are none
+    auto refit = [&](Model& m) {
+        V3d smn{0, 0, 0}, rmn{0, 0, 0};
+        int N = 0;
+        for (int i = 0; i < n; ++i)
+            if (!outlier[i]) {
+                smn = smn + p.s(i);
+                rmn = rmn + p.r(i);
+                ++N;
+            }
+        if (N == 0) return false;
+        smn = smn / N;
+        rmn = rmn / N;
+        M3d Ab{{0, 0, 0, 0, 0, 0, 0, 0, 0}};
+        for (int i = 0; i < n; ++i)
+            if (!outlier[i]) outer_add(Ab, p.s(i) - smn, p.r(i) - rmn);
+        m.R = kabsch(Ab);
+        m.t = smn - rot(m.R, rmn);
+        return true;
+    };
+    Model m{M3d{{1, 0, 0, 0, 1, 0, 0, 0, 1}}, V3d{0, 0, 0}};
+    if (best >= 0) {
+        mark(best);
+        refit(m);
+    }
+    // the final set: the best model's inliers added to the last evaluated hypothesis' (the
+    // reference does not reset the flags first, Solver.cc:138-143)
+    mark(evaluated);
+    for (int i = 0; i < n; ++i)
+        if (inlier(m, p.s(i), p.r(i))) outlier[i] = 0;
+    if (!refit(m) || det(m.R) < 0) return FU_OK;
+    for (int i = 0; i < 3; ++i) {
+        for (int j = 0; j < 3; ++j) T[i * 4 + j] = m.R.a[i * 3 + j];
+    }
+    T[3] = m.t.x;
+    T[7] = m.t.y;
+    T[11] = m.t.z;
+    if (inliers)
+        for (int i = 0; i < n; ++i) inliers[i] = !outlier[i];
+    *ok = 1;
+    return FU_OK;
+}
 
 }  // namespace
 
@@ -682,193 +942,199 @@ extern "C" fu_status fu_match_knn2(const float* query, int32_t nq, const float* 
     return FU_OK;
 }
 
-// Solver::PoseEstimate (Optimization/Solver.cc:6-183), checkAngle = false
+// the counts made here, on the host
 extern "C" fu_status fu_pose_estimate(const double* src, const double* ref, int32_t n, int32_t iterations,
-                                      uint64_t seed, double T[16], uint8_t* inlier, int32_t* ok) {
+                                      uint64_t seed, double T[16], uint8_t* inliers, int32_t* ok) {
     if (!src || !ref || !T || !ok || n < 0 || iterations < 0) return api_error(FU_ERR_ARG, "fu_pose_estimate: bad argument");
-    *ok = 0;
-    for (int k = 0; k < 16; ++k) T[k] = (k % 5 == 0) ? 1.0 : 0.0;
-    if (n < 3) return FU_OK;
-    auto S = [&](int i) { return V3d{src[3 * i], src[3 * i + 1], src[3 * i + 2]}; };
-    auto Rf = [&](int i) { return V3d{ref[3 * i], ref[3 * i + 1], ref[3 * i + 2]}; };
-    M3d R_best{{1, 0, 0, 0, 1, 0, 0, 0, 1}};
-    V3d t_best{0, 0, 0};
-    int inliers_best = 0;
-    const float thresh_inlier = 0.05f;
-    const float thresh_confidence = 0.95f;
-    const int min_iter = 20;
-    float ratio = 0.f, confidence = 0.f;
-    std::vector<char> outlier;  // the last evaluated hypothesis' outliers (Solver.cc:84-93)
-    Rng rng{seed};
-    int it = 0;
-    // a reflection re-draws without counting the iteration (as the reference); a three-point
-    // sample spans at most a plane and its completed bases are right-handed, so that does not
-    // repeat, but the draws are bounded all the same
-    long long draws = 0;
-    const long long max_draws = 64ll * (iterations > 0 ? iterations : 1);
-    while (it < iterations && draws++ < max_draws) {
-        int smp[3];
-        for (int k = 0; k < 3; ++k) smp[k] = (int)rng.next((uint32_t)n);
-        const bool bad = smp[0] == smp[1] || smp[1] == smp[2] || smp[2] == smp[0];
-        V3d sa = S(smp[0]), sb = S(smp[1]), sc = S(smp[2]);
-        V3d ra = Rf(smp[0]), rb = Rf(smp[1]), rc = Rf(smp[2]);
-        const float sd = (float)vnorm(vcross(sb - sa, sa - sc));  // stored in floats (Solver.cc:52-53)
-        const float rd = (float)vnorm(vcross(rb - ra, ra - rc));
-        if (bad || (double)sd < 1e-6 || (double)rd < 1e-6) {
-            ++it;
-            continue;
-        }
-        const V3d sm = (sa + sb + sc) / 3, rm = (ra + rb + rc) / 3;
-        M3d Ab{{0, 0, 0, 0, 0, 0, 0, 0, 0}};
-        outer_add(Ab, sa - sm, ra - rm);
-        outer_add(Ab, sb - sm, rb - rm);
-        outer_add(Ab, sc - sm, rc - rm);
-        M3d R = kabsch(Ab);
-        if (det(R) < 0) continue;  // as Solver.cc:82: a new sample, the iteration not counted
-        const V3d t = sm - rot(R, rm);
-        int nin = 0;
-        outlier.assign(n, 1);
-        for (int i = 0; i < n; ++i)
-            if (vnorm(S(i) - (rot(R, Rf(i)) + t)) <= thresh_inlier) {
-                ++nin;
-                outlier[i] = 0;
-            }
-        if (nin > inliers_best) {
-            V3d smn{0, 0, 0}, rmn{0, 0, 0};
-            for (int i = 0; i < n; ++i)
-                if (!outlier[i]) {
-                    smn = smn + S(i);
-                    rmn = rmn + Rf(i);
-                }
-            smn = smn / nin;
-            rmn = rmn / nin;
-            M3d Ab2{{0, 0, 0, 0, 0, 0, 0, 0, 0}};
-            for (int i = 0; i < n; ++i)
-                if (!outlier[i]) outer_add(Ab2, S(i) - smn, Rf(i) - rmn);
-            R_best = kabsch(Ab2);
-            t_best = smn - rot(R_best, rmn);
-            inliers_best = nin;
-            ratio = (float)nin / (float)n;
-            // pow of a float and an int is the double pow (Solver.cc:124)
-            confidence = (float)(1 - pow(1 - pow((double)ratio, 3), (double)(it + 1)));
-            if (it >= min_iter && confidence >= thresh_confidence) break;
-        }
-        ++it;
-    }
-    if (outlier.empty()) return FU_OK;  // no hypothesis was evaluated
-    // the final set: the best model's inliers added to the last evaluated hypothesis' (the
-    // reference does not reset the flags first, Solver.cc:138-143)
-    for (int i = 0; i < n; ++i)
-        if (vnorm(S(i) - (rot(R_best, Rf(i)) + t_best)) <= thresh_inlier) outlier[i] = 0;
-    int N = 0;
-    V3d smn{0, 0, 0}, rmn{0, 0, 0};
-    for (int i = 0; i < n; ++i)
-        if (!outlier[i]) {
-            smn = smn + S(i);
-            rmn = rmn + Rf(i);
-            ++N;
-        }
-    if (N == 0) return FU_OK;
-    smn = smn / N;
-    rmn = rmn / N;
-    M3d Ab{{0, 0, 0, 0, 0, 0, 0, 0, 0}};
-    for (int i = 0; i < n; ++i)
-        if (!outlier[i]) outer_add(Ab, S(i) - smn, Rf(i) - rmn);
-    R_best = kabsch(Ab);
-    if (det(R_best) < 0) return FU_OK;
-    t_best = smn - rot(R_best, rmn);
-    for (int i = 0; i < 3; ++i) {
-        for (int j = 0; j < 3; ++j) T[i * 4 + j] = R_best.a[i * 3 + j];
-    }
-    T[3] = t_best.x;
-    T[7] = t_best.y;
-    T[11] = t_best.z;
-    if (inlier)
-        for (int i = 0; i < n; ++i) inlier[i] = !outlier[i];
-    (void)inliers_best;
-    *ok = 1;
-    return FU_OK;
+    const HostPoints p{src, ref};
+    auto count = [&](long long d, int& v) {
+        Model m;
+        if (!draw_model(p, n, seed, d, m, v)) return FU_OK;
+        v = 0;
+        for (int i = 0; i < n; ++i) v += inlier(m, p.s(i), p.r(i));
+        return FU_OK;
+    };
+    return pose_estimate(p, n, iterations, seed, count, T, inliers, ok);
 }
 
 namespace {
-// record j of `out` = keys[idx[j]], or zeros where idx[j] < 0 (a query without a neighbour);
-// one lane per 16 bytes
-__global__ void k_gather_keys(const fu_surf* keys, const int32_t* idx, int n, fu_surf* out) {
-    constexpr int Q = (int)(sizeof(fu_surf) / 16);
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n * Q) return;
-    const int j = t / Q, q = t % Q;
-    const int k = idx[j];
-    uint4 v = make_uint4(0u, 0u, 0u, 0u);
-    if (k >= 0) v = reinterpret_cast<const uint4*>(&keys[k])[q];
-    reinterpret_cast<uint4*>(&out[j])[q] = v;
+// parts of one stream-ordered allocation, 256-byte aligned
+struct Block {
+    hipStream_t stream;
+    char* base = nullptr;
+    size_t size = 0;
+    explicit Block(hipStream_t s) : stream(s) {}
+    Block(const Block&) = delete;
+    Block& operator=(const Block&) = delete;
+    ~Block() {
+        if (base) (void)hipFreeAsync(base, stream);
+    }
+    size_t part(size_t bytes) {
+        const size_t at = size;
+        size += (bytes + 255) & ~(size_t)255;
+        return at;
+    }
+    bool allocate() {
+        if (hipMallocAsync((void**)&base, size, stream) == hipSuccess) return true;
+        (void)hipGetLastError();
+        base = nullptr;
+        return false;
+    }
+    template <class T>
+    T* at(size_t part) const {
+        return reinterpret_cast<T*>(base + part);
+    }
+};
+
+// The exclusive prefix over a 1024-lane work-group (lanes in order) of c, 0 to 2 per lane as the
+// sum of two flags, and the total.
+__device__ __forceinline__ int pair_prefix(bool f, bool g, int* wsum, int& total) {
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const unsigned long long bf = __ballot(f), bg = __ballot(g), below = (1ull << lane) - 1ull;
+    __syncthreads();
+    if (lane == 0) wsum[wid] = __popcll(bf) + __popcll(bg);
+    __syncthreads();
+    int before = 0, all = 0;
+    for (int w = 0; w < 16; ++w) {
+        const int c = wsum[w];
+        before += w < wid ? c : 0;
+        all += c;
+    }
+    total = all;
+    return before + __popcll(bf & below) + __popcll(bg & below);
 }
-static_assert(sizeof(fu_surf) % 16 == 0, "records move as 16-byte words");
+
+struct PairArgs {
+    const int* idx;          // the two nearest map keys of each query
+    const float* dist;
+    int nq;
+    const int* slot;         // of each map key, -1 for key 0
+    const SurfHead* heads;   // the map's slots, kSlotHeads apart
+};
+// The pairs that pass the ratio test (Tracking.cc:437-444; with one map key the second distance is
+// infinite) in query order.  One work-group: the prefix is over hundreds of queries.
+__global__ __launch_bounds__(1024) void k_ratio_pairs(PairArgs a, RatioPair* out, int* count) {
+    __shared__ int wsum[16];
+    int n = 0;
+    for (int base = 0; base < a.nq; base += 1024) {
+        const int i = base + threadIdx.x;
+        const int key = i < a.nq ? a.idx[2 * i] : -1;
+        const bool f = key >= 0 && (double)a.dist[2 * i] < 0.90 * (double)a.dist[2 * i + 1];
+        int total;
+        const int at = n + pair_prefix(f, false, wsum, total);
+        if (f) {
+            const int s = a.slot[key];
+            RatioPair p{i, {0.f, 0.f, 0.f}};
+            if (s >= 0)
+                for (int c = 0; c < 3; ++c) p.pos[c] = a.heads[(size_t)s * kSlotHeads].pos[c];
+            out[at] = p;
+        }
+        n += total;
+    }
+    if (threadIdx.x == 0) *count = n;
+}
+// The match list of graph matching (Tracking.cc:437-444): both nearest keys of a query that fails the
+// ratio test.  counts[0]: its length; counts[1]: the pairs whose key is valid (:485-505), which are
+// written as the frame's and the map's records (without descriptors) and their distance.
+__global__ __launch_bounds__(1024) void k_graph_pairs(PairArgs a, const float* fpos, const float* fnrm, SurfHead* fk,
+                                                      SurfHead* mk, float* dd, int* counts) {
+    __shared__ int wsum[16];
+    int listed = 0, n = 0;
+    for (int base = 0; base < a.nq; base += 1024) {
+        const int i = base + threadIdx.x;
+        int key[2] = {-1, -1}, slot[2] = {-1, -1};
+        float d[2] = {0.f, 0.f};
+        if (i < a.nq) {
+            key[0] = a.idx[2 * i];
+            d[0] = a.dist[2 * i];
+            d[1] = a.dist[2 * i + 1];
+            if (key[0] >= 0 && !((double)d[0] < 0.90 * (double)d[1])) key[1] = a.idx[2 * i + 1];
+        }
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+            if (key[k] >= 0) slot[k] = a.slot[key[k]];
+        int total;
+        (void)pair_prefix(key[0] >= 0, key[1] >= 0, wsum, total);
+        listed += total;
+        int at = n + pair_prefix(slot[0] >= 0, slot[1] >= 0, wsum, total);
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+            if (slot[k] >= 0) {
+                SurfHead f;
+                f.valid = 1;  // the reference leaves this record's flag unset
+                f.pad[0] = f.pad[1] = f.pad[2] = 0;
+                for (int c = 0; c < 3; ++c) f.pos[c] = fpos[3 * i + c];
+                for (int c = 0; c < 4; ++c) f.normal[c] = fnrm[4 * i + c];
+                fk[at] = f;
+                mk[at] = a.heads[(size_t)slot[k] * kSlotHeads];
+                dd[at] = d[k];
+                ++at;
+            }
+        n += total;
+    }
+    if (threadIdx.x == 0) {
+        counts[0] = listed;
+        counts[1] = n;
+    }
+}
+// what the host needs of the selection: the lists' counts, then the points of the list whose pose is
+// estimated (frame and map, 6 floats a pair)
+__global__ __launch_bounds__(1024) void k_list_points(ListPoints p, int* counts, float* points) {
+    if ((int)threadIdx.x < p.lists) {
+        counts[threadIdx.x] = p.n_selected[threadIdx.x];
+        counts[p.lists + threadIdx.x] = p.n_refined[threadIdx.x];
+    }
+    const int n = p.begin();
+    for (int i = threadIdx.x; i < n; i += 1024)
+        for (int c = 0; c < 3; ++c) {
+            points[6 * i + c] = p.frame[p.list[i]].pos[c];
+            points[6 * i + 3 + c] = p.map[p.list[i]].pos[c];
+        }
+}
 
 // the map's keys (UpdateMapKeys, Mapping.cc:142-151; the first record is never written by
-// CollectKeyPoints and reads as zeros here) and the two nearest of them to each frame
-// descriptor: `nk` map keys; on the host, the neighbours' indices and distances (2 per query,
-// -1 / +inf where the map has fewer keys) and their records in the same slots (zeros for -1).
-// Device buffers are stream-ordered allocations; only the matched records come back.
-fu_status collect_and_match(fu_keymap* km, const float* frame_desc, int32_t nq, uint32_t& nk,
-                            std::vector<fu_surf>& matched, std::vector<int32_t>& hidx, std::vector<float>& hdist,
-                            fu_stream s, const char* who) {
-    hipStream_t hs = (hipStream_t)s;
-    nk = 0;
-    fu_status st = fu_collect_key_points(km, nullptr, 0, &nk, s);
+// CollectKeyPoints and reads as zeros here) and the two nearest of them to each frame descriptor,
+// on the device.  `out`: idx and dist, 2 per query (-1 / +inf where the map has fewer keys), and the
+// keys' slots, which live in `keys`.
+fu_status collect_and_match(fu_keymap* km, const float* frame_desc, int32_t nq, uint32_t nk, Block& keys, int32_t* idx,
+                            float* dist, PairArgs& out, hipStream_t hs, const char* who) {
+    const size_t desc = keys.part(sizeof(float) * kDesc * nk), slot = keys.part(sizeof(int32_t) * nk);
+    if (!keys.allocate()) return api_error(FU_ERR_NOMEM, "%s: %u keys", who, nk);
+    fu_status st = keymap_pack(km, keys.at<float>(desc), keys.at<int32_t>(slot), hs);
     if (st) return st;
-    matched.clear();
-    if (nk == 0 || nq == 0) return FU_OK;  // no map keys (Tracking.cc:417-418)
-    fu_surf *keys = nullptr, *mrec = nullptr;
-    float* train = nullptr;
-    int32_t* idx = nullptr;
-    float* dist = nullptr;
-    auto release = [&]() {
-        if (keys) (void)hipFreeAsync(keys, hs);
-        if (mrec) (void)hipFreeAsync(mrec, hs);
-        if (train) (void)hipFreeAsync(train, hs);
-        if (idx) (void)hipFreeAsync(idx, hs);
-        if (dist) (void)hipFreeAsync(dist, hs);
-    };
-    const int nm = 2 * nq;
-    if (hipMallocAsync((void**)&keys, sizeof(fu_surf) * nk, hs) != hipSuccess ||
-        hipMallocAsync((void**)&mrec, sizeof(fu_surf) * nm, hs) != hipSuccess ||
-        hipMallocAsync((void**)&train, sizeof(float) * 64 * nk, hs) != hipSuccess ||
-        hipMallocAsync((void**)&idx, sizeof(int32_t) * nm, hs) != hipSuccess ||
-        hipMallocAsync((void**)&dist, sizeof(float) * nm, hs) != hipSuccess) {
-        (void)hipGetLastError();
-        release();
-        return api_error(FU_ERR_NOMEM, "%s: %u keys", who, nk);
-    }
-    matched.resize(nm);
-    hidx.resize(nm);
-    hdist.resize(nm);
-    hipError_t e = hipMemsetAsync(keys, 0, sizeof(fu_surf) * nk, hs);
-    if (e == hipSuccess) {
-        uint32_t again = 0;
-        st = fu_collect_key_points(km, keys, nk, &again, s);
-    }
-    // descriptors packed for the matcher: 256 bytes of each 288-byte record
-    if (!st && e == hipSuccess)
-        e = hipMemcpy2DAsync(train, 64 * sizeof(float), (const char*)keys + offsetof(fu_surf, descriptor), sizeof(fu_surf),
-                             64 * sizeof(float), nk, hipMemcpyDeviceToDevice, hs);
-    if (!st && e == hipSuccess) st = fu_match_knn2(frame_desc, nq, train, (int32_t)nk, idx, dist, s);
-    if (!st && e == hipSuccess) {
-        const int lanes = nm * (int)(sizeof(fu_surf) / 16);
-        hipLaunchKernelGGL(k_gather_keys, dim3((lanes + 255) / 256), dim3(256), 0, hs, keys, idx, nm, mrec);
-        e = hipGetLastError();
-    }
-    if (!st && e == hipSuccess) e = hipMemcpyAsync(matched.data(), mrec, sizeof(fu_surf) * nm, hipMemcpyDeviceToHost, hs);
-    if (!st && e == hipSuccess) e = hipMemcpyAsync(hidx.data(), idx, sizeof(int32_t) * nm, hipMemcpyDeviceToHost, hs);
-    if (!st && e == hipSuccess) e = hipMemcpyAsync(hdist.data(), dist, sizeof(float) * nm, hipMemcpyDeviceToHost, hs);
-    release();
-    // also after a failure: nothing queued may still write into the host vectors
-    const hipError_t es = hipStreamSynchronize(hs);
-    if (e == hipSuccess) e = es;
-    if (st) return st;
-    if (e != hipSuccess) return api_error(FU_ERR_HIP, "%s: %s", who, hipGetErrorString(e));
+    if ((st = fu_match_knn2(frame_desc, nq, keys.at<float>(desc), (int32_t)nk, idx, dist, (fu_stream)hs))) return st;
+    out = PairArgs{idx, dist, nq, keys.at<int32_t>(slot), keymap_heads(km)};
     return FU_OK;
 }
+
+// The draws of the first launch of counts; a call that needs more has the next kMoreDraws counted.
+constexpr int kFirstDraws = 256, kMoreDraws = 4096;
+template <class P>
+struct Counts {
+    P points;
+    uint64_t seed;
+    int dev;
+    hipStream_t stream;
+    std::vector<int> have;  // of draws base .. base + have.size() - 1 (the walk asks for them in order)
+    long long base = 0;
+    fu_status operator()(long long d, int& v) {
+        if (d >= base + (long long)have.size()) {
+            Block block(stream);
+            const size_t part = block.part(sizeof(int) * kMoreDraws);
+            if (!block.allocate()) return api_error(FU_ERR_NOMEM, "PoseEstimate: %d draws", kMoreDraws);
+            hipLaunchKernelGGL(k_hypotheses<P>, dim3(kMoreDraws), dim3(64), 0, stream, points, seed, d, 0,
+                               block.at<int>(part));
+            base = d;
+            have.resize(kMoreDraws);
+            hipError_t e = hipGetLastError();
+            const hipError_t er = mail_read(dev, have.data(), block.at<int>(part), sizeof(int) * kMoreDraws, stream);
+            if (e == hipSuccess) e = er;
+            if (e != hipSuccess) return api_error(FU_ERR_HIP, "PoseEstimate: %s", hipGetErrorString(e));
+        }
+        v = have[(size_t)(d - base)];
+        return FU_OK;
+    }
+};
 
 // the camera pose of a PoseEstimate transform T (frame point = R * map point + t): T^-1
 void rigid_inverse(const double T[16], double pose[16]) {
@@ -894,29 +1160,58 @@ extern "C" fu_status fu_relocalise_keys(fu_keymap* km, const float* frame_desc, 
     *ok = 0;
     if (n_pairs) *n_pairs = 0;
     for (int k = 0; k < 16; ++k) pose[k] = (k % 5 == 0) ? 1.0 : 0.0;
-    std::vector<fu_surf> matched;
-    std::vector<int32_t> hidx;
-    std::vector<float> hdist;
+    hipStream_t hs = (hipStream_t)s;
     uint32_t nk = 0;
-    fu_status st = collect_and_match(km, frame_desc, nq, nk, matched, hidx, hdist, s, "fu_relocalise_keys");
+    fu_status st = keymap_count(km, &nk, hs);
     if (st) return st;
-    if (matched.empty()) return FU_OK;
-    // the ratio test (Tracking.cc:437-444); with one map key the second distance is infinite
-    std::vector<double> src, ref;
-    for (int i = 0; i < nq; ++i) {
-        if (hidx[2 * i] < 0) continue;
-        if ((double)hdist[2 * i] < 0.90 * (double)hdist[2 * i + 1]) {
-            const fu_surf& k = matched[2 * i];
-            src.insert(src.end(), {frame_pos[3 * i], frame_pos[3 * i + 1], frame_pos[3 * i + 2]});
-            ref.insert(ref.end(), {(double)k.pos[0], (double)k.pos[1], (double)k.pos[2]});
-        }
+    if (nk == 0 || nq == 0) return FU_OK;  // no map keys (Tracking.cc:417-418)
+    const int draws = std::max(0, std::min(iterations, kFirstDraws));
+    Block keys(hs), work(hs);
+    const size_t fpos = work.part(sizeof(double) * 3 * nq), idx = work.part(sizeof(int32_t) * 2 * nq),
+                 dist = work.part(sizeof(float) * 2 * nq), head = work.part(sizeof(int) * (1 + kFirstDraws)),
+                 pairs = work.part(sizeof(RatioPair) * nq);
+    if (!work.allocate()) return api_error(FU_ERR_NOMEM, "fu_relocalise_keys: %d keypoints", nq);
+    PairArgs pa{};
+    if ((st = collect_and_match(km, frame_desc, nq, nk, keys, work.at<int32_t>(idx), work.at<float>(dist), pa, hs,
+                                "fu_relocalise_keys")))
+        return st;
+    hipError_t e = hipMemcpyAsync(work.at<double>(fpos), frame_pos, sizeof(double) * 3 * nq, hipMemcpyHostToDevice, hs);
+    int* dhead = work.at<int>(head);
+    RatioPair* dpairs = work.at<RatioPair>(pairs);
+    const RatioPoints points{dhead, dpairs, work.at<double>(fpos)};
+    hipLaunchKernelGGL(k_ratio_pairs, dim3(1), dim3(1024), 0, hs, pa, dpairs, dhead);
+    if (draws > 0)
+        hipLaunchKernelGGL(k_hypotheses<RatioPoints>, dim3(draws), dim3(64), 0, hs, points, seed, 0ll, 0, dhead + 1);
+    if (e == hipSuccess) e = hipGetLastError();
+    // the pairs with the counts, as many as go with them
+    std::vector<int> hhead(1 + draws);
+    std::vector<RatioPair> hp(nq);
+    const size_t hbytes = sizeof(int) * hhead.size();
+    const int first = (int)std::min<size_t>(nq, (kMailBytes - hbytes) / sizeof(RatioPair));
+    const int dev = keymap_device(km);
+    // also after a failure: nothing queued may still read the caller's memory
+    const hipError_t er = mail_read(dev, hhead.data(), dhead, hbytes, hp.data(), dpairs, sizeof(RatioPair) * first, hs);
+    if (e == hipSuccess) e = er;
+    const int np = e == hipSuccess ? hhead[0] : 0;
+    if (np > first) {
+        e = hipMemcpyAsync(hp.data() + first, dpairs + first, sizeof(RatioPair) * (np - first), hipMemcpyDeviceToHost, hs);
+        const hipError_t es = hipStreamSynchronize(hs);
+        if (e == hipSuccess) e = es;
     }
-    const int np = (int)(src.size() / 3);
+    if (e != hipSuccess) return api_error(FU_ERR_HIP, "fu_relocalise_keys: %s", hipGetErrorString(e));
     if (n_pairs) *n_pairs = np;
     if (np < 3) return FU_OK;
+    if (iterations < 0) return api_error(FU_ERR_ARG, "fu_pose_estimate: bad argument");
+    std::vector<double> src(3 * (size_t)np), ref(3 * (size_t)np);
+    for (int k = 0; k < np; ++k)
+        for (int c = 0; c < 3; ++c) {
+            src[3 * k + c] = frame_pos[3 * (size_t)hp[k].query + c];
+            ref[3 * k + c] = (double)hp[k].pos[c];
+        }
+    Counts<RatioPoints> counts{points, seed, dev, hs, std::vector<int>(hhead.begin() + 1, hhead.end())};
     double T[16];
     int32_t good = 0;
-    if ((st = fu_pose_estimate(src.data(), ref.data(), np, iterations, seed, T, nullptr, &good))) return st;
+    if ((st = pose_estimate(HostPoints{src.data(), ref.data()}, np, iterations, seed, counts, T, nullptr, &good))) return st;
     if (!good) return FU_OK;
     rigid_inverse(T, pose);
     *ok = 1;
@@ -934,11 +1229,12 @@ extern "C" fu_status fu_select_subgraphs(const float* matrix, int32_t n, int32_t
         return api_error(FU_ERR_ARG, "fu_select_subgraphs: null argument");
     hipStream_t hs = (hipStream_t)s;
     if (n > 0) {
-        hipLaunchKernelGGL(k_rank_sums, dim3((n + 63) / 64), dim3(256), 0, hs, matrix, n, rank_sum);
-        hipLaunchKernelGGL(k_rank_order, dim3((n + 63) / 64), dim3(256), 0, hs, rank_sum, n, order);
+        hipLaunchKernelGGL(k_rank_sums, dim3((n + kSumCols - 1) / kSumCols), dim3(256), 0, hs, matrix, n, rank_sum);
+        hipLaunchKernelGGL(k_rank_order, dim3((n + 63) / 64), dim3(1024), 0, hs, rank_sum, n, order);
     }
     const SelArgs a{matrix, order, n, max_select, min_score, n_selected, n_refined, refined};
-    hipLaunchKernelGGL(k_subgraphs, dim3(n_lists), dim3(kSelLanes), 0, hs, a);
+    hipLaunchKernelGGL(k_select, dim3(n_lists), dim3(kSelLanes), 0, hs, a);
+    if (n > 0 && max_select > 1) hipLaunchKernelGGL(k_refine, dim3((max_select + 2) / 4, n_lists), dim3(256), 0, hs, a);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return api_error(FU_ERR_HIP, "fu_select_subgraphs: %s", hipGetErrorString(e));
     return FU_OK;
@@ -964,83 +1260,70 @@ extern "C" fu_status fu_relocalise_graph_candidates(fu_keymap* km, const float* 
     constexpr float kMinScore = 0.1f;
     *n_poses = 0;
     if (n_pairs) *n_pairs = 0;
-    std::vector<fu_surf> matched;
-    std::vector<int32_t> hidx;
-    std::vector<float> hdist;
-    uint32_t nk = 0;
-    fu_status st =
-        collect_and_match(km, frame_desc, nq, nk, matched, hidx, hdist, s, "fu_relocalise_graph_candidates");
-    if (st) return st;
-    if (matched.empty()) return FU_OK;
-    // the match list (Tracking.cc:437-444), then the valid map keys (:485-505)
-    std::vector<std::pair<int, int>> refd;  // (query, neighbour slot 2 * query + 0 or 1)
-    std::vector<float> rdist;
-    for (int i = 0; i < nq; ++i) {
-        if (hidx[2 * i] < 0) continue;
-        refd.push_back({i, 2 * i});
-        rdist.push_back(hdist[2 * i]);
-        if (!((double)hdist[2 * i] < 0.90 * (double)hdist[2 * i + 1]) && hidx[2 * i + 1] >= 0) {
-            refd.push_back({i, 2 * i + 1});
-            rdist.push_back(hdist[2 * i + 1]);
-        }
-    }
-    if (n_pairs) *n_pairs = (int32_t)refd.size();
-    if (refd.size() < 3) return FU_OK;
-    std::vector<fu_surf> fk, mk;
-    std::vector<float> dd;
-    for (size_t r = 0; r < refd.size(); ++r) {
-        const fu_surf& key = matched[refd[r].second];
-        if (!key.valid) continue;
-        fu_surf f;
-        memset(&f, 0, sizeof(f));
-        f.valid = 1;  // the reference leaves this record's flag unset
-        memcpy(f.pos, frame_pos + 3 * refd[r].first, sizeof(f.pos));
-        memcpy(f.normal, frame_normal + 4 * refd[r].first, sizeof(f.normal));
-        fk.push_back(f);
-        mk.push_back(key);
-        dd.push_back(rdist[r]);
-    }
-    const int n = (int)fk.size();
-    if (n == 0) return FU_OK;  // rank.cols == 0 (:523-524)
-    if (n > 46340) return api_error(FU_ERR_ARG, "fu_relocalise_graph_candidates: %d pairs (at most 46340)", n);
+    const char* who = "fu_relocalise_graph_candidates";
     hipStream_t hs = (hipStream_t)s;
-    fu_surf *dfk = nullptr, *dmk = nullptr;
-    float *ddist = nullptr, *mat = nullptr, *rank = nullptr;
-    int32_t *order = nullptr, *nsel = nullptr;
-    auto release = [&]() {
-        for (void* p : {(void*)dfk, (void*)dmk, (void*)ddist, (void*)mat, (void*)rank, (void*)order, (void*)nsel})
-            if (p) (void)hipFreeAsync(p, hs);
-    };
-    const size_t nsel_words = 2 * kLists + (size_t)kLists * kSelect;
-    if (hipMallocAsync((void**)&dfk, sizeof(fu_surf) * n, hs) != hipSuccess ||
-        hipMallocAsync((void**)&dmk, sizeof(fu_surf) * n, hs) != hipSuccess ||
-        hipMallocAsync((void**)&ddist, sizeof(float) * n, hs) != hipSuccess ||
-        hipMallocAsync((void**)&mat, sizeof(float) * (size_t)n * n, hs) != hipSuccess ||
-        hipMallocAsync((void**)&rank, sizeof(float) * n, hs) != hipSuccess ||
-        hipMallocAsync((void**)&order, sizeof(int32_t) * n, hs) != hipSuccess ||
-        hipMallocAsync((void**)&nsel, sizeof(int32_t) * nsel_words, hs) != hipSuccess) {
-        (void)hipGetLastError();
-        release();
-        return api_error(FU_ERR_NOMEM, "fu_relocalise_graph_candidates: %d pairs", n);
-    }
-    std::vector<int32_t> hsel(nsel_words);
-    hipError_t e = hipMemcpyAsync(dfk, fk.data(), sizeof(fu_surf) * n, hipMemcpyHostToDevice, hs);
-    if (e == hipSuccess) e = hipMemcpyAsync(dmk, mk.data(), sizeof(fu_surf) * n, hipMemcpyHostToDevice, hs);
-    if (e == hipSuccess) e = hipMemcpyAsync(ddist, dd.data(), sizeof(float) * n, hipMemcpyHostToDevice, hs);
-    if (e == hipSuccess) st = fu_build_adjacency_matrix(dfk, dmk, ddist, n, mat, s);
-    if (e == hipSuccess && !st)
-        st = fu_select_subgraphs(mat, n, kLists, kSelect, kMinScore, rank, order, nsel, nsel + kLists,
-                                 nsel + 2 * kLists, s);
-    if (e == hipSuccess && !st)
-        e = hipMemcpyAsync(hsel.data(), nsel, sizeof(int32_t) * nsel_words, hipMemcpyDeviceToHost, hs);
-    release();
-    const hipError_t es = hipStreamSynchronize(hs);  // also after a failure (host buffers)
-    if (e == hipSuccess) e = es;
+    uint32_t nk = 0;
+    fu_status st = keymap_count(km, &nk, hs);
     if (st) return st;
-    if (e != hipSuccess) return api_error(FU_ERR_HIP, "fu_relocalise_graph_candidates: %s", hipGetErrorString(e));
-    const int32_t* n_selected = hsel.data();
-    const int32_t* n_refined = hsel.data() + kLists;
-    const int32_t* lists = hsel.data() + 2 * kLists;
+    if (nk == 0 || nq == 0) return FU_OK;  // no map keys (Tracking.cc:417-418)
+    const int dev = keymap_device(km);
+    Block keys(hs), work(hs), graph(hs);
+    const size_t nm = 2 * (size_t)nq;
+    const size_t fpos = work.part(sizeof(float) * 3 * nq), fnrm = work.part(sizeof(float) * 4 * nq),
+                 idx = work.part(sizeof(int32_t) * nm), dist = work.part(sizeof(float) * nm),
+                 fk = work.part(sizeof(SurfHead) * nm), mk = work.part(sizeof(SurfHead) * nm),
+                 dd = work.part(sizeof(float) * nm), cnt = work.part(sizeof(int) * 2);
+    if (!work.allocate()) return api_error(FU_ERR_NOMEM, "%s: %d keypoints", who, nq);
+    PairArgs pa{};
+    if ((st = collect_and_match(km, frame_desc, nq, nk, keys, work.at<int32_t>(idx), work.at<float>(dist), pa, hs, who)))
+        return st;
+    hipError_t e = hipMemcpyAsync(work.at<float>(fpos), frame_pos, sizeof(float) * 3 * nq, hipMemcpyHostToDevice, hs);
+    if (e == hipSuccess)
+        e = hipMemcpyAsync(work.at<float>(fnrm), frame_normal, sizeof(float) * 4 * nq, hipMemcpyHostToDevice, hs);
+    SurfHead *dfk = work.at<SurfHead>(fk), *dmk = work.at<SurfHead>(mk);
+    hipLaunchKernelGGL(k_graph_pairs, dim3(1), dim3(1024), 0, hs, pa, work.at<float>(fpos), work.at<float>(fnrm), dfk, dmk,
+                       work.at<float>(dd), work.at<int>(cnt));
+    if (e == hipSuccess) e = hipGetLastError();
+    int counted[2] = {0, 0};
+    // also after a failure: nothing queued may still read the caller's memory
+    const hipError_t er = mail_read(dev, counted, work.at<int>(cnt), sizeof(counted), hs);
+    if (e == hipSuccess) e = er;
+    if (e != hipSuccess) return api_error(FU_ERR_HIP, "%s: %s", who, hipGetErrorString(e));
+    if (n_pairs) *n_pairs = counted[0];
+    const int n = counted[1];
+    if (counted[0] < 3 || n == 0) return FU_OK;  // rank.cols == 0 (:523-524)
+    if (n > 46340) return api_error(FU_ERR_ARG, "%s: %d pairs (at most 46340)", who, n);
+    // counts of the lists, verdicts, points: read back together
+    const int draws = std::min(iterations, kFirstDraws);
+    constexpr size_t kCountInts = 2 * kLists;
+    const size_t head_ints = kCountInts + (size_t)kPoseLists * draws;
+    const size_t mat = graph.part(sizeof(float) * (size_t)n * n), rank = graph.part(sizeof(float) * n),
+                 order = graph.part(sizeof(int32_t) * n),
+                 sel = graph.part(sizeof(int32_t) * (kCountInts + (size_t)kLists * kSelect)),
+                 head = graph.part(sizeof(int) * head_ints), pts = graph.part(sizeof(float) * 6 * kSelect);
+    if (!graph.allocate()) return api_error(FU_ERR_NOMEM, "%s: %d pairs", who, n);
+    int32_t* nsel = graph.at<int32_t>(sel);
+    int* dhead = graph.at<int>(head);
+    float* dpts = graph.at<float>(pts);
+    if ((st = build_adjacency(dfk, dmk, 1, work.at<float>(dd), n, graph.at<float>(mat), hs))) return st;
+    if ((st = fu_select_subgraphs(graph.at<float>(mat), n, kLists, kSelect, kMinScore, graph.at<float>(rank),
+                                  graph.at<int32_t>(order), nsel, nsel + kLists, nsel + 2 * kLists, s)))
+        return st;
+    const ListPoints points{nsel, nsel + kLists, nsel + 2 * kLists, kLists, kSelect, dfk, dmk};
+    hipLaunchKernelGGL(k_list_points, dim3(1), dim3(1024), 0, hs, points, dhead, dpts);
+    if (draws > 0)
+        hipLaunchKernelGGL(k_hypotheses<ListPoints>, dim3(draws, kPoseLists), dim3(64), 0, hs, points, seed, 0ll, draws,
+                           dhead + kCountInts);
+    e = hipGetLastError();
+    std::vector<int> hhead(head_ints);
+    std::vector<float> hpts(6 * kSelect);
+    static_assert((kCountInts + kPoseLists * kFirstDraws + 6 * kSelect) * 4 <= kMailBytes, "one mail");
+    const hipError_t er2 = mail_read(dev, hhead.data(), dhead, sizeof(int) * head_ints, hpts.data(), dpts,
+                                     sizeof(float) * hpts.size(), hs);
+    if (e == hipSuccess) e = er2;
+    if (e != hipSuccess) return api_error(FU_ERR_HIP, "%s: %s", who, hipGetErrorString(e));
+    const int* n_selected = hhead.data();
+    const int* n_refined = hhead.data() + kLists;
     int kept = 0, first = -1;
     for (int i = 0; i < kLists; ++i)
         if (n_selected[i] >= 3) {
@@ -1052,34 +1335,20 @@ extern "C" fu_status fu_relocalise_graph_candidates(fu_keymap* km, const float* 
     const int R = n_refined[first];
     if (R <= 3) return FU_OK;  // every call skipped (:601-602)
     std::vector<double> src(3 * (size_t)R), ref(3 * (size_t)R);
-    for (int k = 0; k < R; ++k) {
-        const int p = lists[(size_t)first * kSelect + k];
+    for (int k = 0; k < R; ++k)
         for (int c = 0; c < 3; ++c) {
-            src[3 * k + c] = (double)fk[p].pos[c];
-            ref[3 * k + c] = (double)mk[p].pos[c];
+            src[3 * k + c] = (double)hpts[6 * k + c];
+            ref[3 * k + c] = (double)hpts[6 * k + 3 + c];
         }
-    }
-    // the M calls are independent (call c draws from seed + c alone), so calls 1 .. M-1 run on
-    // host threads of their own beside call 0; the poses are kept in call order
-    double T[kPoseLists][16];
-    int32_t good[kPoseLists] = {};
-    fu_status cst[kPoseLists] = {};
-    auto call = [&](int c) {
-        cst[c] = fu_pose_estimate(src.data(), ref.data(), R, iterations, seed + (uint64_t)c, T[c], nullptr, &good[c]);
-    };
-    std::vector<std::thread> workers;
-    for (int c = 1; c < M; ++c) {
-        try {
-            workers.emplace_back(call, c);
-        } catch (const std::system_error&) {
-            call(c);  // no thread to be had: the call runs here
-        }
-    }
-    call(0);
-    for (std::thread& w : workers) w.join();
     for (int c = 0; c < M; ++c) {
-        if (cst[c]) return api_error(cst[c], "fu_relocalise_graph_candidates: PoseEstimate call %d failed", c);
-        if (good[c]) rigid_inverse(T[c], poses + 16 * (*n_poses)++);
+        const int* v = hhead.data() + kCountInts + (size_t)c * draws;
+        Counts<ListPoints> counts{points, seed + (uint64_t)c, dev, hs, std::vector<int>(v, v + draws)};
+        double T[16];
+        int32_t good = 0;
+        if ((st = pose_estimate(HostPoints{src.data(), ref.data()}, R, iterations, seed + (uint64_t)c, counts, T, nullptr,
+                                &good)))
+            return st;
+        if (good) rigid_inverse(T, poses + 16 * (*n_poses)++);
     }
     return FU_OK;
 }
