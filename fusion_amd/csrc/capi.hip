@@ -275,6 +275,8 @@ static VisArgs make_vis(const fu_map* m, const PoseF& pose, const TrackState* st
     v.rows = rows;
     v.depth_min = dmin;
     v.depth_max = dmax;
+    v.zmin = v.zmax = nullptr;
+    v.ztiles = 0;
     (void)m;
     return v;
 }
@@ -356,7 +358,7 @@ extern "C" fu_status fu_create_rendering_blocks(fu_map* m, float* zrange_min, fl
     int ov = n_visible == 0xffffffffu ? -1 : (int)(n_visible < m->p.num_blocks ? n_visible : m->p.num_blocks);
     const ZRangeArgs a =
         make_zr(m, zrange_min, zrange_max, zcols, zrows, depth_max, depth_min, posef_from(pose), nullptr, ov, fx, fy, cx, cy);
-    launch_zrange(m->v, a, S(s));
+    launch_zrange(m->v, a, false, S(s));
     LAUNCHCHK();
     if (n_fragments || rendered) {
         fu_status st = FU_OK;
@@ -738,10 +740,11 @@ struct RgbLevels {
 };
 
 // queue the whole coarse-to-fine loop (device-resident)
-static void queue_se3(fu_tracker* t, const float* const nv[3], const float* const nn[3], const float* const lv[3],
-                      const float* const ln[3], const RgbLevels* rgb, const float K[4], const int32_t iters[3],
+// `begun`: the state has begun its frame (track_begin)
+static void queue_se3(fu_tracker* t, bool begun, const float* const nv[3], const float* const nn[3],
+                      const float* const lv[3], const float* const ln[3], const RgbLevels* rgb, const float K[4], const int32_t iters[3],
                       const int32_t minc[3], float thresh, hipStream_t s) {
-    launch_track_begin(t->st, s);
+    if (!begun) launch_track_begin(t->st, s);
     int last_level = -1;
     for (int l = 2; l >= 0; --l)
         if (iters[l] > 0) last_level = l;
@@ -771,7 +774,7 @@ extern "C" fu_status fu_compute_se3(fu_tracker* t, const float* const next_vmap[
     for (int l = 0; l < 3; ++l)
         if (!next_vmap[l] || !next_nmap[l] || !last_vmap[l] || !last_nmap[l] || iters[l] < 0)
             return set_err(FU_ERR_ARG, "fu_compute_se3: bad level %d", l);
-    queue_se3(t, next_vmap, next_nmap, last_vmap, last_nmap, nullptr, K, iters, min_count, thresh, S(s));
+    queue_se3(t, false, next_vmap, next_nmap, last_vmap, last_nmap, nullptr, K, iters, min_count, thresh, S(s));
     LAUNCHCHK();
     return FU_OK;
 }
@@ -792,7 +795,7 @@ extern "C" fu_status fu_compute_se3_rgbd(fu_tracker* t, const float* const next_
             !dIdx[l] || !dIdy[l] || iters[l] < 0)
             return set_err(FU_ERR_ARG, "fu_compute_se3_rgbd: bad level %d", l);
     const RgbLevels rgb{next_image, last_image, dIdx, dIdy};
-    queue_se3(t, next_vmap, next_nmap, last_vmap, last_nmap, &rgb, K, iters, min_count, thresh, S(s));
+    queue_se3(t, false, next_vmap, next_nmap, last_vmap, last_nmap, &rgb, K, iters, min_count, thresh, S(s));
     LAUNCHCHK();
     return FU_OK;
 }
@@ -1170,27 +1173,42 @@ static void queue_image_commit(fu_system* sys, hipStream_t s) {
     launch_image_commit(sys->trk->st, src, dst, n, s);
 }
 
-// Frame::FillImages (Core/Frame.cc:59-78); the intensity images only with the photometric term
-static void queue_pyramid(fu_system* sys, const uint16_t* depth, hipStream_t s) {
+static FrameArgs frame_args(fu_system* sys) {
     const fu_system_params& p = sys->p;
     fu_system_buffers& b = sys->b;
-    launch_filter_depth(depth, b.raw, b.depth[0], p.cols, p.rows, (float)(1.0 / (double)p.depth_scale), p.depth_cutoff, s);
-    for (int l = 1; l < 3; ++l) launch_pyrdown(b.depth[l - 1], sys->lc[l - 1], sys->lr[l - 1], b.depth[l], sys->lc[l], sys->lr[l], s);
+    FrameArgs a;
+    a.raw = b.raw;
     for (int l = 0; l < 3; ++l) {
         const float sc = (float)(1 << l);  // Frame::SetK: K / 2^l (Core/Frame.cc:229-237)
-        const float fx = p.fx / sc, fy = p.fy / sc, cx = p.cx / sc, cy = p.cy / sc;
-        launch_vmap(b.depth[l], (f4*)b.vmap[l], sys->lc[l], sys->lr[l], (float)(1.0 / (double)fx),
-                    (float)(1.0 / (double)fy), cx, cy, p.depth_cutoff, s);
-        launch_nmap((const f4*)b.vmap[l], (f4*)b.nmap[l], sys->lc[l], sys->lr[l], s);
+        a.lc[l] = sys->lc[l];
+        a.lr[l] = sys->lr[l];
+        a.depth[l] = b.depth[l];
+        a.vmap[l] = (f4*)b.vmap[l];
+        a.nmap[l] = (f4*)b.nmap[l];
+        a.model_v[l] = (f4*)b.model_vmap[l];
+        a.model_n[l] = (f4*)b.model_nmap[l];
+        a.invf[l][0] = (float)(1.0 / (double)(p.fx / sc));
+        a.invf[l][1] = (float)(1.0 / (double)(p.fy / sc));
+        a.c[l][0] = p.cx / sc;
+        a.c[l][1] = p.cy / sc;
     }
+    a.scale_inv = (float)(1.0 / (double)p.depth_scale);
+    a.cutoff = p.depth_cutoff;
+    a.px = sys->fuse_px;
+    a.prgb = sys->fuse_rgb;
+    return a;
 }
 
-// LastFrame->ResizeImages (Core/Frame.cc:80-84) on the model maps
-static void queue_resize_model(fu_system* sys, hipStream_t s) {
-    fu_system_buffers& b = sys->b;
-    for (int l = 1; l < 3; ++l)
-        launch_resize((const f4*)b.model_vmap[l - 1], (const f4*)b.model_nmap[l - 1], sys->lc[l - 1],
-                      (f4*)b.model_vmap[l], (f4*)b.model_nmap[l], sys->lc[l], sys->lr[l], s);
+// Frame::FillImages (Core/Frame.cc:59-78) and the integration's packed inputs; the intensity
+// images only with the photometric term
+static void queue_pyramid(fu_system* sys, const uint16_t* depth, const uint8_t* rgb, hipStream_t s) {
+    launch_frame_pyramid(frame_args(sys), depth, rgb, s);
+}
+
+// LastFrame->ResizeImages (Core/Frame.cc:80-84) on the model maps; with `begin`, the tracking state
+// begins its frame
+static void queue_resize_model(fu_system* sys, bool begin, hipStream_t s) {
+    launch_frame_resize(frame_args(sys), begin ? sys->trk->st : nullptr, s);
 }
 
 static void mark(fu_system* sys, int boundary, hipStream_t s) {
@@ -1207,10 +1225,11 @@ static void queue_fuse_raycast(fu_system* sys, const uint8_t* rgb, hipStream_t s
     FuseArgs a = make_fuse(m, b.raw, rgb, b.nmap[0], p.cols, p.rows, dummy, st, p.fx, p.fy, p.cx, p.cy);
     a.px = sys->fuse_px;
     a.prgb = sys->fuse_rgb;
-    const VisArgs v = make_vis(m, dummy, st, p.cols, p.rows, p.fx, p.fy, p.cx, p.cy, m->p.depth_min, m->p.depth_max);
-    launch_begin_pass(m->v, 3, s);
-    launch_fuse_pack(a, s);
-    launch_alloc(m->v, a, s);
+    VisArgs v = make_vis(m, dummy, st, p.cols, p.rows, p.fx, p.fy, p.cx, p.cy, m->p.depth_min, m->p.depth_max);
+    v.zmin = (unsigned*)b.zrange_min;
+    v.zmax = (unsigned*)b.zrange_max;
+    v.ztiles = b.zcols * b.zrows;
+    launch_alloc(m->v, a, s);  // the commit has cleared its counters
     mark(sys, FU_STAGE_ALLOC + 1, s);
     launch_visible(m->v, v, s);
     mark(sys, FU_STAGE_VISIBLE + 1, s);
@@ -1218,7 +1237,7 @@ static void queue_fuse_raycast(fu_system* sys, const uint8_t* rgb, hipStream_t s
     mark(sys, FU_STAGE_INTEGRATE + 1, s);
     const ZRangeArgs z = make_zr(m, b.zrange_min, b.zrange_max, b.zcols, b.zrows, m->p.depth_max, m->p.depth_min, dummy,
                                  st, -1, p.fx, p.fy, p.cx, p.cy);
-    launch_zrange(m->v, z, s);
+    launch_zrange(m->v, z, true, s);
     mark(sys, FU_STAGE_ZRANGE + 1, s);
     RaycastArgs r = make_rc(m, b.model_vmap[0], b.model_nmap[0], p.cols, p.rows, b.zrange_min, b.zrange_max, b.zcols,
                             b.zrows, dummy, st, (float)(1.0 / (double)p.fx), (float)(1.0 / (double)p.fy), p.cx, p.cy);
@@ -1232,9 +1251,9 @@ static void queue_frame_device(fu_system* sys, const uint16_t* depth, const uint
     const fu_system_params& p = sys->p;
     fu_system_buffers& b = sys->b;
     mark(sys, 0, s);
-    if (!first) queue_resize_model(sys, s);
+    if (!first) queue_resize_model(sys, true, s);
     mark(sys, FU_STAGE_RESIZE + 1, s);
-    queue_pyramid(sys, depth, s);
+    queue_pyramid(sys, depth, rgb, s);
     if (p.use_rgb) queue_images(sys, rgb, s);
     mark(sys, FU_STAGE_PYRAMID + 1, s);
     if (!first) {
@@ -1248,9 +1267,9 @@ static void queue_frame_device(fu_system* sys, const uint16_t* depth, const uint
         const int16_t* gx[3] = {b.dIdx[0], b.dIdx[1], b.dIdx[2]};
         const int16_t* gy[3] = {b.dIdy[0], b.dIdy[1], b.dIdy[2]};
         const RgbLevels rgbl{ni, li, gx, gy};
-        queue_se3(sys->trk, nv, nn, lv, ln, p.use_rgb ? &rgbl : nullptr, K, p.iters, p.min_count, p.icp_thresh, s);
+        queue_se3(sys->trk, true, nv, nn, lv, ln, p.use_rgb ? &rgbl : nullptr, K, p.iters, p.min_count, p.icp_thresh, s);
     }
-    launch_track_commit(sys->trk->st, s);
+    launch_track_commit(sys->trk->st, sys->map->v, s);
     if (p.use_rgb) queue_image_commit(sys, s);
     mark(sys, FU_STAGE_ICP + 1, s);
     queue_fuse_raycast(sys, rgb, s);
@@ -1263,8 +1282,8 @@ static fu_status run_frame_plain(fu_system* sys, const uint16_t* depth, const ui
     const fu_system_params& p = sys->p;
     fu_system_buffers& b = sys->b;
     fu_tracker* t = sys->trk;
-    if (!first) queue_resize_model(sys, s);
-    queue_pyramid(sys, depth, s);
+    if (!first) queue_resize_model(sys, false, s);
+    queue_pyramid(sys, depth, rgb, s);
     if (p.use_rgb) queue_images(sys, rgb, s);
     HIPCHK(hipStreamSynchronize(s));
     TrackState h;
@@ -1320,7 +1339,6 @@ static fu_status run_frame_plain(fu_system* sys, const uint16_t* depth, const ui
     const VisArgs v = make_vis(m, dummy, t->st, p.cols, p.rows, p.fx, p.fy, p.cx, p.cy, m->p.depth_min, m->p.depth_max);
     launch_begin_pass(m->v, 3, s);
     if (fuse) {
-        launch_fuse_pack(a, s);
         launch_alloc(m->v, a, s);
         HIPCHK(hipStreamSynchronize(s));
     }
@@ -1337,7 +1355,7 @@ static fu_status run_frame_plain(fu_system* sys, const uint16_t* depth, const ui
     if (nvis > 0) {
         const ZRangeArgs z = make_zr(m, b.zrange_min, b.zrange_max, b.zcols, b.zrows, m->p.depth_max, m->p.depth_min,
                                      dummy, t->st, -1, p.fx, p.fy, p.cx, p.cy);
-        launch_zrange(m->v, z, s);
+        launch_zrange(m->v, z, false, s);
         nfrag = read_ctr(m, C_RENDER, s, &st);
         if (st) return st;
     }
@@ -1513,7 +1531,7 @@ static fu_status render_at(fu_system* sys, const double P[16], unsigned min_vis,
     if (nvis > 0) {
         const ZRangeArgs z = make_zr(m, b.zrange_min, b.zrange_max, b.zcols, b.zrows, m->p.depth_max, m->p.depth_min,
                                      pose, nullptr, -1, p.fx, p.fy, p.cx, p.cy);
-        launch_zrange(m->v, z, s);
+        launch_zrange(m->v, z, false, s);
         LAUNCHCHK();
         nfrag = read_ctr(m, C_RENDER, s, &st);
         if (st) return st;
@@ -1527,7 +1545,7 @@ static fu_status render_at(fu_system* sys, const double P[16], unsigned min_vis,
         HIPCHK(hipMemcpyAsync(b.model_vmap[0], b.vmap[0], (size_t)p.cols * p.rows * 16, hipMemcpyDeviceToDevice, s));
         HIPCHK(hipMemcpyAsync(b.model_nmap[0], b.nmap[0], (size_t)p.cols * p.rows * 16, hipMemcpyDeviceToDevice, s));
     }
-    if (resize) queue_resize_model(sys, s);
+    if (resize) queue_resize_model(sys, false, s);
     LAUNCHCHK();
     return FU_OK;
 }
@@ -1545,7 +1563,7 @@ static fu_status icp_from(fu_system* sys, fu_tracker* t, const double P[16], con
     const float* lv[3] = {b.model_vmap[0], b.model_vmap[1], b.model_vmap[2]};
     const float* ln[3] = {b.model_nmap[0], b.model_nmap[1], b.model_nmap[2]};
     const float K[4] = {p.fx, p.fy, p.cx, p.cy};
-    queue_se3(t, nv, nn, lv, ln, nullptr, K, iters, p.min_count, thresh, s);
+    queue_se3(t, false, nv, nn, lv, ln, nullptr, K, iters, p.min_count, thresh, s);
     LAUNCHCHK();
     return fu_tracker_result(t, out, s);
 }
@@ -1678,7 +1696,6 @@ int batch_layout(BatchLaunch& b, const SessDesc* h, BatchTiling t, int level, in
             case BT_ICP: gx = cnt = d.icp_blocks[level] * fixed; break;
             case BT_ONE: gx = cnt = 1; break;
             case BT_FIXED: gx = cnt = fixed; break;
-            case BT_ZTILES: gx = cnt = (d.zr.zcols * d.zr.zrows + 255) / 256; break;
             case BT_ICP_PAIRS: gx = cnt = (d.icp_blocks[level] + 1) / 2 * fixed; break;
         }
         b.pre[i] = total;
@@ -1867,6 +1884,9 @@ static void fill_desc(fu_system* sys, SessDesc& d) {
     d.fuse.px = sys->fuse_px;
     d.fuse.prgb = sys->fuse_rgb;
     d.vis = make_vis(m, dummy, t->st, p.cols, p.rows, p.fx, p.fy, p.cx, p.cy, m->p.depth_min, m->p.depth_max);
+    d.vis.zmin = (unsigned*)b.zrange_min;
+    d.vis.zmax = (unsigned*)b.zrange_max;
+    d.vis.ztiles = b.zcols * b.zrows;
     d.zr = make_zr(m, b.zrange_min, b.zrange_max, b.zcols, b.zrows, m->p.depth_max, m->p.depth_min, dummy, t->st, -1,
                    p.fx, p.fy, p.cx, p.cy);
     d.rc = make_rc(m, b.model_vmap[0], b.model_nmap[0], p.cols, p.rows, b.zrange_min, b.zrange_max, b.zcols, b.zrows,
@@ -1939,8 +1959,7 @@ static void launch_rest(BatchLaunch& b, const SessDesc* h, const int maxit[3], b
         if (prof) (void)hipEventRecord(ev[k], hs);
     };
     for (int i = 0; i < b.n; ++i) b.in[i] = nullptr;
-    if (track) {
-        launch_b_track_begin(b, h, hs);
+    if (track) {  // the model-map resize has begun the tracking states' frames
         if (use_rgb) launch_b_rgb_lists(b, h, hs);
         for (int l = 2; l >= 0; --l)
             for (int j = 0; j < maxit[l]; ++j) launch_b_icp(b, h, l, j, hs);

@@ -111,6 +111,25 @@ __device__ __forceinline__ int batch_slot(const BatchLaunch& b, int wg, WG& g) {
     return s;
 }
 
+// ---- parts of a frame's passes that run inside another pass's launch ----------------------
+// per-frame counters: the new-key count (1) and the visible count (2) start at zero; one lane
+__device__ __forceinline__ void begin_pass(unsigned* ctr, int which) {
+    if (threadIdx.x == 0) {
+        if (which & 1) ctr[C_NEW] = 0;
+        if (which & 2) ctr[C_VISIBLE] = 0;
+    }
+}
+// the tile maps and the fragment counter at the start of a pass
+__device__ __forceinline__ void zrange_init(WG g, unsigned* ctr, const TrackState* st, unsigned* zmin, unsigned* zmax,
+                                                 int n) {
+    if (g.x == 0 && threadIdx.x == 0) FU_G(unsigned, ctr)[C_RENDER] = 0;
+    if (st && !(FU_G(const TrackState, st)->gates & GATE_RENDER)) return;
+    const unsigned hundred = __float_as_uint(100.0f);
+    for (int i = g.x * blockDim.x + threadIdx.x; i < n; i += g.nx * blockDim.x) {
+        zmin[i] = hundred;
+        zmax[i] = 0u;
+    }
+}
 // Copy of a descriptor part, read through the constant address space: the descriptors do not
 // change while a kernel runs, so the loads are scalar and the values live in SGPRs.
 template <class T>
@@ -135,7 +154,6 @@ enum BatchTiling : int {
     BT_ICP = 2,     // icp_blocks[level] * fixed work-groups
     BT_ONE = 3,     // one work-group per session
     BT_FIXED = 4,   // a fixed number of work-groups per session (grid-stride bodies)
-    BT_ZTILES = 5,  // 256-thread groups over the z-range tiles
     BT_ICP_PAIRS = 7,  // (icp_blocks[level] + 1) / 2 * fixed work-groups (kRgbPixels chunks)
 };
 // fills b.pre, b.gx and b.uniform for one launch; returns the total work-group count

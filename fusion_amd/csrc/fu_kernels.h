@@ -115,6 +115,10 @@ struct VisArgs {
     float fx, fy, cx, cy;
     int cols, rows;
     float depth_min, depth_max;
+    // the tile maps of the z-range pass that follows, cleared on the way (null: it clears its own)
+    unsigned* zmin;
+    unsigned* zmax;
+    int ztiles;
 };
 
 struct ZRangeArgs {
@@ -217,6 +221,25 @@ void launch_derivative(const unsigned char* img, short* dx, short* dy, int cols,
 // Tracker::SwapFrame of the intensity pyramid
 void launch_image_commit(const TrackState* st, const unsigned char* const src[3], unsigned char* const dst[3],
                          const int n[3], hipStream_t s);
+// The pyramid stage of a session's frame, a launch per dependency: what a kernel of a level makes,
+// its neighbours in the list above read back, is made together.
+struct FrameArgs {
+    int lc[3], lr[3];
+    float* raw;
+    float* depth[3];
+    f4* vmap[3];
+    f4* nmap[3];
+    f4* model_v[3];
+    f4* model_n[3];
+    float invf[3][2], c[3][2];  // 1 / fx, 1 / fy; cx, cy
+    float scale_inv, cutoff;
+    f4* px;          // the integration's packed inputs (FuseArgs::px, prgb)
+    unsigned* prgb;
+};
+// both smaller levels of the model maps; with `st`, also the start of its tracking (track_begin)
+void launch_frame_resize(const FrameArgs& a, TrackState* st, hipStream_t s);
+// depths, vertex and normal maps of all levels and the packed inputs
+void launch_frame_pyramid(const FrameArgs& a, const uint16_t* depth, const unsigned char* rgb, hipStream_t s);
 // map.hip
 void launch_reset_map(const MapView& m, hipStream_t s);
 void launch_grid_fill(const MapView& m, unsigned n, hipStream_t s);  // from the first n block keys
@@ -224,9 +247,9 @@ void launch_begin_pass(const MapView& m, int which, hipStream_t s);
 void launch_alloc(const MapView& m, const FuseArgs& a, hipStream_t s);
 void launch_visible(const MapView& m, const VisArgs& v, hipStream_t s);
 void launch_integrate(const MapView& m, const FuseArgs& a, unsigned grid, hipStream_t s);
-void launch_fuse_pack(const FuseArgs& a, hipStream_t s);  // fills a.px / a.prgb
 // raycast.hip
-void launch_zrange(const MapView& m, const ZRangeArgs& a, hipStream_t s);
+// cleared: the visibility pass has cleared the tile maps and the fragment counter
+void launch_zrange(const MapView& m, const ZRangeArgs& a, bool cleared, hipStream_t s);
 void launch_raycast(const MapView& m, const RaycastArgs& a, hipStream_t s);
 // mesh.hip
 void upload_mc_tables();
@@ -240,6 +263,6 @@ void launch_icp_step(const IcpArgs& a, int nblocks, const float Rcurr[9], const 
 // the list of eligible pixels of the photometric term for up to three levels (a[l].use_rgb)
 void launch_rgb_lists(const IcpArgs* a, const int* nblocks, int nlevels, hipStream_t s);
 void launch_track_begin(TrackState* st, hipStream_t s);
-void launch_track_commit(TrackState* st, hipStream_t s);
+void launch_track_commit(TrackState* st, const MapView& m, hipStream_t s);  // and begin_pass(3)
 
 }  // namespace fu

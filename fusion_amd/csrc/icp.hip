@@ -1040,14 +1040,16 @@ __device__ __forceinline__ void track_begin_body(TrackState* st) {
 }
 __global__ void k_track_begin(TrackState* st) { track_begin_body(st); }
 // after tracking: the state machine decides what the frame does, and a swapped frame's pose
-// becomes the last pose (frame_commit)
-__device__ __forceinline__ void track_commit_body(TrackState* st) {
-    if (threadIdx.x != 0) return;
-    frame_commit(st);
+// becomes the last pose (frame_commit); the map's counters for the fusion that follows
+__device__ __forceinline__ void track_commit_body(TrackState* st, unsigned* ctr) {
+    if (threadIdx.x == 0) frame_commit(st);
+    begin_pass(ctr, 3);
 }
-__global__ void k_track_commit(TrackState* st) { track_commit_body(st); }
+__global__ void k_track_commit(TrackState* st, unsigned* ctr) { track_commit_body(st, ctr); }
 void launch_track_begin(TrackState* st, hipStream_t s) { hipLaunchKernelGGL(k_track_begin, dim3(1), dim3(64), 0, s, st); }
-void launch_track_commit(TrackState* st, hipStream_t s) { hipLaunchKernelGGL(k_track_commit, dim3(1), dim3(64), 0, s, st); }
+void launch_track_commit(TrackState* st, const MapView& m, hipStream_t s) {
+    hipLaunchKernelGGL(k_track_commit, dim3(1), dim3(64), 0, s, st, m.ctr);
+}
 
 // ------------------------------------------------------------------ batched launches
 // The iteration schedule is the union of the sessions' schedules: a session runs iteration
@@ -1127,7 +1129,10 @@ __global__ void kb_track_begin(BatchLaunch b) {
     if (slot_first(b, s)) return;
     track_begin_body(b.desc[b.sess[s]].st);
 }
-__global__ void kb_track_commit(BatchLaunch b) { track_commit_body(b.desc[b.sess[blockIdx.x]].st); }
+__global__ void kb_track_commit(BatchLaunch b) {
+    const SessDesc& d = b.desc[b.sess[blockIdx.x]];
+    track_commit_body(d.st, d.m.ctr);
+}
 
 // tracking result and map counters of every slot, into out[slot]
 __global__ void kb_results(BatchLaunch b, FrameBrief* out) {

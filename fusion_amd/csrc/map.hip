@@ -63,13 +63,7 @@ void launch_grid_fill(const MapView& m, unsigned n, hipStream_t s) {
 }
 
 // per-frame counters: the new-key count and the visible count start at zero
-__device__ __forceinline__ void begin_pass_body(unsigned* ctr, int which) {
-    if (threadIdx.x == 0) {
-        if (which & 1) ctr[C_NEW] = 0;
-        if (which & 2) ctr[C_VISIBLE] = 0;
-    }
-}
-__global__ void k_begin_pass(unsigned* ctr, int which) { begin_pass_body(ctr, which); }
+__global__ void k_begin_pass(unsigned* ctr, int which) { begin_pass(ctr, which); }
 void launch_begin_pass(const MapView& m, int which, hipStream_t s) {
     hipLaunchKernelGGL(k_begin_pass, dim3(1), dim3(64), 0, s, m.ctr, which);
 }
@@ -373,6 +367,7 @@ __device__ __forceinline__ bool block_visible(const VisArgs& v, const PoseF& pos
 // set is the same (every allocated block has exactly one live entry).  Compaction is a
 // wave ballot plus one atomic per wave.
 __device__ __forceinline__ void visible_body(WG g, const MapView& m, const VisArgs& v) {
+    if (v.zmin) zrange_init(g, m.ctr, v.st, v.zmin, v.zmax, v.ztiles);  // uniform
     PoseF pose = v.pose;
     if (v.st && !pose_from_state(v.st, pose)) return;
     const unsigned nalloc = min(FU_G(const unsigned, m.ctr)[C_ALLOC], m.num_blocks);
@@ -572,17 +567,6 @@ __global__ __launch_bounds__(kIntThreads) void k_integrate(MapView m, FuseArgs a
     integrate_body<F, kPacked>(hw_wg(), m, a);
 }
 
-// the packed per-pixel inputs of integration (FuseArgs::px, prgb)
-__device__ __forceinline__ void fuse_pack_body(WG g, const FuseArgs& a) {
-    const int i = (g.y * g.nx + g.x) * 256 + threadIdx.x;
-    if (i >= a.cols * a.rows) return;
-    const f4 n = FU_G(const f4, a.nmap)[i];
-    const auto c = FU_G(const unsigned char, a.rgb) + 3 * i;
-    FU_G(f4, a.px)[i] = mk4(FU_G(const float, a.depth)[i], n.x, n.y, n.z);
-    FU_G(unsigned, a.prgb)[i] = (unsigned)c[0] | ((unsigned)c[1] << 8) | ((unsigned)c[2] << 16);
-}
-__global__ __launch_bounds__(256) void k_fuse_pack(FuseArgs a) { fuse_pack_body(hw_wg(), a); }
-
 template <bool kPacked>
 static void integrate_f(const MapView& m, const FuseArgs& a, unsigned grid, hipStream_t s) {
     switch (m.fmt) {
@@ -590,10 +574,6 @@ static void integrate_f(const MapView& m, const FuseArgs& a, unsigned grid, hipS
         case VF_F32_W16: hipLaunchKernelGGL((k_integrate<VF_F32_W16, kPacked>), dim3(grid), dim3(kIntThreads), 0, s, m, a); break;
         default: hipLaunchKernelGGL((k_integrate<VF_F16_W8, kPacked>), dim3(grid), dim3(kIntThreads), 0, s, m, a); break;
     }
-}
-void launch_fuse_pack(const FuseArgs& a, hipStream_t s) {
-    const int n = a.cols * a.rows;
-    hipLaunchKernelGGL(k_fuse_pack, dim3((n + 255) / 256), dim3(256), 0, s, a);
 }
 void launch_integrate(const MapView& m, const FuseArgs& a, unsigned grid, hipStream_t s) {
     if (a.px)
@@ -605,7 +585,6 @@ void launch_integrate(const MapView& m, const FuseArgs& a, unsigned grid, hipStr
 // ------------------------------------------------------------------ batched launches
 // FuseMapColor for every session of a step: counters, allocation (both passes), visible
 // list and integration, each stage one launch over all sessions.
-__global__ void kb_begin_pass(BatchLaunch b) { begin_pass_body(b.desc[b.sess[blockIdx.x]].m.ctr, 3); }
 
 __device__ __forceinline__ FuseArgs slot_fuse(const BatchLaunch& b, const SessDesc& d, int s) {
     FuseArgs a = d.fuse;
@@ -650,8 +629,8 @@ static int per_slot(int total, int n, int lo, int hi) {
 }
 
 void launch_b_alloc(BatchLaunch& b, const SessDesc* h, hipStream_t s) {
-    hipLaunchKernelGGL(kb_begin_pass, dim3(b.n), dim3(64), 0, s, b);
-    // the integration inputs were packed by the normal pass (kb_nmap)
+    // the integration inputs were packed by the normal pass (kb_nmap), the counters cleared with the
+    // tracking's commit
     int grid = batch_layout(b, h, BT_TILES, 0, 0);
     hipLaunchKernelGGL(kb_alloc_a, dim3(grid), dim3(kAllocThreads), 0, s, b);
     grid = batch_layout(b, h, BT_FIXED, 0, per_slot(tuning().alloc_groups, b.n, 16, 512));

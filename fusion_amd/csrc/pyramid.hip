@@ -8,6 +8,7 @@
 #include "fu_device.h"
 #include "fu_kernels.h"
 #include "fu_batch.h"
+#include "fu_track.h"
 
 namespace fu {
 
@@ -223,6 +224,99 @@ __global__ __launch_bounds__(256) void k_resize(const f4* __restrict__ vsrc, con
     resize_body(hw_wg(), vsrc, nsrc, scols, vdst, ndst, dcols, drows);
 }
 
+// ------------------------------------------------------------------ a session's frame
+// The bodies below run for one session (FrameArgs) and for a batch's (SessDesc).
+// Levels 1 and 2 of the model maps in one pass over 16x16 tiles of level 1: each lane makes
+// its level-1 pixel as resize_body does and keeps it in LDS; after the barrier the lanes of
+// even (x, y) make the level-2 pixel of their 2x2 quad from those four values, the ones a
+// level-2 resize would read back.  A level-2 pixel (x2, y2) exists only when 2*x2 + 1 and
+// 2*y2 + 1 are level-1 pixels, and its quad lies in the tile.
+template <class D>
+__device__ __forceinline__ void resize2_body(WG g, const D& d) {
+    __shared__ f4 tv[16][16], tn[16][16];
+    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
+    const int x = g.x * 16 + tx, y = g.y * 16 + ty;
+    const int c0 = d.lc[0], c1 = d.lc[1];
+    if (x < c1 && y < d.lr[1]) {
+        const auto vsrc = FU_G(const f4, d.model_v[0]);
+        const auto nsrc = FU_G(const f4, d.model_n[0]);
+        const int s0 = (2 * y) * c0 + 2 * x, s1 = (2 * y + 1) * c0 + 2 * x;
+        f4 vo, no;
+        resize_px(vsrc[s0], vsrc[s0 + 1], vsrc[s1], vsrc[s1 + 1], nsrc[s0], nsrc[s0 + 1], nsrc[s1], nsrc[s1 + 1], vo,
+                  no);
+        FU_G(f4, d.model_v[1])[y * c1 + x] = vo;
+        FU_G(f4, d.model_n[1])[y * c1 + x] = no;
+        tv[ty][tx] = vo;
+        tn[ty][tx] = no;
+    }
+    __syncthreads();
+    const int x2 = x >> 1, y2 = y >> 1, c2 = d.lc[2];
+    if (!(tx & 1) && !(ty & 1) && x2 < c2 && y2 < d.lr[2]) {
+        f4 vo, no;
+        resize_px(tv[ty][tx], tv[ty][tx + 1], tv[ty + 1][tx], tv[ty + 1][tx + 1], tn[ty][tx], tn[ty][tx + 1],
+                  tn[ty + 1][tx], tn[ty + 1][tx + 1], vo, no);
+        FU_G(f4, d.model_v[2])[y2 * c2 + x2] = vo;
+        FU_G(f4, d.model_n[2])[y2 * c2 + x2] = no;
+    }
+}
+
+// one launch over the tiles of all three levels; `local` -> (level, tile)
+template <class D>
+__device__ __forceinline__ int pyr3_level(const D& d, int local, WG& g) {
+    int l = 0;
+    while (l < 2) {
+        const int tx = (d.lc[l] + 15) / 16, t = tx * ((d.lr[l] + 15) / 16);
+        if (local < t) break;
+        local -= t;
+        ++l;
+    }
+    const int tx = (d.lc[l] + 15) / 16;
+    g.x = local % tx;
+    g.y = local / tx;
+    g.nx = tx;
+    g.ny = (d.lr[l] + 15) / 16;
+    return l;
+}
+
+// the normals of all levels (g.x: a tile of the three), and of level 0 the integration's inputs of
+// the pixel: its normal, depth and colour, packed
+template <class D>
+__device__ __forceinline__ void normals3_body(WG g, const D& d, const unsigned char* rgb, f4* px, unsigned* prgb) {
+    const int l = pyr3_level(d, g.x, g);
+    const int cols = d.lc[l];
+    const int x = g.x * 16 + (threadIdx.x & 15);
+    const int y = g.y * 16 + (threadIdx.x >> 4);
+    if (x >= cols || y >= d.lr[l]) return;
+    const int i = y * cols + x;
+    const f4 n = normal_of(d.vmap[l], x, y, cols, d.lr[l]);
+    FU_G(f4, d.nmap[l])[i] = n;
+    if (l == 0) {  // uniform
+        const auto c = FU_G(const unsigned char, rgb) + 3 * i;
+        FU_G(f4, px)[i] = mk4(FU_G(const float, d.raw)[i], n.x, n.y, n.z);
+        FU_G(unsigned, prgb)[i] = (unsigned)c[0] | ((unsigned)c[1] << 8) | ((unsigned)c[2] << 16);
+    }
+}
+
+// A frame's launches are bound by their gaps and latency (640x480: 2.5 to 5 us each).  Those of one
+// map at a time, as the entry points of the single operations launch them, were eleven with the
+// packing and the start of tracking; these are five: a 640x480 frame 405 -> 392 us.
+__global__ __launch_bounds__(256) void k_frame_resize(FrameArgs a, TrackState* st) {
+    if (st && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) frame_begin(st);
+    resize2_body(hw_wg(), a);
+}
+__global__ __launch_bounds__(256) void k_frame_filter(FrameArgs a, const uint16_t* depth) {
+    filter_depth_body(hw_wg(), depth, a.raw, a.depth[0], a.lc[0], a.lr[0], a.scale_inv, a.cutoff,
+                      VertexOut{a.vmap[0], a.invf[0][0], a.invf[0][1], a.c[0][0], a.c[0][1]});
+}
+template <int L>
+__global__ __launch_bounds__(256) void k_frame_pyrdown(FrameArgs a) {
+    pyrdown_body(hw_wg(), a.depth[L - 1], a.lc[L - 1], a.lr[L - 1], a.depth[L], a.lc[L], a.lr[L],
+                 VertexOut{a.vmap[L], a.invf[L][0], a.invf[L][1], a.c[L][0], a.c[L][1]}, a.cutoff);
+}
+__global__ __launch_bounds__(256) void k_frame_normals(FrameArgs a, const unsigned char* rgb) {
+    normals3_body(hw_wg(), a, rgb, a.px, a.prgb);
+}
+
 // ------------------------------------------------------------------ intensity pyramid
 // ImageToIntensityKernel (Pyrdown.cu:183-194): (int)(0.2125 c1 + 0.7154 c0 + 0.0721 c2) in
 // double, evaluated as written (no fused multiply-add), stored as a byte
@@ -411,45 +505,29 @@ void launch_resize(const f4* vsrc, const f4* nsrc, int scols, f4* vdst, f4* ndst
     hipLaunchKernelGGL(k_resize, grid16(dcols, drows), dim3(256), 0, s, vsrc, nsrc, scols, vdst, ndst, dcols, drows);
 }
 
+void launch_frame_resize(const FrameArgs& a, TrackState* st, hipStream_t s) {
+    hipLaunchKernelGGL(k_frame_resize, grid16(a.lc[1], a.lr[1]), dim3(256), 0, s, a, st);
+}
+void launch_frame_pyramid(const FrameArgs& a, const uint16_t* depth, const unsigned char* rgb, hipStream_t s) {
+    hipLaunchKernelGGL(k_frame_filter, grid16(a.lc[0], a.lr[0]), dim3(256), 0, s, a, depth);
+    hipLaunchKernelGGL(k_frame_pyrdown<1>, grid16(a.lc[1], a.lr[1]), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(k_frame_pyrdown<2>, grid16(a.lc[2], a.lr[2]), dim3(256), 0, s, a);
+    int tiles = 0;
+    for (int l = 0; l < 3; ++l) tiles += ((a.lc[l] + 15) / 16) * ((a.lr[l] + 15) / 16);
+    hipLaunchKernelGGL(k_frame_normals, dim3(tiles), dim3(256), 0, s, a, rgb);
+}
+
 // ------------------------------------------------------------------ batched launches
 // Each work-group finds its session's share (batch_slot) and runs the body the single-session
 // kernel runs, with the same work-group ids.
 
-// levels 1 and 2 of the model maps in one pass over 16x16 tiles of level 1: each lane makes
-// its level-1 pixel as resize_body does and keeps it in LDS; after the barrier the lanes of
-// even (x, y) make the level-2 pixel of their 2x2 quad from those four values, the ones a
-// level-2 resize would read back.  A level-2 pixel (x2, y2) exists only when 2*x2 + 1 and
-// 2*y2 + 1 are level-1 pixels, and its quad lies in the tile.
 __global__ __launch_bounds__(256) void kb_resize(BatchLaunch b) {
     WG g;
     const int s = batch_slot(b, blockIdx.x, g);
     if (slot_first(b, s)) return;  // uniform: the first frame has no model maps
     const SessDesc& d = b.desc[b.sess[s]];
-    __shared__ f4 tv[16][16], tn[16][16];
-    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-    const int x = g.x * 16 + tx, y = g.y * 16 + ty;
-    const int c0 = d.lc[0], c1 = d.lc[1];
-    if (x < c1 && y < d.lr[1]) {
-        const auto vsrc = FU_G(const f4, d.model_v[0]);
-        const auto nsrc = FU_G(const f4, d.model_n[0]);
-        const int s0 = (2 * y) * c0 + 2 * x, s1 = (2 * y + 1) * c0 + 2 * x;
-        f4 vo, no;
-        resize_px(vsrc[s0], vsrc[s0 + 1], vsrc[s1], vsrc[s1 + 1], nsrc[s0], nsrc[s0 + 1], nsrc[s1], nsrc[s1 + 1], vo,
-                  no);
-        FU_G(f4, d.model_v[1])[y * c1 + x] = vo;
-        FU_G(f4, d.model_n[1])[y * c1 + x] = no;
-        tv[ty][tx] = vo;
-        tn[ty][tx] = no;
-    }
-    __syncthreads();
-    const int x2 = x >> 1, y2 = y >> 1, c2 = d.lc[2];
-    if (!(tx & 1) && !(ty & 1) && x2 < c2 && y2 < d.lr[2]) {
-        f4 vo, no;
-        resize_px(tv[ty][tx], tv[ty][tx + 1], tv[ty + 1][tx], tv[ty + 1][tx + 1], tn[ty][tx], tn[ty][tx + 1],
-                  tn[ty + 1][tx], tn[ty + 1][tx + 1], vo, no);
-        FU_G(f4, d.model_v[2])[y2 * c2 + x2] = vo;
-        FU_G(f4, d.model_n[2])[y2 * c2 + x2] = no;
-    }
+    if (g.x == 0 && g.y == 0 && threadIdx.x == 0) frame_begin(d.st);
+    resize2_body(g, d);
 }
 
 __global__ __launch_bounds__(256) void kb_filter(BatchLaunch b) {
@@ -469,42 +547,11 @@ __global__ __launch_bounds__(256) void kb_pyrdown(BatchLaunch b) {
                  VertexOut{d.vmap[l], d.invf[l][0], d.invf[l][1], d.Kl[l][2], d.Kl[l][3]}, d.cutoff);
 }
 
-// one launch over the tiles of all three levels; `local` -> (level, tile)
-__device__ __forceinline__ int pyr3_level(const SessDesc& d, int local, WG& g) {
-    int l = 0;
-    while (l < 2) {
-        const int tx = (d.lc[l] + 15) / 16, t = tx * ((d.lr[l] + 15) / 16);
-        if (local < t) break;
-        local -= t;
-        ++l;
-    }
-    const int tx = (d.lc[l] + 15) / 16;
-    g.x = local % tx;
-    g.y = local / tx;
-    g.nx = tx;
-    g.ny = (d.lr[l] + 15) / 16;
-    return l;
-}
-
 __global__ __launch_bounds__(256) void kb_nmap(BatchLaunch b) {
     WG g;
     const int s = batch_slot(b, blockIdx.x, g);
     const SessDesc& d = b.desc[b.sess[s]];
-    const int l = pyr3_level(d, g.x, g);
-    const int cols = d.lc[l];
-    const int x = g.x * 16 + (threadIdx.x & 15);
-    const int y = g.y * 16 + (threadIdx.x >> 4);
-    if (x >= cols || y >= d.lr[l]) return;
-    const int i = y * cols + x;
-    const f4 n = normal_of(d.vmap[l], x, y, cols, d.lr[l]);
-    FU_G(f4, d.nmap[l])[i] = n;
-    if (l == 0) {
-        // uniform: the integration inputs of the pixel (k_fuse_pack) from the normal above,
-        // the level-0 depth and the step's colour frame (b.in)
-        const auto c = FU_G(const unsigned char, (const unsigned char*)b.in[s]) + 3 * i;
-        FU_G(f4, d.fuse.px)[i] = mk4(FU_G(const float, d.fuse.depth)[i], n.x, n.y, n.z);
-        FU_G(unsigned, d.fuse.prgb)[i] = (unsigned)c[0] | ((unsigned)c[1] << 8) | ((unsigned)c[2] << 16);
-    }
+    normals3_body(g, d, (const unsigned char*)b.in[s], d.fuse.px, d.fuse.prgb);
 }
 
 // intensity pyramid of the sessions with the photometric term (the others have no share)

@@ -18,19 +18,8 @@
 
 namespace fu {
 
-// the tile maps and the fragment counter at the start of a pass
-__device__ __forceinline__ void zrange_init_body(WG g, unsigned* ctr, const TrackState* st, unsigned* zmin, unsigned* zmax,
-                                                 int n) {
-    if (g.x == 0 && threadIdx.x == 0) FU_G(unsigned, ctr)[C_RENDER] = 0;
-    if (st && !(FU_G(const TrackState, st)->gates & GATE_RENDER)) return;
-    const unsigned hundred = __float_as_uint(100.0f);
-    for (int i = g.x * blockDim.x + threadIdx.x; i < n; i += g.nx * blockDim.x) {
-        zmin[i] = hundred;
-        zmax[i] = 0u;
-    }
-}
 __global__ void k_zrange_init(unsigned* ctr, const TrackState* st, unsigned* zmin, unsigned* zmax, int n) {
-    zrange_init_body(hw_wg(), ctr, st, zmin, zmax, n);
+    zrange_init(hw_wg(), ctr, st, zmin, zmax, n);
 }
 
 // exclusive prefix sum of `v` over the lanes of a wave, and the wave total in `total`
@@ -156,9 +145,10 @@ __global__ __launch_bounds__(kLds ? kProjectLanes : 256) void k_project_blocks(M
     project_body<kLds>(hw_wg(), m, a);
 }
 
-void launch_zrange(const MapView& m, const ZRangeArgs& a, hipStream_t s) {
+void launch_zrange(const MapView& m, const ZRangeArgs& a, bool cleared, hipStream_t s) {
     const int n = a.zcols * a.zrows;
-    hipLaunchKernelGGL(k_zrange_init, dim3((n + 255) / 256), dim3(256), 0, s, m.ctr, a.st, a.zmin, a.zmax, n);
+    if (!cleared)
+        hipLaunchKernelGGL(k_zrange_init, dim3((n + 255) / 256), dim3(256), 0, s, m.ctr, a.st, a.zmin, a.zmax, n);
     if (n <= kZTilesLds)
         hipLaunchKernelGGL(k_project_blocks<true>, dim3(kProjectGroups), dim3(kProjectLanes), 0, s, m, a);
     else
@@ -483,12 +473,6 @@ void launch_raycast(const MapView& m, const RaycastArgs& a, hipStream_t s) {
 
 // ------------------------------------------------------------------ batched launches
 // Mapping::RayTrace for every session of a step: z-range tiles, block projection, ray march.
-__global__ void kb_zrange_init(BatchLaunch b) {
-    WG g;
-    const int s = batch_slot(b, blockIdx.x, g);
-    const SessDesc& d = b.desc[b.sess[s]];
-    zrange_init_body(g, d.m.ctr, d.st, d.zr.zmin, d.zr.zmax, d.zr.zcols * d.zr.zrows);
-}
 template <bool kLds>
 __global__ __launch_bounds__(kLds ? kProjectLanes : 256) void kb_project(BatchLaunch b) {
     WG g;
@@ -505,9 +489,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
 }
 
 void launch_b_zrange(BatchLaunch& b, const SessDesc* h, hipStream_t s) {
-    int grid = batch_layout(b, h, BT_ZTILES, 0, 0);
-    hipLaunchKernelGGL(kb_zrange_init, dim3(grid), dim3(256), 0, s, b);
-    bool lds = true;
+    int grid = 0;
+    bool lds = true;  // (the visibility pass has cleared the tile maps)
     for (int i = 0; i < b.n; ++i) lds = lds && h[b.sess[i]].zr.zcols * h[b.sess[i]].zr.zrows <= kZTilesLds;
     if (lds) {
         grid = batch_layout(b, h, BT_FIXED, 0, kProjectGroups);

@@ -52,3 +52,38 @@ def test_image_forms_bit_exact(gpu, cols, rows):
     ox, oy = O.derivative_image(img)
     assert np.array_equal(dx.cpu().numpy(), ox)
     assert np.array_equal(dy.cpu().numpy(), oy)
+
+
+@pytest.mark.parametrize("cols,rows", [(32, 32), (36, 44), (100, 68), (128, 64)])
+def test_frame_pyramid_equals_the_single_operations(gpu, cols, rows):
+    # a session's frame makes its maps in launches of its own, level by level; the model maps of a
+    # frame are those of the raycast before it, halved
+    print("frame %dx%d" % (cols, rows), flush=True)
+    K = (0.9 * cols, 0.9 * cols, cols / 2 - 0.5, rows / 2 - 0.5)
+    rng = np.random.default_rng(cols)
+    y, x = np.mgrid[0:rows, 0:cols]
+    mp = dict(num_buckets=1 << 14, num_excess=1 << 13, num_blocks=1 << 13, voxel_size=0.02, trunc_dist=0.06,
+              max_new_blocks=1 << 14)
+    s = A.System(A.system_params(cols=cols, rows=rows, K=K, map=mp))
+    bits = lambda t: t.cpu().numpy()
+    for k in range(2):
+        d = (5000 * (1.2 + 0.002 * x + 0.003 * y) + 5 * rng.standard_normal((rows, cols))).astype(np.uint16)
+        d[rng.random((rows, cols)) < 0.02] = 0
+        rgb = rng.integers(0, 256, (rows, cols, 3), dtype=np.uint8)
+        last = [s.view("model_vmap").clone(), s.view("model_nmap").clone()]
+        s.GrabImage(*A.to_device(d, rgb))
+        torch.cuda.synchronize()
+        raw, f = A.FilterDepth(torch.from_numpy(d.view(np.int16)).cuda(), s.params.depth_scale, s.params.depth_cutoff)
+        assert same_bits(bits(s.view("raw")), bits(raw))
+        for l in range(3):
+            f = A.PyrDownGauss(f) if l else f
+            v = A.ComputeVMap(f, *A.level_k(K, l), s.params.depth_cutoff)
+            assert same_bits(bits(s.view("depth", l)), bits(f)), l
+            assert same_bits(bits(s.view("vmap", l)), bits(v)), l
+            assert same_bits(bits(s.view("nmap", l)), bits(A.ComputeNMap(v))), l
+        for l in (1, 2):
+            if k:
+                last = A.ResizeMap(*last)
+                assert same_bits(bits(s.view("model_vmap", l)), bits(last[0])), l
+                assert same_bits(bits(s.view("model_nmap", l)), bits(last[1])), l
+    s.close()
