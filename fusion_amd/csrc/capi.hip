@@ -713,7 +713,20 @@ static IcpArgs make_icp(fu_tracker* t, int level, const float* nv, const float* 
     a.thresh = thresh;
     a.use_rgb = 0;
     memset(&a.rgb, 0, sizeof(a.rgb));
+    a.zcurr = nullptr;
+    a.invfx = a.invfy = a.cutoff = 0.f;
+    a.row_magic = 0;
     return a;
+}
+// the current vertices are those of the system's own pyramid
+static void set_depth(IcpArgs& a, const fu_system* sys, int level) {
+    // i * row_magic >> 32 is i / cols for every pixel i (exact while i * cols < 2^32)
+    if ((unsigned long long)a.cols * a.cols * a.rows > 0xFFFFFFFFull) return;
+    a.zcurr = sys->b.depth[level];
+    a.invfx = (float)(1.0 / (double)a.fx);
+    a.invfy = (float)(1.0 / (double)a.fy);
+    a.cutoff = sys->p.depth_cutoff;
+    a.row_magic = (unsigned)(0x100000000ull / (unsigned)a.cols + 1);
 }
 
 // the photometric inputs of one level (RGBStep's images, Tracking.cc:319-325)
@@ -740,11 +753,11 @@ struct RgbLevels {
 };
 
 // queue the whole coarse-to-fine loop (device-resident)
-// `begun`: the state has begun its frame (track_begin)
-static void queue_se3(fu_tracker* t, bool begun, const float* const nv[3], const float* const nn[3],
+// `frame`: the system whose frame this is, whose tracking state has begun it (track_begin); or null
+static void queue_se3(fu_tracker* t, const fu_system* frame, const float* const nv[3], const float* const nn[3],
                       const float* const lv[3], const float* const ln[3], const RgbLevels* rgb, const float K[4], const int32_t iters[3],
                       const int32_t minc[3], float thresh, hipStream_t s) {
-    if (!begun) launch_track_begin(t->st, s);
+    if (!frame) launch_track_begin(t->st, s);
     int last_level = -1;
     for (int l = 2; l >= 0; --l)
         if (iters[l] > 0) last_level = l;
@@ -761,6 +774,7 @@ static void queue_se3(fu_tracker* t, bool begun, const float* const nv[3], const
         for (int j = 0; j < iters[l]; ++j) {
             const int fin = (l == last_level && j == iters[l] - 1);
             IcpArgs a = make_icp(t, l, nv[l], nn[l], lv[l], ln[l], K, 1, minc[l], fin, thresh);
+            if (frame) set_depth(a, frame, l);
             if (rgb) set_rgb(a, t, l, rgb->next_image[l], rgb->last_image[l], rgb->dx[l], rgb->dy[l]);
             launch_icp(a, a.use_rgb ? t->nblocks[l] : t->ngroups[l], s);
         }
@@ -774,7 +788,7 @@ extern "C" fu_status fu_compute_se3(fu_tracker* t, const float* const next_vmap[
     for (int l = 0; l < 3; ++l)
         if (!next_vmap[l] || !next_nmap[l] || !last_vmap[l] || !last_nmap[l] || iters[l] < 0)
             return set_err(FU_ERR_ARG, "fu_compute_se3: bad level %d", l);
-    queue_se3(t, false, next_vmap, next_nmap, last_vmap, last_nmap, nullptr, K, iters, min_count, thresh, S(s));
+    queue_se3(t, nullptr, next_vmap, next_nmap, last_vmap, last_nmap, nullptr, K, iters, min_count, thresh, S(s));
     LAUNCHCHK();
     return FU_OK;
 }
@@ -795,7 +809,7 @@ extern "C" fu_status fu_compute_se3_rgbd(fu_tracker* t, const float* const next_
             !dIdx[l] || !dIdy[l] || iters[l] < 0)
             return set_err(FU_ERR_ARG, "fu_compute_se3_rgbd: bad level %d", l);
     const RgbLevels rgb{next_image, last_image, dIdx, dIdy};
-    queue_se3(t, false, next_vmap, next_nmap, last_vmap, last_nmap, &rgb, K, iters, min_count, thresh, S(s));
+    queue_se3(t, nullptr, next_vmap, next_nmap, last_vmap, last_nmap, &rgb, K, iters, min_count, thresh, S(s));
     LAUNCHCHK();
     return FU_OK;
 }
@@ -1267,7 +1281,7 @@ static void queue_frame_device(fu_system* sys, const uint16_t* depth, const uint
         const int16_t* gx[3] = {b.dIdx[0], b.dIdx[1], b.dIdx[2]};
         const int16_t* gy[3] = {b.dIdy[0], b.dIdy[1], b.dIdy[2]};
         const RgbLevels rgbl{ni, li, gx, gy};
-        queue_se3(sys->trk, true, nv, nn, lv, ln, p.use_rgb ? &rgbl : nullptr, K, p.iters, p.min_count, p.icp_thresh, s);
+        queue_se3(sys->trk, sys, nv, nn, lv, ln, p.use_rgb ? &rgbl : nullptr, K, p.iters, p.min_count, p.icp_thresh, s);
     }
     launch_track_commit(sys->trk->st, sys->map->v, s);
     if (p.use_rgb) queue_image_commit(sys, s);
@@ -1563,7 +1577,7 @@ static fu_status icp_from(fu_system* sys, fu_tracker* t, const double P[16], con
     const float* lv[3] = {b.model_vmap[0], b.model_vmap[1], b.model_vmap[2]};
     const float* ln[3] = {b.model_nmap[0], b.model_nmap[1], b.model_nmap[2]};
     const float K[4] = {p.fx, p.fy, p.cx, p.cy};
-    queue_se3(t, false, nv, nn, lv, ln, nullptr, K, iters, p.min_count, thresh, s);
+    queue_se3(t, nullptr, nv, nn, lv, ln, nullptr, K, iters, p.min_count, thresh, s);
     LAUNCHCHK();
     return fu_tracker_result(t, out, s);
 }
@@ -1869,6 +1883,7 @@ static void fill_desc(fu_system* sys, SessDesc& d) {
         d.model_n[l] = (f4*)b.model_nmap[l];
         d.icp[l] = make_icp(t, l, b.vmap[l], b.nmap[l], b.model_vmap[l], b.model_nmap[l], K, 1, p.min_count[l], 0,
                             p.icp_thresh);
+        set_depth(d.icp[l], sys, l);
         if (p.use_rgb) {
             set_rgb(d.icp[l], t, l, b.image[l], b.last_image[l], b.dIdx[l], b.dIdy[l]);
             d.image[l] = b.image[l];

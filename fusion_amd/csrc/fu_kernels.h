@@ -183,6 +183,16 @@ struct RgbArgs {
     int* corr;    // 2 ints per residual-pass work-group: count, sum of diff^2 (32-bit, wrapping)
 };
 
+// ComputeVMapKernel's vertex of pixel (x, y) with depth z (Pyrdown.cu:56-78)
+__device__ __forceinline__ f4 vertex_of(float z, int x, int y, float invfx, float invfy, float cx, float cy,
+                                        float cutoff) {
+    // `z > 0.1` compares in double (Pyrdown.cu:69)
+    if (!isnanf_(z) && (double)z > 0.1 && z < cutoff)
+        return mk4(z * ((float)x - cx) * invfx, z * ((float)y - cy) * invfy, z, 1.0f);
+    // the reference sets only x = NaN; every consumer tests x alone
+    return mk4(fnan(), fnan(), fnan(), fnan());
+}
+
 struct IcpArgs {
     const f4* vcurr;
     const f4* ncurr;
@@ -198,6 +208,11 @@ struct IcpArgs {
     float thresh;
     int use_rgb;      // 1: RGBStep is blended into every iteration (ComputeSE3 icpOnly = false)
     RgbArgs rgb;
+    // where the caller made vcurr from a depth map (null: it did not): the depth, the inverse focal
+    // lengths and the cutoff of vertex_of, and floor(2^32 / cols) + 1 (a pixel's row)
+    const float* zcurr;
+    float invfx, invfy, cutoff;
+    unsigned row_magic;
 };
 
 // frames with the photometric term are limited to 2^22 pixels (the residual record packs

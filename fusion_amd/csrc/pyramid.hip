@@ -16,15 +16,6 @@ namespace fu {
 constexpr float kSigSpace = 0.5f / 16.0f;
 constexpr float kSigRange = 2.0f;
 
-// ComputeVMapKernel's vertex of pixel (x, y) with depth z (Pyrdown.cu:56-78)
-__device__ __forceinline__ f4 vertex_of(float z, int x, int y, float invfx, float invfy, float cx, float cy,
-                                        float cutoff) {
-    // `z > 0.1` compares in double (Pyrdown.cu:69)
-    if (!isnanf_(z) && (double)z > 0.1 && z < cutoff)
-        return mk4(z * ((float)x - cx) * invfx, z * ((float)y - cy) * invfy, z, 1.0f);
-    // the reference sets only x = NaN; every consumer tests x alone
-    return mk4(fnan(), fnan(), fnan(), fnan());
-}
 // where a depth kernel also writes the vertex map of its level (null vmap: it does not)
 struct VertexOut {
     f4* vmap;
