@@ -16,7 +16,7 @@ struct alignas(16) SurfHead {
     float normal[4];
 };
 
-fu_status keymap_count(fu_keymap* k, uint32_t* n_keys, hipStream_t s);
+uint32_t keymap_count(const fu_keymap* k);
 fu_status keymap_pack(fu_keymap* k, float* desc, int32_t* slot, hipStream_t s);
 const SurfHead* keymap_heads(const fu_keymap* k);  // of the map's slots, kSlotHeads apart
 constexpr int kSlotHeads = sizeof(fu_surf) / sizeof(SurfHead);

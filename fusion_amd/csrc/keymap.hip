@@ -48,6 +48,8 @@ struct KeyArgs {
     Surf* keys;        // the map: max_keys * nbuckets records
     int* mutex;        // KeyMap::Mutex (reset to -1; the inserts here do not lock)
     int* owner;        // per bucket: INT_MAX, or the lowest index of a waiting key this round
+    unsigned* bits;    // a bit per slot: its key is valid
+    unsigned* valid;   // their number
     int max_keys, nbuckets;
     float grid;
 };
@@ -58,6 +60,8 @@ __global__ void k_reset_keys(KeyArgs a, int n) {
     if (i >= n) return;
     a.mutex[i] = -1;
     a.keys[i].valid = 0;
+    if ((i & 31) == 0) a.bits[i >> 5] = 0u;
+    if (i == 0) *a.valid = 0u;
     if (i < a.max_keys) a.owner[i] = INT_MAX;
 }
 
@@ -100,26 +104,31 @@ __global__ void k_insert_apply(KeyArgs a, Surf* in, int* index, unsigned char* d
         const uint4* src = reinterpret_cast<const uint4*>(&in[i]);
         uint4* dst = reinterpret_cast<uint4*>(&a.keys[first]);
         for (int q = 0; q < (int)(sizeof(Surf) / 16); ++q) dst[q] = src[q];
+        if (in[i].valid) {
+            atomicOr(&a.bits[first >> 5], 1u << (first & 31));
+            atomicAdd(a.valid, 1u);
+        }
     }
     done[i] = 1;
     a.owner[b] = INT_MAX;
 }
 
 // CollectKeys (FuseMap.cu:384-406) in slot order: valid key j (0-based over the slots) goes to
-// out[j] when 0 < j < cap (the reference copies only at offsets > 0).  k_collect_count leaves a
-// word of valid bits per 64 slots and the count of each 1024-slot group, and its last group to
-// end turns the counts into their exclusive prefix (16 us in all, as with a launch for the prefix,
-// without the gap between the two).  It is bound by the records' first lines (500,000 slots: 32 MB,
-// 11 us); the copies that follow read only the bits and the valid records (20,000 of 500,000 slots,
-// a lane per record behind its slot's flag: 20 us, now 6).
-constexpr int kCollect = 1024;
+// out[j] when 0 < j < cap (the reference copies only at offsets > 0).  k_collect_count counts the
+// valid bits of each 1024-slot group, and its last work-group to end turns the counts into their
+// exclusive prefix; the copies that follow read only the bits and the valid records (20,000 of
+// 500,000 slots: a lane per record behind its slot's flag took 20 us, now 6).  Inserts keep the bits:
+// reading a flag in every slot's record was 32 MB and 11 us, with the prefix 16, now 5.
+constexpr int kCollect = 1024;              // slots per group
+constexpr int kWords = kCollect / 64;       // 64-bit words per group
+constexpr int kCountGroups = 256 / kWords;  // groups per work-group of k_collect_count, a word per lane
 struct CollectArgs {
     const Surf* keys;
-    int n, groups;
-    unsigned* counts;          // per group; then its exclusive prefix
+    int groups;
+    unsigned* counts;                // per group; then its exclusive prefix
     unsigned* total;
-    unsigned* arrived;         // groups that have counted; 0 between calls
-    unsigned long long* bits;  // 16 words per group
+    unsigned* arrived;               // work-groups that have counted; 0 between calls
+    const unsigned long long* bits;  // kWords per group, zero past the slots
 };
 // between work-groups of a launch: through the memory that all XCDs share
 __device__ __forceinline__ void store_shared(unsigned* p, unsigned v) {
@@ -128,29 +137,25 @@ __device__ __forceinline__ void store_shared(unsigned* p, unsigned v) {
 __device__ __forceinline__ unsigned load_shared(const unsigned* p) {
     return __hip_atomic_load(FU_G(const unsigned, p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__global__ __launch_bounds__(kCollect) void k_collect_count(CollectArgs a) {
-    __shared__ unsigned wsum[kCollect / 64];
+__global__ __launch_bounds__(256) void k_collect_count(CollectArgs a) {
+    __shared__ unsigned wsum[4];
     __shared__ int last;
-    const int i = blockIdx.x * kCollect + threadIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const unsigned long long m = __ballot(i < a.n && a.keys[i].valid);
-    if (lane == 0) {
-        a.bits[blockIdx.x * (kCollect / 64) + w] = m;
-        wsum[w] = (unsigned)__popcll(m);
-    }
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int group = blockIdx.x * kCountGroups + threadIdx.x / kWords;
+    unsigned c = group < a.groups ? (unsigned)__popcll(a.bits[blockIdx.x * 256 + threadIdx.x]) : 0u;
+#pragma unroll
+    for (int d = 1; d < kWords; d <<= 1) c += __shfl_xor(c, d);
+    if (group < a.groups && threadIdx.x % kWords == 0) store_shared(&a.counts[group], c);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the wave's counts are in place
     __syncthreads();
-    if (threadIdx.x == 0) {
-        unsigned c = 0;
-        for (int k = 0; k < kCollect / 64; ++k) c += wsum[k];
-        store_shared(&a.counts[blockIdx.x], c);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the count is in place
+    if (threadIdx.x == 0)
         last = __hip_atomic_fetch_add(FU_G(unsigned, a.arrived), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-               (unsigned)a.groups - 1u;
-    }
+               gridDim.x - 1u;
     __syncthreads();
     if (!last) return;  // uniform
     // lane t owns a run of consecutive counts; the runs' sums are scanned across the work-group
     // (integer sums: the same as one lane walking the counts in order)
-    const int per = (a.groups + kCollect - 1) / kCollect;
+    const int per = (a.groups + 255) / 256;
     const int b = min(a.groups, (int)threadIdx.x * per), e = min(a.groups, b + per);
     unsigned own = 0;
     for (int g = b; g < e; ++g) own += load_shared(&a.counts[g]);
@@ -164,16 +169,15 @@ __global__ __launch_bounds__(kCollect) void k_collect_count(CollectArgs a) {
     __syncthreads();
     unsigned before = 0, all = 0;
 #pragma unroll
-    for (int k = 0; k < kCollect / 64; ++k) {
-        const unsigned c = wsum[k];
-        before += k < w ? c : 0u;
-        all += c;
+    for (int k = 0; k < 4; ++k) {
+        before += k < w ? wsum[k] : 0u;
+        all += wsum[k];
     }
     unsigned run = before + x - own;
     for (int g = b; g < e; ++g) {
-        const unsigned c = load_shared(&a.counts[g]);
+        const unsigned n = load_shared(&a.counts[g]);
         a.counts[g] = run;
-        run += c;
+        run += n;
     }
     if (threadIdx.x == 0) {
         *a.total = all;
@@ -186,7 +190,6 @@ __global__ __launch_bounds__(kCollect) void k_collect_count(CollectArgs a) {
 template <bool kPack>
 __global__ __launch_bounds__(256) void k_collect_copy(CollectArgs a, Surf* out, float* desc, int* slot, unsigned cap) {
     const int word = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    constexpr int kWords = kCollect / 64;
     if (word >= a.groups * kWords) return;  // uniform
     unsigned long long m = a.bits[word];
     if (!m) return;  // uniform
@@ -267,8 +270,10 @@ __global__ void k_adjacency(const SurfHead* frame, const SurfHead* map, int stri
 struct fu_keymap {
     fu_keymap_params p;
     KeyArgs a;
-    unsigned* aux = nullptr;    // [0] keys left in a round, [1] collect total, [2] groups counted,
-                                // from [4] a 64-slot word of valid bits each, then group counts
+    unsigned* aux = nullptr;    // [0] keys left in a round, [1] collect total, [2] work-groups that
+                                // have counted, [3] valid keys, from [4] the slots' valid bits,
+                                // then group counts
+    uint32_t n_valid = 0;       // aux[3] as of the last insert
     int dev = -1;               // the device the map was created on
     unsigned char* done = nullptr;  // per key of an insert call, grown on demand
     int* bucket = nullptr;
@@ -302,11 +307,11 @@ extern "C" fu_status fu_keymap_destroy(fu_keymap* k) {
 
 static int n_slots(const fu_keymap* k) { return k->a.max_keys * k->a.nbuckets; }
 static int n_groups(const fu_keymap* k) { return (n_slots(k) + kCollect - 1) / kCollect; }
+static size_t aux_bytes(const fu_keymap* k) { return (4 + (size_t)n_groups(k) * (2 * kWords + 1)) * 4; }
 static CollectArgs collect_args(const fu_keymap* k) {
     const int g = n_groups(k);
-    unsigned* bits = k->aux + 4;
-    return CollectArgs{k->a.keys, n_slots(k),         g, bits + (size_t)g * (2 * kCollect / 64), k->aux + 1,
-                       k->aux + 2, (unsigned long long*)bits};
+    return CollectArgs{k->a.keys,  g,          k->a.bits + (size_t)g * (2 * kWords), k->aux + 1,
+                       k->aux + 2, (const unsigned long long*)k->a.bits};
 }
 
 extern "C" fu_status fu_keymap_create(const fu_keymap_params* p, fu_keymap** out) {
@@ -323,7 +328,7 @@ extern "C" fu_status fu_keymap_create(const fu_keymap_params* p, fu_keymap** out
     const size_t n = (size_t)n_slots(k);
     if (hipMalloc(&k->a.keys, n * sizeof(Surf)) != hipSuccess || hipMalloc(&k->a.mutex, n * 4) != hipSuccess ||
         hipMalloc(&k->a.owner, (size_t)p->max_keys * 4) != hipSuccess ||
-        hipMalloc(&k->aux, (4 + (size_t)n_groups(k) * (2 * kCollect / 64 + 1)) * 4) != hipSuccess) {
+        hipMalloc(&k->aux, aux_bytes(k)) != hipSuccess) {
         (void)hipGetLastError();
         fu_keymap_destroy(k);
         return api_error(FU_ERR_NOMEM, "fu_keymap_create: allocation failed");
@@ -331,7 +336,9 @@ extern "C" fu_status fu_keymap_create(const fu_keymap_params* p, fu_keymap** out
     // records start zeroed (ResetKeys clears only the valid flags, so a record's other bytes
     // keep what the last key there left)
     k->dev = current_device();
-    if (hipMemset(k->a.keys, 0, n * sizeof(Surf)) != hipSuccess || hipMemset(k->aux, 0, 16) != hipSuccess) {
+    k->a.bits = k->aux + 4;
+    k->a.valid = k->aux + 3;
+    if (hipMemset(k->a.keys, 0, n * sizeof(Surf)) != hipSuccess || hipMemset(k->aux, 0, aux_bytes(k)) != hipSuccess) {
         (void)hipGetLastError();
         fu_keymap_destroy(k);
         return api_error(FU_ERR_HIP, "fu_keymap_create: clearing the records failed");
@@ -352,6 +359,7 @@ extern "C" fu_status fu_keymap_create(const fu_keymap_params* p, fu_keymap** out
 extern "C" fu_status fu_reset_key_points(fu_keymap* k, fu_stream s) {
     if (!k) return api_error(FU_ERR_ARG, "fu_reset_key_points: null key map");
     const int n = n_slots(k);
+    k->n_valid = 0;
     hipLaunchKernelGGL(k_reset_keys, dim3((n + 255) / 256), dim3(256), 0, (hipStream_t)s, k->a, n);
     KM_HIP(hipGetLastError());
     return FU_OK;
@@ -384,19 +392,24 @@ extern "C" fu_status fu_insert_key_points(fu_keymap* k, fu_surf* keys, int32_t* 
         hipLaunchKernelGGL(k_insert_apply, grid, dim3(256), 0, hs, k->a, (Surf*)keys, index, k->done, k->bucket, (int)n,
                            k->aux);
         KM_HIP(hipGetLastError());
-        unsigned left = 0;
-        KM_HIP(hipMemcpyAsync(&left, k->aux, 4, hipMemcpyDeviceToHost, hs));
+        unsigned aux[4] = {};
+        KM_HIP(hipMemcpyAsync(aux, k->aux, sizeof(aux), hipMemcpyDeviceToHost, hs));
         KM_HIP(hipStreamSynchronize(hs));
-        if (left == 0) return FU_OK;
+        k->n_valid = aux[3];
+        if (aux[0] == 0) return FU_OK;
     }
     return api_error(FU_ERR_STATE, "fu_insert_key_points: inserts did not finish");
+}
+
+static void launch_count(const CollectArgs& a, hipStream_t s) {
+    hipLaunchKernelGGL(k_collect_count, dim3((a.groups + kCountGroups - 1) / kCountGroups), dim3(256), 0, s, a);
 }
 
 extern "C" fu_status fu_collect_key_points(fu_keymap* k, fu_surf* out, uint32_t cap, uint32_t* n_keys, fu_stream s) {
     if (!k || !n_keys || (cap && !out)) return api_error(FU_ERR_ARG, "fu_collect_key_points: null argument");
     hipStream_t hs = (hipStream_t)s;
     const CollectArgs a = collect_args(k);
-    hipLaunchKernelGGL(k_collect_count, dim3(a.groups), dim3(kCollect), 0, hs, a);
+    launch_count(a, hs);
     if (cap)
         hipLaunchKernelGGL(k_collect_copy<false>, dim3(a.groups * (kCollect / 256)), dim3(256), 0, hs, a, (Surf*)out,
                            nullptr, nullptr, cap);
@@ -406,14 +419,12 @@ extern "C" fu_status fu_collect_key_points(fu_keymap* k, fu_surf* out, uint32_t 
 }
 
 namespace fu {
-// the number of valid keys; synchronises the stream
-fu_status keymap_count(fu_keymap* k, uint32_t* n_keys, hipStream_t s) {
-    return fu_collect_key_points(k, nullptr, 0, n_keys, (fu_stream)s);
-}
-// after keymap_count with nothing inserted since, for its n keys: their descriptors (n x 64,
-// 16-byte aligned) and slots, key 0 as zeros and slot -1
+// the number of valid keys (an insert returns when its keys are in place)
+uint32_t keymap_count(const fu_keymap* k) { return k->n_valid; }
+// for its n keys: their descriptors (n x 64, 16-byte aligned) and slots, key 0 as zeros and slot -1
 fu_status keymap_pack(fu_keymap* k, float* desc, int32_t* slot, hipStream_t s) {
     const CollectArgs a = collect_args(k);
+    launch_count(a, s);
     hipLaunchKernelGGL(k_collect_copy<true>, dim3(a.groups * (kCollect / 256)), dim3(256), 0, s, a, nullptr, desc, slot, 0u);
     KM_HIP(hipGetLastError());
     return FU_OK;
