@@ -277,6 +277,7 @@ static VisArgs make_vis(const fu_map* m, const PoseF& pose, const TrackState* st
     v.depth_max = dmax;
     v.zmin = v.zmax = nullptr;
     v.ztiles = 0;
+    v.after_alloc = 0;
     (void)m;
     return v;
 }
@@ -293,9 +294,9 @@ extern "C" fu_status fu_fuse_map_color(fu_map* m, const float* depth, const uint
     const PoseF p = posef_from(pose);
     const FuseArgs a = make_fuse(m, depth, rgb, nmap, cols, rows, p, nullptr, fx, fy, cx, cy);
     // the fusion visibility test uses DeviceMap::DepthMin/DepthMax (FuseMap.cu:288-289)
-    const VisArgs v = make_vis(m, p, nullptr, cols, rows, fx, fy, cx, cy, m->p.depth_min, m->p.depth_max);
-    launch_begin_pass(m->v, 3, S(s));
-    launch_alloc(m->v, a, S(s));
+    VisArgs v = make_vis(m, p, nullptr, cols, rows, fx, fy, cx, cy, m->p.depth_min, m->p.depth_max);
+    v.after_alloc = 1;
+    launch_alloc(m->v, a, true, S(s));
     launch_visible(m->v, v, S(s));
     launch_integrate(m->v, a, kIntegrateGrid, S(s));
     LAUNCHCHK();
@@ -1243,7 +1244,8 @@ static void queue_fuse_raycast(fu_system* sys, const uint8_t* rgb, hipStream_t s
     v.zmin = (unsigned*)b.zrange_min;
     v.zmax = (unsigned*)b.zrange_max;
     v.ztiles = b.zcols * b.zrows;
-    launch_alloc(m->v, a, s);  // the commit has cleared its counters
+    v.after_alloc = 1;
+    launch_alloc(m->v, a, false, s);  // the commit has cleared the counters
     mark(sys, FU_STAGE_ALLOC + 1, s);
     launch_visible(m->v, v, s);
     mark(sys, FU_STAGE_VISIBLE + 1, s);
@@ -1350,10 +1352,11 @@ static fu_status run_frame_plain(fu_system* sys, const uint16_t* depth, const ui
     FuseArgs a = make_fuse(m, b.raw, rgb, b.nmap[0], p.cols, p.rows, dummy, t->st, p.fx, p.fy, p.cx, p.cy);
     a.px = sys->fuse_px;
     a.prgb = sys->fuse_rgb;
-    const VisArgs v = make_vis(m, dummy, t->st, p.cols, p.rows, p.fx, p.fy, p.cx, p.cy, m->p.depth_min, m->p.depth_max);
+    VisArgs v = make_vis(m, dummy, t->st, p.cols, p.rows, p.fx, p.fy, p.cx, p.cy, m->p.depth_min, m->p.depth_max);
+    v.after_alloc = 1;
     launch_begin_pass(m->v, 3, s);
     if (fuse) {
-        launch_alloc(m->v, a, s);
+        launch_alloc(m->v, a, false, s);
         HIPCHK(hipStreamSynchronize(s));
     }
     launch_visible(m->v, v, s);
@@ -1902,6 +1905,7 @@ static void fill_desc(fu_system* sys, SessDesc& d) {
     d.vis.zmin = (unsigned*)b.zrange_min;
     d.vis.zmax = (unsigned*)b.zrange_max;
     d.vis.ztiles = b.zcols * b.zrows;
+    d.vis.after_alloc = 1;
     d.zr = make_zr(m, b.zrange_min, b.zrange_max, b.zcols, b.zrows, m->p.depth_max, m->p.depth_min, dummy, t->st, -1,
                    p.fx, p.fy, p.cx, p.cy);
     d.rc = make_rc(m, b.model_vmap[0], b.model_nmap[0], p.cols, p.rows, b.zrange_min, b.zrange_max, b.zcols, b.zrows,

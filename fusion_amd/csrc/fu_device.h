@@ -33,13 +33,13 @@ enum Counter : int {
     C_ALLOC = 0,    // blocks taken from the pool (bump index; may exceed capacity, clamp on read)
     C_EXCESS = 1,   // excess slots used
     C_VISIBLE = 2,  // entries of the visible list
-    C_NEW = 3,      // new keys found by the current allocation pass
+    C_NEW = 3,      // new keys found by the last allocation pass
     C_FLAGS = 4,    // sticky overflow flags (FU_FLAG_*)
     C_RENDER = 5,   // rendering fragments of the last z-range pass
     C_TRI = 6,      // triangles of the last mesh pass
     C_DONE = 7,     // chunks of the running mesh scan whose sums are in place
     C_OCC = 8,      // occupied blocks seen by the last mesh pass
-    C_SPARE = 9,
+    C_PENDING = 9,  // new keys of the running allocation pass, 0 between passes
     C_COUNT = 16
 };
 

@@ -119,6 +119,7 @@ struct VisArgs {
     unsigned* zmin;
     unsigned* zmax;
     int ztiles;
+    int after_alloc;  // ends an allocation pass: C_PENDING becomes C_NEW
 };
 
 struct ZRangeArgs {
@@ -259,7 +260,8 @@ void launch_frame_pyramid(const FrameArgs& a, const uint16_t* depth, const unsig
 void launch_reset_map(const MapView& m, hipStream_t s);
 void launch_grid_fill(const MapView& m, unsigned n, hipStream_t s);  // from the first n block keys
 void launch_begin_pass(const MapView& m, int which, hipStream_t s);
-void launch_alloc(const MapView& m, const FuseArgs& a, hipStream_t s);
+// clear: also starts the visible count at zero; launch_visible with after_alloc follows
+void launch_alloc(const MapView& m, const FuseArgs& a, bool clear, hipStream_t s);
 void launch_visible(const MapView& m, const VisArgs& v, hipStream_t s);
 void launch_integrate(const MapView& m, const FuseArgs& a, unsigned grid, hipStream_t s);
 // raycast.hip

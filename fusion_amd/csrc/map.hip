@@ -92,7 +92,7 @@ __device__ __forceinline__ void claim_block(const MapView& m, bool want, unsigne
     bool won = false;
     unsigned slot = 0;
     if (want && find_block(m, bp) < 0) won = newset_claim(m, key, slot);
-    const unsigned idx = wave_append(&m.ctr[C_NEW], won);
+    const unsigned idx = wave_append(&m.ctr[C_PENDING], won);
     if (won) {
         if (idx < m.max_new) {
             m.newkeys[idx] = key;
@@ -239,14 +239,19 @@ __device__ __forceinline__ void alloc_a_body(WG g, const MapView& m, const FuseA
         claim_block(m, i < n && in, pack_key(b), b);
     }
 }
-__global__ __launch_bounds__(kAllocThreads) void k_alloc_pass_a(MapView m, FuseArgs p) { alloc_a_body(hw_wg(), m, p); }
+// clear: a fusion outside a session's frame, whose visible count nobody has cleared yet (as a launch
+// of its own, with the new keys' count, 4.5 of the 109 us that a 640x480 fusion and raycast take)
+__global__ __launch_bounds__(kAllocThreads) void k_alloc_pass_a(MapView m, FuseArgs p, bool clear) {
+    if (clear && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) m.ctr[C_VISIBLE] = 0;
+    alloc_a_body(hw_wg(), m, p);
+}
 
 // ------------------------------------------------------------ allocation pass B (per new key)
 // one wave per new block: lane 0 links the key, all lanes initialise the block's voxels
 // (sdf NaN, weight 0, colour 0: Voxel::release, DeviceMap.h:75-79)
 __device__ __forceinline__ void alloc_b_body(WG g, const MapView& m, const TrackState* st) {
     if (st && !frame_fuses(st)) return;
-    const unsigned nnew = min(m.ctr[C_NEW], m.max_new);
+    const unsigned nnew = min(m.ctr[C_PENDING], m.max_new);
     const int wave = (g.x * blockDim.x + threadIdx.x) >> 6;
     const int nwaves = (g.nx * blockDim.x) >> 6;
     const int lane = lane_id();
@@ -322,8 +327,9 @@ __device__ __forceinline__ void alloc_b_body(WG g, const MapView& m, const Track
 }
 __global__ __launch_bounds__(256) void k_alloc_pass_b(MapView m, const TrackState* st) { alloc_b_body(hw_wg(), m, st); }
 
-void launch_alloc(const MapView& m, const FuseArgs& p, hipStream_t s) {
-    hipLaunchKernelGGL(k_alloc_pass_a, dim3((p.cols + 15) / 16, (p.rows + 15) / 16), dim3(kAllocThreads), 0, s, m, p);
+void launch_alloc(const MapView& m, const FuseArgs& p, bool clear, hipStream_t s) {
+    hipLaunchKernelGGL(k_alloc_pass_a, dim3((p.cols + 15) / 16, (p.rows + 15) / 16), dim3(kAllocThreads), 0, s, m, p,
+                       clear);
     hipLaunchKernelGGL(k_alloc_pass_b, dim3(512), dim3(256), 0, s, m, p.st);
 }
 
@@ -367,6 +373,11 @@ __device__ __forceinline__ bool block_visible(const VisArgs& v, const PoseF& pos
 // set is the same (every allocated block has exactly one live entry).  Compaction is a
 // wave ballot plus one atomic per wave.
 __device__ __forceinline__ void visible_body(WG g, const MapView& m, const VisArgs& v) {
+    // no later reader of this launch: the visible count has been cleared before the allocation
+    if (v.after_alloc && g.x == 0 && threadIdx.x == 0) {
+        m.ctr[C_NEW] = m.ctr[C_PENDING];
+        m.ctr[C_PENDING] = 0;
+    }
     if (v.zmin) zrange_init(g, m.ctr, v.st, v.zmin, v.zmax, v.ztiles);  // uniform
     PoseF pose = v.pose;
     if (v.st && !pose_from_state(v.st, pose)) return;
