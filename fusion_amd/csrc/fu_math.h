@@ -152,12 +152,17 @@ FU_HD float fu_expf(float x) {
     s2.u = (uint32_t)(k2 + 127) << 23;
     return (p * s1.f) * s2.f;
 }
-// fu_expf for x <= 0 that is not NaN (the bilateral weights), without the NaN and overflow
-// tests and with the scaling in one exponent-field add and one multiply: k is in [-149, 0],
-// p * 2^(k+64) is a normal float (exact) and the multiply by 2^-64 rounds once, as the
-// second multiply of fu_expf does, so both give the same bits
+// fu_expf for x <= 0 that is not NaN (the bilateral weights), without the NaN and overflow tests.
+// On the device the scaling is v_ldexp_f32, which rounds once, as the second multiply of fu_expf
+// does (whatever it makes of a p and k from below -103 is discarded).  On the host it is one
+// exponent-field add and one multiply: k is in [-149, 0], p * 2^(k+64) is a normal float (exact)
+// and the multiply by 2^-64 rounds once.  All three give the same bits.
 FU_HD float fu_expf_nonpos(float x) {
     int k;
+#if defined(__HIP_DEVICE_COMPILE__)
+    const float p = fu_expf_poly(x, k);
+    return x < -103.0f ? 0.0f : __builtin_amdgcn_ldexpf(p, k);
+#else
     const float p = fu_expf_poly(fmaxf(x, -103.0f), k);
     union { uint32_t u; float f; } s;
     union { float f; uint32_t u; } pb;
@@ -165,6 +170,7 @@ FU_HD float fu_expf_nonpos(float x) {
     s.u = pb.u + ((uint32_t)(k + 64) << 23);
     const float e = s.f * 0x1p-64f;
     return x < -103.0f ? 0.0f : e;
+#endif
 }
 
 // ---------------------------------------------------------------------------------------

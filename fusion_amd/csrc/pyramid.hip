@@ -46,19 +46,34 @@ __device__ __forceinline__ void filter_depth_body(WG g, const uint16_t* __restri
     raw[y * cols + x] = center < cutoff ? center : fnan();
     // the window is [max(p-2,0), min(p+3, n-1)) in each axis: the last row/column of the
     // image never contributes (Pyrdown.cu:23-29)
-    const int tx = min(x + 3, cols - 1);
-    const int ty = min(y + 3, rows - 1);
     float sum1 = 0.f, sum2 = 0.f;
-    for (int cy = max(y - 2, 0); cy < ty; ++cy) {
-        for (int cx = max(x - 2, 0); cx < tx; ++cx) {
-            const float val = tile[(cy - y0) * T + (cx - x0)];
-            const float space2 = (float)((x - cx) * (x - cx) + (y - cy) * (y - cy));
-            const float color2 = (center - val) * (center - val);
-            // the argument is never positive or NaN: depths are finite
-            const float weight = fu_expf_nonpos(-(space2 * kSigSpace + color2 * kSigRange));
-            sum1 += val * weight;
-            sum2 += weight;
+    auto tap = [&](float val, float space2) {
+        const float color2 = (center - val) * (center - val);
+        // the argument is never positive or NaN: depths are finite
+        const float weight = fu_expf_nonpos(-(space2 * kSigSpace + color2 * kSigRange));
+        sum1 += val * weight;
+        sum2 += weight;
+    };
+    // Bound by the taps' instructions: a tile inside the image (uniform) takes its 25 unrolled, with
+    // constant distances and places, and its centre, whose weight is exp(-0) = 1, without one: about
+    // 31 instructions a tap instead of 47.  1280x720: 25.3 -> 20.3 us; 22 sessions of 640x480
+    // 71 -> 57 us.
+    if (x0 >= 0 && y0 >= 0 && x0 + T < cols && y0 + T < rows) {
+        const float* const at = &tile[(y - y0 - 2) * T + (x - x0 - 2)];
+#pragma unroll
+        for (int q = 0; q < 25; ++q) {
+            if (q == 12) {
+                sum1 += center;
+                sum2 += 1.0f;
+            } else {
+                tap(at[(q / 5) * T + q % 5], (float)((q % 5 - 2) * (q % 5 - 2) + (q / 5 - 2) * (q / 5 - 2)));
+            }
         }
+    } else {
+        const int tx = min(x + 3, cols - 1), ty = min(y + 3, rows - 1);
+        for (int cy = max(y - 2, 0); cy < ty; ++cy)
+            for (int cx = max(x - 2, 0); cx < tx; ++cx)
+                tap(tile[(cy - y0) * T + (cx - x0)], (float)((x - cx) * (x - cx) + (y - cy) * (y - cy)));
     }
     const float fin = sum1 / sum2;
     const float z = fin < cutoff ? fin : fnan();
