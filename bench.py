@@ -637,11 +637,12 @@ def rooflines(st, sizes, nsess):
     # raycast: lower bound of W*H*32 B written (vertex + normal) plus each visible block's
     # sdf and weight planes read once (8 B per voxel)
     b_rc = per_step * (px * 32 + nvis * 512 * 8)
-    # ICP: 64 B per pixel-iteration (current vertex+normal, last vertex+normal)
-    b_icp = (st["icp_pixels"] / steps) * 64
+    # ICP: 52 B per pixel-iteration (current depth, from which the vertex is made, and normal, last
+    # vertex+normal)
+    b_icp = (st["icp_pixels"] / steps) * 52
     for name, b, kern, tkey in (("integrate", b_int, "kb_integrate<VF_F32_W8>", "kb_integrate<0>"),
                                 ("raycast", b_rc, "kb_raycast<VF_F32_W8>", "kb_raycast<0>"),
-                                ("icp", b_icp, "kb_icp + kb_icp_final (stage)", None)):
+                                ("icp", b_icp, "kb_icp (stage)", None)):
         ms = st["ms"][name] / steps
         ach = b / (ms * 1e-3) / 1e9 if ms > 0 else 0.0
         # measured HBM bytes of a 32-frame launch (counter runs), scaled to this step size
@@ -655,24 +656,24 @@ def rooflines(st, sizes, nsess):
                          frac=round(ach / HBM_PEAK_GBS, 4), traffic=traffic, kernel=kern, bytes_per_launch=int(b),
                          avg_launch_us=round(ms * 1e3, 2), frames_per_launch=round(per_step, 2),
                          n_visible_per_frame=round(nvis, 1))
-        if name == "icp":  # a stage: the figures are per step, over the step's launch pairs
-            out[name]["note"] = ("per step: %d kb_icp + kb_icp_final launch pairs (ICP iterations), bytes and "
-                                 "time summed over them" % round(st["icp_iterations"] / frames))
+        if name == "icp":  # a stage: the figures are per step, over the step's iterations
+            out[name]["note"] = ("per step: %d kb_icp launches (ICP iterations), bytes and time summed over them"
+                                 % round(st["icp_iterations"] / frames))
     return out
 
 
 def rgb_tracking_roofline(st):
-    """the tracking stage with the photometric term: per pixel-iteration the ICP inputs (64 B)
+    """the tracking stage with the photometric term: per pixel-iteration the ICP inputs (52 B)
     plus this frame's intensity, the last frame's intensity at the match, the two derivatives
-    and the residual record written and read back (1 + 1 + 4 + 8 B) - 78 B as the algorithmic
-    lower bound, over the stage's HIP-event time (three launches per iteration)"""
+    and the residual record written and read back (1 + 1 + 4 + 8 B) - 66 B as the algorithmic
+    lower bound, over the stage's HIP-event time (two launches per iteration)"""
     steps = max(1.0, st["steps"])
-    b = (st["icp_pixels"] / steps) * 78
+    b = (st["icp_pixels"] / steps) * 66
     ms = st["ms"]["icp"] / steps
     ach = b / (ms * 1e-3) / 1e9 if ms > 0 else 0.0
     return dict(bound="hbm", achieved=round(ach, 1), peak=HBM_PEAK_GBS, unit="GB/s", frac=round(ach / HBM_PEAK_GBS, 4),
                 bytes_per_step=int(b), stage_ms_per_step=round(ms, 4),
-                kernels="kb_rgb_resid + kb_icp_rgb + kb_icp_rgb_final per iteration")
+                kernels="kb_rgb_resid + kb_icp_rgb per iteration")
 
 
 def cpu_baseline(A, seconds):
@@ -787,8 +788,8 @@ def main():
     fps = r["tracked"] / r["wall"]
     st = r.get("stages")
     rl = rooflines(st, sizes, ns) if st else None
-    # the kernel with the most GPU time per step: the ICP reduction (kb_icp with its final sum,
-    # one launch pair per iteration) ahead of the raycast and the integration
+    # the kernel with the most GPU time per step: the ICP reduction (kb_icp, one launch per
+    # iteration) ahead of the raycast and the integration
     dominant = max(("integrate", "raycast", "icp"), key=lambda k: rl[k]["avg_launch_us"]) if rl else None
     steps_p = max(1.0, st["steps"]) if st else 1.0
     out = {

@@ -349,7 +349,7 @@ def _track_result(r):
 
 
 class IcpBatch:
-    """fu_compute_se3_batch: ComputeSE3 for many trackers, each iteration one launch pair"""
+    """fu_compute_se3_batch: ComputeSE3 for many trackers, each iteration one launch"""
 
     def __init__(self, capacity=256):
         _dev()

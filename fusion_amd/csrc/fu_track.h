@@ -1,9 +1,7 @@
 // FP64 pose arithmetic of Tracker::ComputeSE3 (Tracking/Tracking.cc:368-408): unpacking of
 // the 29 reduced sums (Reduction.cu:6-16), the 6x6 solve, the SE(3) exponential and the
-// pose composition.  Host and device share this code: the device-resident tracker runs it
-// on one lane of the last ICP work-group, the reference-style path on the host.  Every loop
-// has a constant trip count and is unrolled, so on the device all matrices live in
-// registers (no private-memory spills on the critical path of each ICP iteration).
+// pose composition, as the reference-style path runs them on the host; the device-resident
+// tracker's form is a wave's (icp_update_wave, icp.hip).  frame_begin and frame_commit are shared.
 #pragma once
 
 #include <math.h>

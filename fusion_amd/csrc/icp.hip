@@ -10,14 +10,14 @@
 // one partial row per work-group (frames with more pixel chunks than work-groups sum their
 // chunks per lane with Neumaier-compensated FP32 adds first).
 // The work-group whose row arrives last sums the rows with the same compensated tree and
-// (mode 1) unpacks A (6x6) and b (6) in FP64, solves by Cholesky, takes the SE(3) exponential
+// (mode 1) unpacks A (6x6) and b (6) in FP64, solves by Gauss-Jordan, takes the SE(3) exponential
 // and composes the pose on its first wave: the only FP64 steps of the pipeline.
 //
 // With the photometric term (ComputeSE3 icpOnly = false) every iteration is two launches:
 // the RGB residual pass (RGBReduction::ComputeResidual, Reduction.cu:469-483: one residual
 // record per pixel and the integer sums of each work-group) and one pass that computes both
-// the ICP and the weighted RGB rows of each pixel (each work-group first adds the integer sums
-// up to sigma itself) and reduces 64 values per lane; its last work-group blends
+// the ICP rows of the pixels and the weighted RGB rows of the list in work-groups of their own (the
+// latter first add the integer sums up to sigma themselves); the last to end blends
 // A_rgb * 1e-4f + A_icp in FP64 before the solve.
 #include "fu_device.h"
 #include "fu_kernels.h"
