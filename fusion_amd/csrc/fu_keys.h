@@ -17,7 +17,7 @@ struct alignas(16) SurfHead {
 };
 
 uint32_t keymap_count(const fu_keymap* k);
-fu_status keymap_pack(fu_keymap* k, float* desc, int32_t* slot, hipStream_t s);
+fu_status keymap_pack(fu_keymap* k, float* desc, int32_t* slot, uint32_t n, hipStream_t s);
 const SurfHead* keymap_heads(const fu_keymap* k);  // of the map's slots, kSlotHeads apart
 constexpr int kSlotHeads = sizeof(fu_surf) / sizeof(SurfHead);
 int keymap_device(const fu_keymap* k);

@@ -125,7 +125,8 @@ constexpr int kCountGroups = 256 / kWords;  // groups per work-group of k_collec
 struct CollectArgs {
     const Surf* keys;
     int groups;
-    unsigned* counts;                // per group; then its exclusive prefix
+    unsigned* counts;                // per group
+    unsigned* base;                  // their exclusive prefix
     unsigned* total;
     unsigned* arrived;               // work-groups that have counted; 0 between calls
     const unsigned long long* bits;  // kWords per group, zero past the slots
@@ -149,8 +150,7 @@ __global__ __launch_bounds__(256) void k_collect_count(CollectArgs a) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the wave's counts are in place
     __syncthreads();
     if (threadIdx.x == 0)
-        last = __hip_atomic_fetch_add(FU_G(unsigned, a.arrived), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-               gridDim.x - 1u;
+        last = atomicInc(a.arrived, gridDim.x - 1u) == gridDim.x - 1u;  // and back to 0
     __syncthreads();
     if (!last) return;  // uniform
     // lane t owns a run of consecutive counts; the runs' sums are scanned across the work-group
@@ -176,20 +176,24 @@ __global__ __launch_bounds__(256) void k_collect_count(CollectArgs a) {
     unsigned run = before + x - own;
     for (int g = b; g < e; ++g) {
         const unsigned n = load_shared(&a.counts[g]);
-        a.counts[g] = run;
+        a.base[g] = run;
         run += n;
     }
-    if (threadIdx.x == 0) {
-        *a.total = all;
-        *a.arrived = 0u;
-    }
+    if (threadIdx.x == 0) *a.total = all;
 }
 // A wave per word of bits, 16 lanes per record, four records at a time.  kPack: the descriptors
 // alone, packed for the matcher, and each one's slot (record 0 as the zeros that CollectKeys
-// leaves there, slot -1); else whole records into `out`, where they are below `cap`.
+// leaves there, slot -1), and such zeros up to `cap`; else whole records into `out`.  Nothing is
+// written from `cap` on (an insert or a reset on another stream may have changed the number).
 template <bool kPack>
 __global__ __launch_bounds__(256) void k_collect_copy(CollectArgs a, Surf* out, float* desc, int* slot, unsigned cap) {
     const int word = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if constexpr (kPack) {
+        for (unsigned j = *a.total + blockIdx.x * 16 + threadIdx.x / 16; j < cap; j += gridDim.x * 16) {
+            reinterpret_cast<uint4*>(desc)[(size_t)j * 16 + threadIdx.x % 16] = make_uint4(0u, 0u, 0u, 0u);
+            if (threadIdx.x % 16 == 0) slot[j] = -1;
+        }
+    }
     if (word >= a.groups * kWords) return;  // uniform
     unsigned long long m = a.bits[word];
     if (!m) return;  // uniform
@@ -200,7 +204,7 @@ __global__ __launch_bounds__(256) void k_collect_copy(CollectArgs a, Surf* out, 
 #pragma unroll
     for (int d = 1; d < kWords; d <<= 1) before += __shfl_xor(before, d);
     before = (unsigned)__builtin_amdgcn_readfirstlane((int)before);
-    const unsigned j0 = a.counts[word / kWords] + before;
+    const unsigned j0 = a.base[word / kWords] + before;
     const int sub = lane >> 4, q = lane & 15, n = __popcll(m);
     for (int k = 0; k < sub; ++k) m &= m - 1;
     for (int r = sub; r < n; r += 4) {
@@ -209,10 +213,12 @@ __global__ __launch_bounds__(256) void k_collect_copy(CollectArgs a, Surf* out, 
         const uint4* src = reinterpret_cast<const uint4*>(&a.keys[i]);
         if constexpr (kPack) {
             static_assert(offsetof(Surf, desc) == 32, "two 16-byte words ahead of the descriptor");
-            uint4 v = src[2 + q];
-            if (j == 0) v = make_uint4(0u, 0u, 0u, 0u);
-            reinterpret_cast<uint4*>(desc)[(size_t)j * 16 + q] = v;
-            if (q == 0) slot[j] = j == 0 ? -1 : i;
+            if (j < cap) {
+                uint4 v = src[2 + q];
+                if (j == 0) v = make_uint4(0u, 0u, 0u, 0u);
+                reinterpret_cast<uint4*>(desc)[(size_t)j * 16 + q] = v;
+                if (q == 0) slot[j] = j == 0 ? -1 : i;
+            }
         } else if (j > 0 && j < cap) {
             uint4* dst = reinterpret_cast<uint4*>(&out[j]);
             dst[q] = src[q];
@@ -272,7 +278,7 @@ struct fu_keymap {
     KeyArgs a;
     unsigned* aux = nullptr;    // [0] keys left in a round, [1] collect total, [2] work-groups that
                                 // have counted, [3] valid keys, from [4] the slots' valid bits,
-                                // then group counts
+                                // then group counts and their prefix
     uint32_t n_valid = 0;       // aux[3] as of the last insert
     int dev = -1;               // the device the map was created on
     unsigned char* done = nullptr;  // per key of an insert call, grown on demand
@@ -307,11 +313,11 @@ extern "C" fu_status fu_keymap_destroy(fu_keymap* k) {
 
 static int n_slots(const fu_keymap* k) { return k->a.max_keys * k->a.nbuckets; }
 static int n_groups(const fu_keymap* k) { return (n_slots(k) + kCollect - 1) / kCollect; }
-static size_t aux_bytes(const fu_keymap* k) { return (4 + (size_t)n_groups(k) * (2 * kWords + 1)) * 4; }
+static size_t aux_bytes(const fu_keymap* k) { return (4 + (size_t)n_groups(k) * (2 * kWords + 2)) * 4; }
 static CollectArgs collect_args(const fu_keymap* k) {
     const int g = n_groups(k);
-    return CollectArgs{k->a.keys,  g,          k->a.bits + (size_t)g * (2 * kWords), k->aux + 1,
-                       k->aux + 2, (const unsigned long long*)k->a.bits};
+    unsigned* counts = k->a.bits + (size_t)g * (2 * kWords);
+    return CollectArgs{k->a.keys, g, counts, counts + g, k->aux + 1, k->aux + 2, (const unsigned long long*)k->a.bits};
 }
 
 extern "C" fu_status fu_keymap_create(const fu_keymap_params* p, fu_keymap** out) {
@@ -422,10 +428,10 @@ namespace fu {
 // the number of valid keys (an insert returns when its keys are in place)
 uint32_t keymap_count(const fu_keymap* k) { return k->n_valid; }
 // for its n keys: their descriptors (n x 64, 16-byte aligned) and slots, key 0 as zeros and slot -1
-fu_status keymap_pack(fu_keymap* k, float* desc, int32_t* slot, hipStream_t s) {
+fu_status keymap_pack(fu_keymap* k, float* desc, int32_t* slot, uint32_t n, hipStream_t s) {
     const CollectArgs a = collect_args(k);
     launch_count(a, s);
-    hipLaunchKernelGGL(k_collect_copy<true>, dim3(a.groups * (kCollect / 256)), dim3(256), 0, s, a, nullptr, desc, slot, 0u);
+    hipLaunchKernelGGL(k_collect_copy<true>, dim3(a.groups * (kCollect / 256)), dim3(256), 0, s, a, nullptr, desc, slot, n);
     KM_HIP(hipGetLastError());
     return FU_OK;
 }

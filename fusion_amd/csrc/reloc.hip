@@ -175,9 +175,8 @@ __global__ __launch_bounds__(256, 4) void k_match_bound(const float* q, int nq, 
                                                         float2* bound) {
     const int lane = threadIdx.x & 63, n = lane & 31, half = lane >> 5;
     // work-groups go to the eight XCDs in turn: each XCD takes every eighth chunk, all its queries
-    const int groups = (nq + 127) / 128, slot = blockIdx.x >> 3;
-    const int c = slot / groups * 8 + (blockIdx.x & 7);
-    const int q0 = (slot % groups * 4 + (threadIdx.x >> 6)) * 32;
+    const int c = blockIdx.y * 8 + (blockIdx.x & 7);
+    const int q0 = ((blockIdx.x >> 3) * 4 + (threadIdx.x >> 6)) * 32;
     const int c0 = c * chunk, c1 = min(nt, c0 + chunk);
     if (q0 >= nq || c0 >= nt) return;  // uniform
     auto fetch = [&](const float* base, int row, v4f (&x)[8]) {
@@ -928,8 +927,8 @@ extern "C" fu_status fu_match_knn2(const float* query, int32_t nq, const float* 
             (void)hipGetLastError();
             return api_error(FU_ERR_NOMEM, "fu_match_knn2: %d partial lists", nchunks);
         }
-        hipLaunchKernelGGL(k_match_bound, dim3((nq + 127) / 128 * ((nchunks + 7) / 8 * 8)), dim3(256), 0, hs, query, nq, train, nt, chunk,
-                           bound);
+        hipLaunchKernelGGL(k_match_bound, dim3((nq + 127) / 128 * 8, (nchunks + 7) / 8), dim3(256), 0, hs, query, nq, train, nt,
+                           chunk, bound);
     }
     hipLaunchKernelGGL(k_match_scan, dim3((nq + 3) / 4), dim3(256), 0, hs, query, nq, train, nt, chunk, nchunks, bound,
                        idx, dist);
@@ -1100,7 +1099,7 @@ fu_status collect_and_match(fu_keymap* km, const float* frame_desc, int32_t nq, 
                             float* dist, PairArgs& out, hipStream_t hs, const char* who) {
     const size_t desc = keys.part(sizeof(float) * kDesc * nk), slot = keys.part(sizeof(int32_t) * nk);
     if (!keys.allocate()) return api_error(FU_ERR_NOMEM, "%s: %u keys", who, nk);
-    fu_status st = keymap_pack(km, keys.at<float>(desc), keys.at<int32_t>(slot), hs);
+    fu_status st = keymap_pack(km, keys.at<float>(desc), keys.at<int32_t>(slot), nk, hs);
     if (st) return st;
     if ((st = fu_match_knn2(frame_desc, nq, keys.at<float>(desc), (int32_t)nk, idx, dist, (fu_stream)hs))) return st;
     out = PairArgs{idx, dist, nq, keys.at<int32_t>(slot), keymap_heads(km)};
