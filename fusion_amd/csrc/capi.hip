@@ -922,13 +922,12 @@ extern "C" fu_status fu_icp_step(const float* next_vmap, const float* last_vmap,
     launch_icp_step(icp_step_args(scratch->st, scratch->partials, next_vmap, last_vmap, next_nmap, last_nmap, cols, rows, fx,
                                   fy, cx, cy),
                     icp_groups(cols * rows), Rcurr, tcurr, Rlast, RlastInv, tlast, (float*)mail.dev, S(s));
-    const hipError_t le = hipGetLastError();
-    if (le != hipSuccess) {
-        mail.done();
-        return set_err(FU_ERR_HIP, "kernel launch: %s", hipGetErrorString(le));
-    }
-    HIPCHK(hipStreamSynchronize(S(s)));
-    mail.done();
+    // also after an error: it may be one that an earlier call of this thread left, with the launch
+    // under way, which writes the slot
+    const hipError_t le = hipGetLastError(), se = hipStreamSynchronize(S(s));
+    if (se == hipSuccess) mail.done();
+    if (le != hipSuccess) return set_err(FU_ERR_HIP, "kernel launch: %s", hipGetErrorString(le));
+    HIPCHK(se);
     icp_step_outputs((const float*)mail.host, residual, A, b);
     return FU_OK;
 }

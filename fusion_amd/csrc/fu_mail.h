@@ -22,7 +22,8 @@ public:
     Mail& operator=(const Mail&) = delete;
     void* host = nullptr;
     void* dev = nullptr;
-    // the stream is synchronised: nothing writes the slot any more, so it may be reused
+    // the stream is synchronised after the last launch that was given the slot (whether or not an
+    // error was seen since), or none was: nothing writes the slot any more, so it may be reused
     void done() { idle = true; }
 
 private:

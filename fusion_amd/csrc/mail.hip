@@ -55,17 +55,18 @@ int current_device() {
 hipError_t mail_read(int dev, void* dst0, const void* src0, size_t bytes0, void* dst1, const void* src1, size_t bytes1,
                      hipStream_t s) {
     Mail mail;
-    bool sent = mail.dev && bytes0 + bytes1 <= kMailBytes && !((bytes0 | bytes1) & 3) && dev == current_device();
-    if (sent) {
+    const bool post = mail.dev && bytes0 + bytes1 <= kMailBytes && !((bytes0 | bytes1) & 3) && dev == current_device();
+    bool sent = false;
+    if (post) {
         hipLaunchKernelGGL(k_mail, dim3(1), dim3(256), 0, s, (unsigned*)mail.dev, (const unsigned*)src0, (int)(bytes0 / 4),
                            (const unsigned*)src1, (int)(bytes1 / 4));
-        sent = hipGetLastError() == hipSuccess;
+        sent = hipGetLastError() == hipSuccess;  // or an error that an earlier call left
     }
     if (!sent) {
-        mail.done();  // nothing writes the slot
         hipError_t e = hipMemcpyAsync(dst0, src0, bytes0, hipMemcpyDeviceToHost, s);
         if (e == hipSuccess && bytes1) e = hipMemcpyAsync(dst1, src1, bytes1, hipMemcpyDeviceToHost, s);
         const hipError_t es = hipStreamSynchronize(s);
+        if (!post || es == hipSuccess) mail.done();
         return e == hipSuccess ? es : e;
     }
     const hipError_t e = hipStreamSynchronize(s);
