@@ -16,8 +16,24 @@ struct alignas(16) SurfHead {
     float normal[4];
 };
 
+// The scratch of one call's collection, from its launch until the call has waited for its stream;
+// `set` is null when there is no memory for it.
+class KeyScratch {
+public:
+    KeyScratch(fu_keymap* k, hipStream_t s);
+    ~KeyScratch();
+    KeyScratch(const KeyScratch&) = delete;
+    KeyScratch& operator=(const KeyScratch&) = delete;
+    void done() { waited = true; }  // the stream has been waited for
+    unsigned* set = nullptr;
+
+private:
+    fu_keymap* k;
+    hipStream_t stream;
+    bool waited = false;
+};
 uint32_t keymap_count(const fu_keymap* k);
-fu_status keymap_pack(fu_keymap* k, float* desc, int32_t* slot, uint32_t n, hipStream_t s);
+fu_status keymap_pack(fu_keymap* k, const KeyScratch& scratch, float* desc, int32_t* slot, uint32_t n, hipStream_t s);
 const SurfHead* keymap_heads(const fu_keymap* k);  // of the map's slots, kSlotHeads apart
 constexpr int kSlotHeads = sizeof(fu_surf) / sizeof(SurfHead);
 int keymap_device(const fu_keymap* k);

@@ -14,6 +14,9 @@
 #include <stddef.h>
 #include <string.h>
 
+#include <mutex>
+#include <vector>
+
 #include "fu_api.h"
 #include "fu_keys.h"
 #include "fu_mail.h"
@@ -138,9 +141,12 @@ __device__ __forceinline__ void store_shared(unsigned* p, unsigned v) {
 __device__ __forceinline__ unsigned load_shared(const unsigned* p) {
     return __hip_atomic_load(FU_G(const unsigned, p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__global__ __launch_bounds__(256) void k_collect_count(CollectArgs a) {
+// slot (with kPack below, else null): the `cap` slots of the copy that follows, all -1 until it writes them
+__global__ __launch_bounds__(256) void k_collect_count(CollectArgs a, int* slot, unsigned cap) {
     __shared__ unsigned wsum[4];
     __shared__ int last;
+    if (slot)
+        for (unsigned j = blockIdx.x * 256 + threadIdx.x; j < cap; j += gridDim.x * 256) slot[j] = -1;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int group = blockIdx.x * kCountGroups + threadIdx.x / kWords;
     unsigned c = group < a.groups ? (unsigned)__popcll(a.bits[blockIdx.x * 256 + threadIdx.x]) : 0u;
@@ -184,15 +190,15 @@ __global__ __launch_bounds__(256) void k_collect_count(CollectArgs a) {
 // A wave per word of bits, 16 lanes per record, four records at a time.  kPack: the descriptors
 // alone, packed for the matcher, and each one's slot (record 0 as the zeros that CollectKeys
 // leaves there, slot -1), and such zeros up to `cap`; else whole records into `out`.  Nothing is
-// written from `cap` on (an insert or a reset on another stream may have changed the number).
+// written from `cap` on and every slot is one of the map's or -1, whatever the bits: an insert or a
+// reset that runs beside the copy, which the caller has to rule out, may change what is found, but
+// nothing is read or written outside the arrays.
 template <bool kPack>
 __global__ __launch_bounds__(256) void k_collect_copy(CollectArgs a, Surf* out, float* desc, int* slot, unsigned cap) {
     const int word = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if constexpr (kPack) {
-        for (unsigned j = *a.total + blockIdx.x * 16 + threadIdx.x / 16; j < cap; j += gridDim.x * 16) {
+        for (unsigned j = *a.total + blockIdx.x * 16 + threadIdx.x / 16; j < cap; j += gridDim.x * 16)
             reinterpret_cast<uint4*>(desc)[(size_t)j * 16 + threadIdx.x % 16] = make_uint4(0u, 0u, 0u, 0u);
-            if (threadIdx.x % 16 == 0) slot[j] = -1;
-        }
     }
     if (word >= a.groups * kWords) return;  // uniform
     unsigned long long m = a.bits[word];
@@ -276,10 +282,11 @@ __global__ void k_adjacency(const SurfHead* frame, const SurfHead* map, int stri
 struct fu_keymap {
     fu_keymap_params p;
     KeyArgs a;
-    unsigned* aux = nullptr;    // [0] keys left in a round, [1] collect total, [2] work-groups that
-                                // have counted, [3] valid keys, from [4] the slots' valid bits,
-                                // then group counts and their prefix
-    uint32_t n_valid = 0;       // aux[3] as of the last insert
+    unsigned* aux = nullptr;    // [0] keys left in a round, [1] valid keys, from [4] the slots' valid bits
+    uint32_t n_valid = 0;       // aux[1] as of the last insert
+    // scratch of the collections (KeyScratch): the sets that no call uses, and all there are
+    std::mutex lock;
+    std::vector<unsigned*> idle, sets;
     int dev = -1;               // the device the map was created on
     unsigned char* done = nullptr;  // per key of an insert call, grown on demand
     int* bucket = nullptr;
@@ -307,17 +314,66 @@ extern "C" fu_status fu_keymap_destroy(fu_keymap* k) {
     (void)hipFree(k->aux);
     (void)hipFree(k->done);
     (void)hipFree(k->bucket);
+    for (unsigned* set : k->sets) (void)hipFree(set);
     delete k;
     return FU_OK;
 }
 
 static int n_slots(const fu_keymap* k) { return k->a.max_keys * k->a.nbuckets; }
 static int n_groups(const fu_keymap* k) { return (n_slots(k) + kCollect - 1) / kCollect; }
-static size_t aux_bytes(const fu_keymap* k) { return (4 + (size_t)n_groups(k) * (2 * kWords + 2)) * 4; }
-static CollectArgs collect_args(const fu_keymap* k) {
+static size_t aux_bytes(const fu_keymap* k) { return (4 + (size_t)n_groups(k) * (2 * kWords)) * 4; }
+
+// A set: total, arrived, the groups' counts and their prefix.  One is made with the map, so that
+// calls that follow one another never allocate; a further one for each call that runs beside others,
+// on a stream or thread of its own (sharing one, the arrivals of two calls mixed, and a prefix was
+// made of counts that were not all in place).
+constexpr size_t kIdleSets = 16;
+static unsigned* make_set(fu_keymap* k) {
+    unsigned* set = nullptr;
+    const size_t bytes = (2 + 2 * (size_t)n_groups(k)) * 4;
+    // cleared before any stream may use it
+    if (hipMalloc(&set, bytes) == hipSuccess && hipMemset(set, 0, bytes) == hipSuccess &&
+        hipStreamSynchronize(nullptr) == hipSuccess) {
+        std::lock_guard<std::mutex> g(k->lock);
+        k->sets.push_back(set);
+        return set;
+    }
+    (void)hipGetLastError();
+    (void)hipFree(set);
+    return nullptr;
+}
+fu::KeyScratch::KeyScratch(fu_keymap* km, hipStream_t s) : k(km), stream(s) {
+    {
+        std::lock_guard<std::mutex> g(k->lock);
+        if (!k->idle.empty()) {
+            set = k->idle.back();
+            k->idle.pop_back();
+            return;
+        }
+    }
+    set = make_set(k);
+}
+fu::KeyScratch::~KeyScratch() {
+    // a set that kernels may still write is not used again (it is freed with the map)
+    if (!set || (!waited && hipStreamSynchronize(stream) != hipSuccess)) return;
+    {
+        std::lock_guard<std::mutex> g(k->lock);
+        if (k->idle.size() < kIdleSets) {
+            k->idle.push_back(set);
+            return;
+        }
+        for (unsigned*& x : k->sets)
+            if (x == set) {
+                x = k->sets.back();
+                k->sets.pop_back();
+                break;
+            }
+    }
+    (void)hipFree(set);
+}
+static CollectArgs collect_args(const fu_keymap* k, unsigned* set) {
     const int g = n_groups(k);
-    unsigned* counts = k->a.bits + (size_t)g * (2 * kWords);
-    return CollectArgs{k->a.keys, g, counts, counts + g, k->aux + 1, k->aux + 2, (const unsigned long long*)k->a.bits};
+    return CollectArgs{k->a.keys, g, set + 2, set + 2 + g, set, set + 1, (const unsigned long long*)k->a.bits};
 }
 
 extern "C" fu_status fu_keymap_create(const fu_keymap_params* p, fu_keymap** out) {
@@ -334,16 +390,17 @@ extern "C" fu_status fu_keymap_create(const fu_keymap_params* p, fu_keymap** out
     const size_t n = (size_t)n_slots(k);
     if (hipMalloc(&k->a.keys, n * sizeof(Surf)) != hipSuccess || hipMalloc(&k->a.mutex, n * 4) != hipSuccess ||
         hipMalloc(&k->a.owner, (size_t)p->max_keys * 4) != hipSuccess ||
-        hipMalloc(&k->aux, aux_bytes(k)) != hipSuccess) {
+        hipMalloc(&k->aux, aux_bytes(k)) != hipSuccess || !make_set(k)) {
         (void)hipGetLastError();
         fu_keymap_destroy(k);
         return api_error(FU_ERR_NOMEM, "fu_keymap_create: allocation failed");
     }
+    k->idle = k->sets;
     // records start zeroed (ResetKeys clears only the valid flags, so a record's other bytes
     // keep what the last key there left)
     k->dev = current_device();
     k->a.bits = k->aux + 4;
-    k->a.valid = k->aux + 3;
+    k->a.valid = k->aux + 1;
     if (hipMemset(k->a.keys, 0, n * sizeof(Surf)) != hipSuccess || hipMemset(k->aux, 0, aux_bytes(k)) != hipSuccess) {
         (void)hipGetLastError();
         fu_keymap_destroy(k);
@@ -398,39 +455,43 @@ extern "C" fu_status fu_insert_key_points(fu_keymap* k, fu_surf* keys, int32_t* 
         hipLaunchKernelGGL(k_insert_apply, grid, dim3(256), 0, hs, k->a, (Surf*)keys, index, k->done, k->bucket, (int)n,
                            k->aux);
         KM_HIP(hipGetLastError());
-        unsigned aux[4] = {};
+        unsigned aux[2] = {};
         KM_HIP(hipMemcpyAsync(aux, k->aux, sizeof(aux), hipMemcpyDeviceToHost, hs));
         KM_HIP(hipStreamSynchronize(hs));
-        k->n_valid = aux[3];
+        k->n_valid = aux[1];
         if (aux[0] == 0) return FU_OK;
     }
     return api_error(FU_ERR_STATE, "fu_insert_key_points: inserts did not finish");
 }
 
-static void launch_count(const CollectArgs& a, hipStream_t s) {
-    hipLaunchKernelGGL(k_collect_count, dim3((a.groups + kCountGroups - 1) / kCountGroups), dim3(256), 0, s, a);
+static void launch_count(const CollectArgs& a, int* slot, unsigned cap, hipStream_t s) {
+    hipLaunchKernelGGL(k_collect_count, dim3((a.groups + kCountGroups - 1) / kCountGroups), dim3(256), 0, s, a, slot, cap);
 }
 
 extern "C" fu_status fu_collect_key_points(fu_keymap* k, fu_surf* out, uint32_t cap, uint32_t* n_keys, fu_stream s) {
     if (!k || !n_keys || (cap && !out)) return api_error(FU_ERR_ARG, "fu_collect_key_points: null argument");
     hipStream_t hs = (hipStream_t)s;
-    const CollectArgs a = collect_args(k);
-    launch_count(a, hs);
+    KeyScratch scratch(k, hs);
+    if (!scratch.set) return api_error(FU_ERR_NOMEM, "fu_collect_key_points: scratch allocation failed");
+    const CollectArgs a = collect_args(k, scratch.set);
+    launch_count(a, nullptr, 0, hs);
     if (cap)
         hipLaunchKernelGGL(k_collect_copy<false>, dim3(a.groups * (kCollect / 256)), dim3(256), 0, hs, a, (Surf*)out,
                            nullptr, nullptr, cap);
     KM_HIP(hipGetLastError());
     KM_HIP(mail_read(k->dev, n_keys, a.total, 4, hs));
+    scratch.done();
     return FU_OK;
 }
 
 namespace fu {
 // the number of valid keys (an insert returns when its keys are in place)
 uint32_t keymap_count(const fu_keymap* k) { return k->n_valid; }
-// for its n keys: their descriptors (n x 64, 16-byte aligned) and slots, key 0 as zeros and slot -1
-fu_status keymap_pack(fu_keymap* k, float* desc, int32_t* slot, uint32_t n, hipStream_t s) {
-    const CollectArgs a = collect_args(k);
-    launch_count(a, s);
+// for n of its keys: their descriptors (n x 64, 16-byte aligned) and slots, key 0 as zeros and slot -1
+fu_status keymap_pack(fu_keymap* k, const KeyScratch& scratch, float* desc, int32_t* slot, uint32_t n, hipStream_t s) {
+    if (!scratch.set) return api_error(FU_ERR_NOMEM, "key map: scratch allocation failed");
+    const CollectArgs a = collect_args(k, scratch.set);
+    launch_count(a, slot, n, s);
     hipLaunchKernelGGL(k_collect_copy<true>, dim3(a.groups * (kCollect / 256)), dim3(256), 0, s, a, nullptr, desc, slot, n);
     KM_HIP(hipGetLastError());
     return FU_OK;

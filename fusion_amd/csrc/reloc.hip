@@ -1095,11 +1095,11 @@ __global__ __launch_bounds__(1024) void k_list_points(ListPoints p, int* counts,
 // CollectKeyPoints and reads as zeros here) and the two nearest of them to each frame descriptor,
 // on the device.  `out`: idx and dist, 2 per query (-1 / +inf where the map has fewer keys), and the
 // keys' slots, which live in `keys`.
-fu_status collect_and_match(fu_keymap* km, const float* frame_desc, int32_t nq, uint32_t nk, Block& keys, int32_t* idx,
-                            float* dist, PairArgs& out, hipStream_t hs, const char* who) {
+fu_status collect_and_match(fu_keymap* km, const KeyScratch& scratch, const float* frame_desc, int32_t nq, uint32_t nk,
+                            Block& keys, int32_t* idx, float* dist, PairArgs& out, hipStream_t hs, const char* who) {
     const size_t desc = keys.part(sizeof(float) * kDesc * nk), slot = keys.part(sizeof(int32_t) * nk);
     if (!keys.allocate()) return api_error(FU_ERR_NOMEM, "%s: %u keys", who, nk);
-    fu_status st = keymap_pack(km, keys.at<float>(desc), keys.at<int32_t>(slot), nk, hs);
+    fu_status st = keymap_pack(km, scratch, keys.at<float>(desc), keys.at<int32_t>(slot), nk, hs);
     if (st) return st;
     if ((st = fu_match_knn2(frame_desc, nq, keys.at<float>(desc), (int32_t)nk, idx, dist, (fu_stream)hs))) return st;
     out = PairArgs{idx, dist, nq, keys.at<int32_t>(slot), keymap_heads(km)};
@@ -1163,6 +1163,7 @@ extern "C" fu_status fu_relocalise_keys(fu_keymap* km, const float* frame_desc, 
     const uint32_t nk = keymap_count(km);
     fu_status st = FU_OK;
     if (nk == 0 || nq == 0) return FU_OK;  // no map keys (Tracking.cc:417-418)
+    KeyScratch scratch(km, hs);
     const int draws = std::max(0, std::min(iterations, kFirstDraws));
     Block keys(hs), work(hs);
     const size_t fpos = work.part(sizeof(double) * 3 * nq), idx = work.part(sizeof(int32_t) * 2 * nq),
@@ -1170,7 +1171,7 @@ extern "C" fu_status fu_relocalise_keys(fu_keymap* km, const float* frame_desc, 
                  pairs = work.part(sizeof(RatioPair) * nq);
     if (!work.allocate()) return api_error(FU_ERR_NOMEM, "fu_relocalise_keys: %d keypoints", nq);
     PairArgs pa{};
-    if ((st = collect_and_match(km, frame_desc, nq, nk, keys, work.at<int32_t>(idx), work.at<float>(dist), pa, hs,
+    if ((st = collect_and_match(km, scratch, frame_desc, nq, nk, keys, work.at<int32_t>(idx), work.at<float>(dist), pa, hs,
                                 "fu_relocalise_keys")))
         return st;
     hipError_t e = hipMemcpyAsync(work.at<double>(fpos), frame_pos, sizeof(double) * 3 * nq, hipMemcpyHostToDevice, hs);
@@ -1189,6 +1190,7 @@ extern "C" fu_status fu_relocalise_keys(fu_keymap* km, const float* frame_desc, 
     const int dev = keymap_device(km);
     // also after a failure: nothing queued may still read the caller's memory
     const hipError_t er = mail_read(dev, hhead.data(), dhead, hbytes, hp.data(), dpairs, sizeof(RatioPair) * first, hs);
+    if (er == hipSuccess) scratch.done();
     if (e == hipSuccess) e = er;
     const int np = e == hipSuccess ? hhead[0] : 0;
     if (np > first) {
@@ -1263,6 +1265,7 @@ extern "C" fu_status fu_relocalise_graph_candidates(fu_keymap* km, const float* 
     const uint32_t nk = keymap_count(km);
     fu_status st = FU_OK;
     if (nk == 0 || nq == 0) return FU_OK;  // no map keys (Tracking.cc:417-418)
+    KeyScratch scratch(km, hs);
     const int dev = keymap_device(km);
     Block keys(hs), work(hs), graph(hs);
     const size_t nm = 2 * (size_t)nq;
@@ -1272,7 +1275,7 @@ extern "C" fu_status fu_relocalise_graph_candidates(fu_keymap* km, const float* 
                  dd = work.part(sizeof(float) * nm), cnt = work.part(sizeof(int) * 2);
     if (!work.allocate()) return api_error(FU_ERR_NOMEM, "%s: %d keypoints", who, nq);
     PairArgs pa{};
-    if ((st = collect_and_match(km, frame_desc, nq, nk, keys, work.at<int32_t>(idx), work.at<float>(dist), pa, hs, who)))
+    if ((st = collect_and_match(km, scratch, frame_desc, nq, nk, keys, work.at<int32_t>(idx), work.at<float>(dist), pa, hs, who)))
         return st;
     hipError_t e = hipMemcpyAsync(work.at<float>(fpos), frame_pos, sizeof(float) * 3 * nq, hipMemcpyHostToDevice, hs);
     if (e == hipSuccess)
@@ -1284,6 +1287,7 @@ extern "C" fu_status fu_relocalise_graph_candidates(fu_keymap* km, const float* 
     int counted[2] = {0, 0};
     // also after a failure: nothing queued may still read the caller's memory
     const hipError_t er = mail_read(dev, counted, work.at<int>(cnt), sizeof(counted), hs);
+    if (er == hipSuccess) scratch.done();
     if (e == hipSuccess) e = er;
     if (e != hipSuccess) return api_error(FU_ERR_HIP, "%s: %s", who, hipGetErrorString(e));
     if (n_pairs) *n_pairs = counted[0];

@@ -357,7 +357,9 @@ typedef struct fu_surf {
 } fu_surf;
 typedef struct fu_keymap fu_keymap;
 /* KeyMap's constants (DeviceMap.h:163-170) as parameters: grid cell 0.01 m, 100000 buckets
- * of 5 slots */
+ * of 5 slots.  Calls that read a key map (collect, read, relocalise) may run side by side on
+ * streams and threads of their own; an insert or a reset changes the map and must be ordered
+ * with every other call of it by the caller. */
 typedef struct fu_keymap_params {
     float grid_size;
     uint32_t max_keys;
