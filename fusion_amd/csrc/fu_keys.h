@@ -32,7 +32,7 @@ private:
     hipStream_t stream;
     bool waited = false;
 };
-uint32_t keymap_count(const fu_keymap* k);
+fu_status keymap_count(const fu_keymap* k, uint32_t& n, hipStream_t s);
 fu_status keymap_pack(fu_keymap* k, const KeyScratch& scratch, float* desc, int32_t* slot, uint32_t n, hipStream_t s);
 const SurfHead* keymap_heads(const fu_keymap* k);  // of the map's slots, kSlotHeads apart
 constexpr int kSlotHeads = sizeof(fu_surf) / sizeof(SurfHead);

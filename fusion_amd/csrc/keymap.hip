@@ -14,6 +14,7 @@
 #include <stddef.h>
 #include <string.h>
 
+#include <atomic>
 #include <mutex>
 #include <vector>
 
@@ -283,7 +284,8 @@ struct fu_keymap {
     fu_keymap_params p;
     KeyArgs a;
     unsigned* aux = nullptr;    // [0] keys left in a round, [1] valid keys, from [4] the slots' valid bits
-    uint32_t n_valid = 0;       // aux[1] as of the last insert
+    // aux[1] as of the last insert or reset call, kUnknown while an insert runs and after one failed
+    std::atomic<long long> n_valid{0};
     // scratch of the collections (KeyScratch): the sets that no call uses, and all there are
     std::mutex lock;
     std::vector<unsigned*> idle, sets;
@@ -322,6 +324,7 @@ extern "C" fu_status fu_keymap_destroy(fu_keymap* k) {
 static int n_slots(const fu_keymap* k) { return k->a.max_keys * k->a.nbuckets; }
 static int n_groups(const fu_keymap* k) { return (n_slots(k) + kCollect - 1) / kCollect; }
 static size_t aux_bytes(const fu_keymap* k) { return (4 + (size_t)n_groups(k) * (2 * kWords)) * 4; }
+constexpr long long kUnknown = -1;
 
 // A set: total, arrived, the groups' counts and their prefix.  One is made with the map, so that
 // calls that follow one another never allocate; a further one for each call that runs beside others,
@@ -422,9 +425,10 @@ extern "C" fu_status fu_keymap_create(const fu_keymap_params* p, fu_keymap** out
 extern "C" fu_status fu_reset_key_points(fu_keymap* k, fu_stream s) {
     if (!k) return api_error(FU_ERR_ARG, "fu_reset_key_points: null key map");
     const int n = n_slots(k);
-    k->n_valid = 0;
+    k->n_valid = kUnknown;
     hipLaunchKernelGGL(k_reset_keys, dim3((n + 255) / 256), dim3(256), 0, (hipStream_t)s, k->a, n);
     KM_HIP(hipGetLastError());
+    k->n_valid = 0;
     return FU_OK;
 }
 
@@ -446,6 +450,7 @@ extern "C" fu_status fu_insert_key_points(fu_keymap* k, fu_surf* keys, int32_t* 
         }
         k->cap = (int)n;
     }
+    k->n_valid = kUnknown;
     KM_HIP(hipMemsetAsync(k->done, 0, n, hs));
     const dim3 grid((n + 255) / 256);
     // rounds until every key is placed; each round places at least the lowest waiting index
@@ -458,8 +463,10 @@ extern "C" fu_status fu_insert_key_points(fu_keymap* k, fu_surf* keys, int32_t* 
         unsigned aux[2] = {};
         KM_HIP(hipMemcpyAsync(aux, k->aux, sizeof(aux), hipMemcpyDeviceToHost, hs));
         KM_HIP(hipStreamSynchronize(hs));
-        k->n_valid = aux[1];
-        if (aux[0] == 0) return FU_OK;
+        if (aux[0] == 0) {
+            k->n_valid = aux[1];
+            return FU_OK;
+        }
     }
     return api_error(FU_ERR_STATE, "fu_insert_key_points: inserts did not finish");
 }
@@ -485,8 +492,14 @@ extern "C" fu_status fu_collect_key_points(fu_keymap* k, fu_surf* out, uint32_t 
 }
 
 namespace fu {
-// the number of valid keys (an insert returns when its keys are in place)
-uint32_t keymap_count(const fu_keymap* k) { return k->n_valid; }
+// the number of valid keys: as the host knows it (an insert returns when its keys are in place), else
+// from the device
+fu_status keymap_count(const fu_keymap* k, uint32_t& n, hipStream_t s) {
+    const long long known = k->n_valid;
+    n = (uint32_t)known;
+    if (known == kUnknown) KM_HIP(mail_read(k->dev, &n, k->a.valid, 4, s));
+    return FU_OK;
+}
 // for n of its keys: their descriptors (n x 64, 16-byte aligned) and slots, key 0 as zeros and slot -1
 fu_status keymap_pack(fu_keymap* k, const KeyScratch& scratch, float* desc, int32_t* slot, uint32_t n, hipStream_t s) {
     if (!scratch.set) return api_error(FU_ERR_NOMEM, "key map: scratch allocation failed");

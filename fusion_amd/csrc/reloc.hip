@@ -1160,8 +1160,9 @@ extern "C" fu_status fu_relocalise_keys(fu_keymap* km, const float* frame_desc, 
     if (n_pairs) *n_pairs = 0;
     for (int k = 0; k < 16; ++k) pose[k] = (k % 5 == 0) ? 1.0 : 0.0;
     hipStream_t hs = (hipStream_t)s;
-    const uint32_t nk = keymap_count(km);
-    fu_status st = FU_OK;
+    uint32_t nk = 0;
+    fu_status st = keymap_count(km, nk, hs);
+    if (st) return st;
     if (nk == 0 || nq == 0) return FU_OK;  // no map keys (Tracking.cc:417-418)
     KeyScratch scratch(km, hs);
     const int draws = std::max(0, std::min(iterations, kFirstDraws));
@@ -1262,8 +1263,9 @@ extern "C" fu_status fu_relocalise_graph_candidates(fu_keymap* km, const float* 
     if (n_pairs) *n_pairs = 0;
     const char* who = "fu_relocalise_graph_candidates";
     hipStream_t hs = (hipStream_t)s;
-    const uint32_t nk = keymap_count(km);
-    fu_status st = FU_OK;
+    uint32_t nk = 0;
+    fu_status st = keymap_count(km, nk, hs);
+    if (st) return st;
     if (nk == 0 || nq == 0) return FU_OK;  // no map keys (Tracking.cc:417-418)
     KeyScratch scratch(km, hs);
     const int dev = keymap_device(km);

@@ -359,7 +359,8 @@ typedef struct fu_keymap fu_keymap;
 /* KeyMap's constants (DeviceMap.h:163-170) as parameters: grid cell 0.01 m, 100000 buckets
  * of 5 slots.  Calls that read a key map (collect, read, relocalise) may run side by side on
  * streams and threads of their own; an insert or a reset changes the map and must be ordered
- * with every other call of it by the caller. */
+ * with every other call of it by the caller: an insert has taken effect when it returns, a
+ * reset in its stream's order, though relocalisations find no keys from its return on. */
 typedef struct fu_keymap_params {
     float grid_size;
     uint32_t max_keys;

@@ -69,3 +69,36 @@ def test_reads_side_by_side(gpu, max_keys, n_buckets):
                 else:
                     assert b == len(want) and a[1 : len(want)].tobytes() == want[1:].tobytes()
     km.close()
+
+
+def test_number_of_keys_after_a_failed_insert(gpu):
+    """an insert that fails part way (here refused by its stream, which is being captured) leaves the
+    number of keys to be read from the device"""
+    import ctypes as C
+
+    from fusion_amd import native as N
+    from tests.test_gpu_results import _hip
+
+    rng = np.random.default_rng(4)
+    km = A.KeyMap(max_keys=997, n_buckets=5)
+    keys = _keys(rng, 300)
+    km.InsertKeyPoints(A.surf_to_device(keys), torch.full((300,), -1, dtype=torch.int32, device="cuda"))
+    slots = km.read()
+    want = slots[slots["valid"] != 0]
+    desc = torch.from_numpy(want["descriptor"][1:] + np.float32(0.01)).cuda()
+    cam = want["pos"][1:].astype(np.float64) + 0.25
+    pose, pairs = km.relocalise(desc, cam, iterations=40, seed=3)
+    more, index = A.surf_to_device(_keys(rng, 50)), torch.full((50,), -1, dtype=torch.int32, device="cuda")
+    hip, s, graph = _hip(), torch.cuda.Stream(), C.c_void_p()
+    torch.cuda.synchronize()
+    stream = C.c_void_p(s.cuda_stream)
+    assert hip.hipStreamBeginCapture(stream, 2) == 0
+    st = N.lib().fu_insert_key_points(km.handle, C.c_void_p(more.data_ptr()), C.c_void_p(index.data_ptr()), 50, stream)
+    end = hip.hipStreamEndCapture(stream, C.byref(graph))
+    hip.hipGetLastError()
+    assert st != 0 and (end != 0 or not graph.value)
+    again, n = km.relocalise(desc, cam, iterations=40, seed=3)
+    assert pose is not None and np.array_equal(again, pose) and n == pairs == len(want) - 1
+    km.InsertKeyPoints(more, index)
+    assert km.CollectKeyPoints(4)[1] == int((km.read()["valid"] != 0).sum()) == len(want) + int((index >= 0).sum())
+    km.close()
