@@ -2164,9 +2164,10 @@ struct fu_icp_batch {
     int cap = 0;
     SessDesc* d_desc = nullptr;
     std::vector<SessDesc> h_desc;
-    int ran = 0;                 // pairs of the last call
+    int ran = 0;                  // pairs of the last call
     TrackState* h_res = nullptr;  // pinned: their states (fu_icp_batch_results), cap of them
-    void* d_res = nullptr;       // its device address
+    void* d_res = nullptr;        // its device address
+    hipEvent_t written = nullptr;  // the last call has written them
 };
 
 extern "C" fu_status fu_icp_batch_create(int capacity, fu_icp_batch** out) {
@@ -2181,38 +2182,46 @@ extern "C" fu_status fu_icp_batch_create(int capacity, fu_icp_batch** out) {
         delete b;
         return set_err(FU_ERR_NOMEM, "descriptor allocation failed");
     }
+    if (hipEventCreateWithFlags(&b->written, hipEventDisableTiming) != hipSuccess) {
+        (void)hipGetLastError();
+        (void)hipFree(b->d_desc);
+        delete b;
+        return set_err(FU_ERR_HIP, "event creation failed");
+    }
     *out = b;
     return FU_OK;
 }
 
 extern "C" fu_status fu_icp_batch_destroy(fu_icp_batch* b) {
     if (!b) return FU_OK;
+    if (b->ran) (void)hipEventSynchronize(b->written);
+    (void)hipEventDestroy(b->written);
     (void)hipFree(b->d_desc);
     if (b->h_res) (void)hipHostFree(b->h_res);
     delete b;
     return FU_OK;
 }
 
-// the results of every tracker of the last fu_compute_se3_batch call: their states gathered into
-// pinned memory by one launch, one synchronisation for all of them
-extern "C" fu_status fu_icp_batch_results(fu_icp_batch* b, int n, fu_track_result* out, fu_stream s) {
+// The pairs' states are gathered into pinned memory by one launch at the end of the call that made
+// them, on its stream, while its trackers are there; the results wait for that launch.  Null after
+// a failure: the results are then refused.
+static TrackState* batch_results(fu_icp_batch* b) {
+    if (b->h_res) return b->h_res;
+    void* p = nullptr;
+    if (hipHostMalloc(&p, sizeof(TrackState) * b->cap, hipHostMallocMapped) != hipSuccess ||
+        hipHostGetDevicePointer(&b->d_res, p, 0) != hipSuccess) {
+        (void)hipGetLastError();
+        if (p) (void)hipHostFree(p);
+        return nullptr;
+    }
+    return b->h_res = (TrackState*)p;
+}
+
+extern "C" fu_status fu_icp_batch_results(fu_icp_batch* b, int n, fu_track_result* out, fu_stream) {
     if (!b || !out) return set_err(FU_ERR_ARG, "fu_icp_batch_results: null argument");
     if (n < 1 || n != b->ran) return set_err(FU_ERR_STATE, "fu_icp_batch_results: %d results of a call with %d pairs", n, b->ran);
-    if (!b->h_res) {
-        void* p = nullptr;
-        if (hipHostMalloc(&p, sizeof(TrackState) * b->cap, hipHostMallocMapped) != hipSuccess) {
-            (void)hipGetLastError();
-            return set_err(FU_ERR_NOMEM, "fu_icp_batch_results: pinned memory");
-        }
-        if (hipHostGetDevicePointer(&b->d_res, p, 0) != hipSuccess) {
-            (void)hipHostFree(p);
-            return set_err(FU_ERR_HIP, "fu_icp_batch_results: pinned memory is not mapped");
-        }
-        b->h_res = (TrackState*)p;
-    }
-    launch_states(b->d_desc, n, b->d_res, S(s));
-    LAUNCHCHK();
-    HIPCHK(hipStreamSynchronize(S(s)));
+    if (!b->h_res) return set_err(FU_ERR_NOMEM, "fu_icp_batch_results: pinned memory");
+    HIPCHK(hipEventSynchronize(b->written));
     for (int i = 0; i < n; ++i) fill_result(b->h_res[i], &out[i]);
     return FU_OK;
 }
@@ -2269,7 +2278,9 @@ extern "C" fu_status fu_compute_se3_batch(fu_icp_batch* ib, int n, fu_tracker* c
         for (int l = 2; l >= 0; --l)
             for (int j = 0; j < iters[l]; ++j) launch_b_icp(b, h, l, j, hs);
     }
+    if (batch_results(ib)) launch_states(ib->d_desc, n, ib->d_res, hs);
     LAUNCHCHK();
+    HIPCHK(hipEventRecord(ib->written, hs));
     ib->ran = n;
     return FU_OK;
 }

@@ -566,7 +566,8 @@ fu_status fu_compute_se3_batch(fu_icp_batch* b, int n, fu_tracker* const* tracke
                                const float* const* last_vmap, const float* const* last_nmap, const float* K,
                                const int32_t iters[3], const int32_t min_count[3], float thresh, fu_stream s);
 /* fu_tracker_result of every tracker of the handle's last fu_compute_se3_batch call (n pairs), in
- * their order, with one synchronisation of `s` */
+ * their order, as that call left them: waits for it alone, whatever `s`, and reads no tracker
+ * (they may be in use again or destroyed).  A handle takes one call at a time. */
 fu_status fu_icp_batch_results(fu_icp_batch* b, int n, fu_track_result* out, fu_stream s);
 
 /* ---- batched frames of many systems -------------------------------------------------------
