@@ -214,7 +214,10 @@ __device__ __forceinline__ void alloc_a_body(WG g, const MapView& m, const FuseA
             }
             if (!done) {
                 const i3 b = unpack(o);
-                if (key_in_range(b)) claim_block(m, true, pack_key(b), b);
+                if (key_in_range(b))
+                    claim_block(m, true, pack_key(b), b);
+                else
+                    atomicOr(&m.ctr[C_FLAGS], (unsigned)FLAG_COORD_RANGE);
             }
         }
     }

@@ -54,3 +54,20 @@ def test_key_range_is_flagged(gpu, blocks_from_limit):
     g.FuseMapColor(d, torch.zeros((16, 16, 3), dtype=torch.uint8, device="cuda"),
                    torch.full((16, 16, 4), float("nan"), device="cuda"), pose, (20.0, 20.0, 8.0, 8.0))
     assert g.stats()["flags"] & 8 and g.stats()["n_allocated"] == 0
+
+
+def test_key_range_is_flagged_by_rays_past_a_full_set(gpu):
+    """rays spread over a block each per pixel and fourteen in depth fill the tile's set before any of
+    them leaves the key range, so every block past it is one that found no slot"""
+    voxel, n = 0.01, 16
+    d = torch.full((n, n), 1.1, dtype=torch.float32, device="cuda")
+    pose = np.eye(4)
+    pose[2, 3] = (1 << 20) * 8 * voxel - 1.6
+    g = A.Mapping(num_buckets=1 << 14, num_excess=1 << 13, num_blocks=1 << 14, voxel_size=voxel, trunc_dist=1.2,
+                  max_new_blocks=1 << 14)
+    print("alloc: full set at the key range's end", flush=True)
+    g.FuseMapColor(d, torch.zeros((n, n, 3), dtype=torch.uint8, device="cuda"),
+                   torch.full((n, n, 4), float("nan"), device="cuda"), pose, (10.0, 10.0, 7.5, 7.5))
+    z = g.export_blocks()[:, 2]
+    assert len(z) > 2000 and z.min() < (1 << 20) - 13 and z.max() == (1 << 20) - 1
+    assert g.stats()["flags"] == 8
