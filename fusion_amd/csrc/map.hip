@@ -159,13 +159,15 @@ __device__ __forceinline__ void alloc_a_body(WG g, const MapView& m, const FuseA
             nsteps = d2i(ceil(2.0 * (double)len));
             dir = divs(dir, (float)(nsteps - 1));
             pt = a;
-            // steps lie between the ends, but for rounding far below a block
+            // steps lie between the ends but for their rounding: 2^-24 of the largest coordinate each,
+            // 80 voxels in all, where the margins below are 96
+            const float far = fmaxf(fmaxf(fmaxf(fabsf(a.x), fabsf(a.y)), fmaxf(fabsf(a.z), fabsf(b.x))), fmaxf(fabsf(b.y), fabsf(b.z)));
             auto inside = [&](f3 q) {
                 const i3 c = voxel_to_block(f2i3(q));
                 return (unsigned)(c.x - base.x - 12) < 1000u && (unsigned)(c.y - base.y - 12) < 1000u &&
                        (unsigned)(c.z - base.z - 12) < 1000u;
             };
-            near = inside(a) && inside(b);
+            near = inside(a) && inside(b) && (float)nsteps * far <= 80.0f * 0x1p24f;
         }
     }
     if (!near) {

@@ -57,17 +57,33 @@ def test_key_range_is_flagged(gpu, blocks_from_limit):
 
 
 def test_key_range_is_flagged_by_rays_past_a_full_set(gpu):
-    """rays spread over a block each per pixel and fourteen in depth fill the tile's set before any of
-    them leaves the key range, so every block past it is one that found no slot"""
+    """rays spread over a block each per pixel and ten in depth fill the tile's set before any of them
+    leaves the key range, so every block past it is one that found no slot"""
     voxel, n = 0.01, 16
-    d = torch.full((n, n), 1.1, dtype=torch.float32, device="cuda")
+    d = torch.full((n, n), 2.5, dtype=torch.float32, device="cuda")
     pose = np.eye(4)
-    pose[2, 3] = (1 << 20) * 8 * voxel - 1.6
-    g = A.Mapping(num_buckets=1 << 14, num_excess=1 << 13, num_blocks=1 << 14, voxel_size=voxel, trunc_dist=1.2,
+    pose[2, 3] = (1 << 20) * 8 * voxel - 2.8
+    g = A.Mapping(num_buckets=1 << 14, num_excess=1 << 13, num_blocks=1 << 14, voxel_size=voxel, trunc_dist=0.72,
                   max_new_blocks=1 << 14)
     print("alloc: full set at the key range's end", flush=True)
     g.FuseMapColor(d, torch.zeros((n, n, 3), dtype=torch.uint8, device="cuda"),
-                   torch.full((n, n, 4), float("nan"), device="cuda"), pose, (10.0, 10.0, 7.5, 7.5))
+                   torch.full((n, n, 4), float("nan"), device="cuda"), pose, (25.0, 25.0, 7.5, 7.5))
     z = g.export_blocks()[:, 2]
-    assert len(z) > 2000 and z.min() < (1 << 20) - 13 and z.max() == (1 << 20) - 1
+    assert len(z) > 2000 and z.min() < (1 << 20) - 8 and z.max() == (1 << 20) - 1
     assert g.stats()["flags"] == 8
+
+
+def test_rays_where_a_step_rounds_up(gpu):
+    """past 2^23 voxels a march's step of just over half a voxel rounds to a whole one, so the ray ends
+    as far again behind its band, beyond the offsets' range; it takes no block of the key range"""
+    voxel = 0.01
+    pose = np.eye(4)
+    pose[:3, :3] = [[0, 0, 1], [0, 1, 0], [-1, 0, 0]]  # looking along x
+    pose[0, 3] = ((1 << 20) - 470) * 8 * voxel
+    g = A.Mapping(num_buckets=1 << 10, num_excess=1 << 10, num_blocks=1 << 10, voxel_size=voxel, trunc_dist=2.24,
+                  depth_max=50.0, max_new_blocks=1 << 10)
+    print("alloc: steps that round up", flush=True)
+    g.FuseMapColor(torch.full((1, 1), 484 * 8 * voxel, device="cuda"),
+                   torch.zeros((1, 1, 3), dtype=torch.uint8, device="cuda"),
+                   torch.full((1, 1, 4), float("nan"), device="cuda"), pose, (525.0, 525.0, 0.0, 0.0))
+    assert len(g.export_blocks()) == 0 and g.stats()["flags"] == 8
