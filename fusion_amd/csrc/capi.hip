@@ -1353,7 +1353,7 @@ static fu_status run_frame_plain(fu_system* sys, const uint16_t* depth, const ui
     a.prgb = sys->fuse_rgb;
     VisArgs v = make_vis(m, dummy, t->st, p.cols, p.rows, p.fx, p.fy, p.cx, p.cy, m->p.depth_min, m->p.depth_max);
     v.after_alloc = 1;
-    launch_begin_pass(m->v, 3, s);
+    launch_begin_pass(m->v, 7, s);  // no z-range pass follows where nothing is visible
     if (fuse) {
         launch_alloc(m->v, a, false, s);
         HIPCHK(hipStreamSynchronize(s));

@@ -112,11 +112,13 @@ __device__ __forceinline__ int batch_slot(const BatchLaunch& b, int wg, WG& g) {
 }
 
 // ---- parts of a frame's passes that run inside another pass's launch ----------------------
-// per-frame counters: the new-key count (1) and the visible count (2) start at zero; one lane
+// per-frame counters: the new-key count (1), the visible count (2) and the fragment count (4) start at
+// zero; one lane
 __device__ __forceinline__ void begin_pass(unsigned* ctr, int which) {
     if (threadIdx.x == 0) {
         if (which & 1) ctr[C_NEW] = 0;
         if (which & 2) ctr[C_VISIBLE] = 0;
+        if (which & 4) ctr[C_RENDER] = 0;
     }
 }
 // the tile maps and the fragment counter at the start of a pass

@@ -62,7 +62,6 @@ void launch_grid_fill(const MapView& m, unsigned n, hipStream_t s) {
     hipLaunchKernelGGL(k_grid_fill, dim3(1024), dim3(256), 0, s, m, n);
 }
 
-// per-frame counters: the new-key count and the visible count start at zero
 __global__ void k_begin_pass(unsigned* ctr, int which) { begin_pass(ctr, which); }
 void launch_begin_pass(const MapView& m, int which, hipStream_t s) {
     hipLaunchKernelGGL(k_begin_pass, dim3(1), dim3(64), 0, s, m.ctr, which);

@@ -272,3 +272,29 @@ def test_mapping_disabled_matches_the_oracle(gpu, tmp_path):
     assert t.result()["fused"] == 0 and len(t.mapping().export_blocks()) == 0
     s.close()
     t.close()
+
+
+def test_a_frame_without_a_visible_block_counts_no_fragments(gpu):
+    """a lost system placed where it sees no block of its map: the frame's counts are its own in every
+    mode, not those of the frame rendered before it"""
+    cols, rows = 160, 120
+    sc, K, fr = scene_frames(frames=(0,), cols=cols, rows=rows)
+    mp = dict(num_buckets=1 << 14, num_excess=1 << 13, num_blocks=1 << 13, voxel_size=0.02,
+              trunc_dist=float(np.float32(0.02) * np.float32(3.0)), max_new_blocks=1 << 13)
+    away = np.eye(4)
+    away[2, 3] = 50.0
+    for mode in ("device", "graph", "plain"):
+        s = A.System(A.system_params(cols=cols, rows=rows, K=K, plain=mode == "plain", use_graph=mode == "graph", map=mp))
+        d, c = A.to_device(*fr[0])
+        s.GrabImage(d, c)
+        first = s.result()
+        assert first["n_fragments"] > 100 and first["n_visible"] > 100, mode
+        for _ in range(11):
+            s.GrabImage(torch.zeros_like(d), c)
+        s.relocalise(away)
+        s.GrabImage(d, c)
+        r = s.result()
+        print("no visible block:", mode, r["track_status"], r["n_visible"], r["n_fragments"], flush=True)
+        assert not r["fused"] and np.array_equal(r["pose"], away), mode
+        assert r["n_visible"] == 0 and r["n_fragments"] == 0, mode
+        s.close()
