@@ -114,29 +114,41 @@ __global__ void k_lift_keys(LiftArgs a) {
 
 // ---------------------------------------------------------------------------- matching
 // The two nearest train descriptors of every query descriptor by L2 distance (sqrt of the sum
-// of the 64 squared differences, in dimension order); ties go to the lower train index.
-// Few of the pairs need that exact sum.  k_match_bound prices every pair on the matrix cores
+// of the 64 squared differences, in dimension order); ties go to the lower train index.  All forms
+// keep the two smallest (distance, index) pairs in lexicographic order, a total order over the
+// candidates (NaN and +inf distances never enter), so the result is that of one lane scanning the
+// train set in index order with strict comparisons, whatever the form, the chunks and the order of
+// merges:
+//   k_match_tile  all pairs by the exact sum.  Work-group: 256 queries, one per lane (its
+//                 descriptor in registers), against a chunk of train descriptors staged through
+//                 LDS kTile at a time (every lane reads the same record: LDS broadcast); the
+//                 chunks' best two are merged by k_match_merge.  Bound by VALU issue, 192
+//                 operations a pair;
+//   k_match_scan  alone: a wave per query, a lane per train descriptor, for few of both;
+//   k_match_bound and k_match_scan, where they leave most pairs out.
+// Few of the pairs need the exact sum.  k_match_bound prices every pair on the matrix cores
 // (|t|^2 - 2 q.t, FP32) and keeps, per query and chunk of train descriptors, the least lower and
 // the least upper bound; k_match_scan, a wave per query, takes the second least upper bound and
 // evaluates the chunks whose lower bound does not exceed it, a lane per train descriptor, with
-// the sum's own operations and order.  It keeps the two smallest (distance, index) pairs in
-// lexicographic order, a total order over the candidates (NaN and +inf distances never enter), so
-// the result is that of one lane scanning the train set in index order with strict comparisons.
+// the sum's own operations and order.  How many remain depends on the descriptors: equal ones,
+// distances far below the norms and magnitudes near overflow leave most of them.  A query with
+// more than max_scan chunks left goes on a list instead, whose queries k_match_tile takes.
 //
 // The bounds.  u = 2^-24, Q = |q|^2, T = |t|^2: the price errs by at most 64 u (Q + T) (the dot
 // product, doubled, with 2 |q||t| <= Q + T) + 64 u T + 4 u (Q + 3 T) from |q - t|^2 - Q, and the
 // exact sum by 67 u |q - t|^2 <= 134 u (Q + T), its root's rounding (ties) by another 8 u (Q + T).
 // kSlack = 512 u times (2 T + Q) covers twice that; kTiny covers sums that round towards zero
-// below the normal range.  The chunk of a T that is not below kHuge (or not a number: products may
-// overflow) is always evaluated, a query with such a Q evaluates all of them.
+// below the normal range.  The chunk of a T of kHuge and more (products may overflow) is always
+// evaluated, a query with a Q that is not below it evaluates all of them; a T that is NaN is that of a
+// descriptor with a NaN, whose distances never enter.
 //
-// 900 queries against 20,000: all pairs by the exact sum, bound by VALU issue (192 operations a
-// pair), took 153 us; the two passes take 43 + 14.  The first is bound by its matrix instructions
+// 900 queries against 20,000: all pairs by the exact sum take 153 us; the two passes take 43 + 14.
+// The first is bound by its matrix instructions
 // (17 us) and the loads under them: with a quarter of the instructions it still takes 28 us.
 constexpr int kDesc = 64;
-constexpr int kChunkMin = 128, kChunkMax = 8192;  // train descriptors
+constexpr int kTile = 128;
+constexpr int kChunkMin = kTile, kChunkMax = 8192;  // train descriptors
 constexpr int kTargetGroups = 4096;
-constexpr int kScanAll = 512;  // up to so many train descriptors are all evaluated: no first pass
 constexpr float kSlack = 0x1p-15f, kTiny = 0x1p-100f, kHuge = 1e37f;
 
 struct Best2 {
@@ -171,8 +183,10 @@ typedef v4f v4f_word __attribute__((aligned(4)));  // descriptors are aligned as
 // descriptors loaded ahead, which leave registers for three (44 and 50 us); a chunk's work-groups
 // share an XCD's L2 (43 us).
 // bound[chunk * nq + query] = {lower, upper}, without the query's own share.
+// todo: the list's length, zero for the scan behind.
 __global__ __launch_bounds__(256, 4) void k_match_bound(const float* q, int nq, const float* t, int nt, int chunk,
-                                                        float2* bound) {
+                                                        float2* bound, int* todo) {
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *todo = 0;
     const int lane = threadIdx.x & 63, n = lane & 31, half = lane >> 5;
     // work-groups go to the eight XCDs in turn: each XCD takes every eighth chunk, all its queries
     const int c = blockIdx.y * 8 + (blockIdx.x & 7);
@@ -204,7 +218,7 @@ __global__ __launch_bounds__(256, 4) void k_match_bound(const float* q, int nq, 
             }
         T += __shfl_xor(T, 32);
         const bool in = base + n < c1, sane = T < kHuge;
-        bad = bad || (in && !sane);
+        bad = bad || (in && T >= kHuge);
         const float tl = in && sane ? fmaf(T, -2.f * kSlack, T) : INFINITY;
         const float th = in && sane ? fmaf(T, 2.f * kSlack, T) : INFINITY;
         // an infinite price or NaN (columns outside, or whose chunk is evaluated anyway) is no bound
@@ -255,14 +269,22 @@ __device__ __forceinline__ float exact_dist(const Q& q, FU_GPTR(const v4f_word) 
     return sqrtf(s);
 }
 
+// the queries that a scan leaves to k_match_tile, and their number (null: there is no list)
+struct Todo {
+    int* n;
+    int* list;
+};
+
 // a wave per query; without bounds (null) every chunk is evaluated
 __global__ __launch_bounds__(256) void k_match_scan(const float* q, int nq, const float* t, int nt, int chunk, int nchunks,
-                                                    const float2* bound, int* idx, float* dist) {
+                                                    const float2* bound, int max_scan, Todo todo, int* idx, float* dist) {
     const int qi = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
     const int lane = threadIdx.x & 63;
     if (qi >= nq) return;  // uniform
     typedef const __attribute__((address_space(4))) float CF;
     CF* qc = (CF*)(q + (size_t)qi * kDesc);
+    constexpr int kKeep = 4;  // of the lane's chunks the lower bounds kept, others are read again
+    unsigned long long left[kKeep];
     float limit = INFINITY;  // NaN or +inf: all chunks
     if (bound) {
         const float mine = q[(size_t)qi * kDesc + lane];
@@ -270,12 +292,19 @@ __global__ __launch_bounds__(256) void k_match_scan(const float* q, int nq, cons
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) Q += __shfl_xor(Q, off);
         // the two least upper bounds
-        float h0 = INFINITY, h1 = INFINITY;
-        for (int c = lane; c < nchunks; c += 64) {
-            const float h = bound[(size_t)c * nq + qi].y;
+        float h0 = INFINITY, h1 = INFINITY, lo[kKeep];
+        auto upper = [&](float h) {
             h1 = fminf(h1, fmaxf(h0, h));
             h0 = fminf(h0, h);
+        };
+#pragma unroll
+        for (int k = 0; k < kKeep; ++k) {
+            const int c = k * 64 + lane;
+            const float2 b = c < nchunks ? bound[(size_t)c * nq + qi] : make_float2(INFINITY, INFINITY);
+            lo[k] = b.x;
+            upper(b.y);
         }
+        for (int c = kKeep * 64 + lane; c < nchunks; c += 64) upper(bound[(size_t)c * nq + qi].y);
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) {
             const float g0 = __shfl_xor(h0, off), g1 = __shfl_xor(h1, off);
@@ -283,13 +312,29 @@ __global__ __launch_bounds__(256) void k_match_scan(const float* q, int nq, cons
             h0 = fminf(h0, g0);
         }
         limit = Q < kHuge ? h1 + 2.f * fmaf(Q, kSlack, kTiny) : INFINITY;
+        int count = 0;
+#pragma unroll
+        for (int k = 0; k < kKeep; ++k) {
+            left[k] = __ballot(k * 64 + lane < nchunks && !(lo[k] > limit));
+            count += __popcll(left[k]);
+        }
+        for (int c = kKeep * 64 + lane; c - lane < nchunks; c += 64)
+            count += __popcll(__ballot(c < nchunks && !(bound[(size_t)min(c, nchunks - 1) * nq + qi].x > limit)));
+        if (count > max_scan) {  // uniform
+            if (lane == 0) todo.list[atomicAdd(todo.n, 1)] = qi;
+            return;
+        }
     }
     Best2 b{INFINITY, INFINITY, -1, -1};
     for (int base = 0; base < nchunks; base += 64) {
         const int c = base + lane;
-        bool take = c < nchunks;
-        if (bound && take) take = !(bound[(size_t)c * nq + qi].x > limit);
-        unsigned long long m = __ballot(take);
+        unsigned long long m;
+        if (!bound)
+            m = __ballot(c < nchunks);
+        else if (base >= kKeep * 64)
+            m = __ballot(c < nchunks && !(bound[(size_t)min(c, nchunks - 1) * nq + qi].x > limit));
+        else
+            m = base == 0 ? left[0] : base == 64 ? left[1] : base == 128 ? left[2] : left[3];
         while (m) {
             const int k = base + __builtin_ctzll(m);
             m &= m - 1;
@@ -318,6 +363,66 @@ __global__ __launch_bounds__(256) void k_match_scan(const float* q, int nq, cons
     }
 }
 
+__device__ __forceinline__ void merge(Best2& b, const Best2& p) {
+    if (p.i0 >= 0) push2(b, p.d0, p.i0);
+    if (p.i1 >= 0) push2(b, p.d1, p.i1);
+}
+
+// The best two of each query in each chunk, part[chunk * nq + query]; of the queries of the list
+// (todo.n not null), in its order.  Launch: a work-group per 256 queries and chunk, of a chunk one after
+// the other, or with a list, whose first groups alone may hold queries, of a group, so that all XCDs
+// have some.
+__global__ __launch_bounds__(256) void k_match_tile(const float* q, int nq, const float* t, int nt, int chunk, int nchunks,
+                                                    Todo todo, Best2* part) {
+    __shared__ float tile[kTile * kDesc];
+    const unsigned groups = (nq + 255) / 256, id = blockIdx.x;
+    const int c = (int)(todo.n ? id % nchunks : id / groups), g = (int)(todo.n ? id / nchunks : id % groups);
+    const int at = g * 256 + threadIdx.x, total = todo.n ? *todo.n : nq;
+    if (g * 256 >= total) return;  // uniform
+    const int c0 = c * chunk, c1 = min(nt, c0 + chunk);
+    const int qi = at < total ? (todo.n ? todo.list[at] : at) : -1;
+    float mine[kDesc];
+#pragma unroll
+    for (int j = 0; j < kDesc; ++j) mine[j] = qi >= 0 ? q[(size_t)qi * kDesc + j] : 0.f;
+    Best2 b{INFINITY, INFINITY, -1, -1};
+    const bool any = __any(qi >= 0);
+    for (int base = c0; base < c1; base += kTile) {
+        const int cnt = min(kTile, c1 - base);
+        __syncthreads();
+        for (int k = threadIdx.x; k < cnt * kDesc; k += 256) tile[k] = t[(size_t)base * kDesc + k];
+        __syncthreads();
+        if (!any) continue;  // uniform in the wave, which only helps to bring the tiles
+        for (int r = 0; r < cnt; ++r) {
+            float s = 0.f;
+#pragma unroll
+            for (int j = 0; j < kDesc; ++j) {
+                const float dj = mine[j] - tile[r * kDesc + j];
+                s = s + dj * dj;
+            }
+            const float d = sqrtf(s);
+            if (d < b.d1) push2(b, d, base + r);  // indices rise within the chunk: d < d1 is the test
+        }
+    }
+    if (qi >= 0) part[(size_t)c * nq + at] = b;
+}
+// the chunks' best merged, a wave per query
+__global__ __launch_bounds__(256) void k_match_merge(const Best2* part, int nq, int nchunks, Todo todo, int* idx, float* dist) {
+    const int at = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (at >= (todo.n ? *todo.n : nq)) return;
+    Best2 b{INFINITY, INFINITY, -1, -1};
+    for (int c = lane; c < nchunks; c += 64) merge(b, part[(size_t)c * nq + at]);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1)
+        merge(b, Best2{__shfl_xor(b.d0, off), __shfl_xor(b.d1, off), __shfl_xor(b.i0, off), __shfl_xor(b.i1, off)});
+    if (lane == 0) {
+        const int qi = todo.n ? todo.list[at] : at;
+        idx[2 * qi] = b.i0;
+        idx[2 * qi + 1] = b.i1;
+        dist[2 * qi] = b.d0;
+        dist[2 * qi + 1] = b.d1;
+    }
+}
+
 // train descriptors per chunk: about kTargetGroups chunks of 256 queries in all, at least
 // kChunkMin and at most kChunkMax, a whole number of kChunkMin
 static int match_chunk_len(int nq, int nt) {
@@ -325,6 +430,30 @@ static int match_chunk_len(int nq, int nt) {
     long long want = ((long long)nt * qgroups + kTargetGroups - 1) / kTargetGroups;
     want = (want + kChunkMin - 1) / kChunkMin * kChunkMin;
     return (int)std::min<long long>(kChunkMax, std::max<long long>(kChunkMin, want));
+}
+
+// Which form a call takes, by times of all three in us (all pairs / scan alone / bounds, random unit
+// descriptors):
+//     1000 x 512     98 /  18 /  28      8000 x 256    102 /   61 /   84     16000 x 1000   132 /  438 /  156
+//     1000 x 1000    99 /  33 /  28      8000 x 512    104 /  116 /   85     20000 x 2100   271 / 1150 /  242
+//     1000 x 20000  157 /  -  /  62     16000 x 256    106 /  116 /  154     20000 x 4000   409 /    - /  290
+//     4000 x 4000   121 / 439 /  74     16000 x 20000 1285 /    - /  817    100000 x 4000  1574 /    - / 2877
+// A scan alone costs by the pair, all pairs at least 95 us, which 2^22 pairs fill; the bounds need chunks
+// to leave out, and many queries make few long ones.
+enum MatchForm : int { kAll, kScan, kBounds };
+static MatchForm match_form(int nq, int nt, int nchunks) {
+    if (nt <= 512 && nq <= 16384 && (long long)nq * nt <= 1ll << 21) return kScan;
+    return nq <= 8192 || nchunks >= 32 ? kBounds : kAll;
+}
+// The most chunks that a query's scan takes: those that take as long as the list would if every query
+// were on it.  A scan takes 3.7 us per 128 descriptors while its waves find SIMDs of their own, then
+// 4.9 ns per query; the list 95 us, then 0.67 ns per query and 128 descriptors.  Two chunks hold a
+// query's nearest, so three at least.  Equal descriptors in every chunk, of which none can be left out,
+// 900 x 20000: 590 us with every chunk scanned, now 215, where all pairs take 156; 4000 x 600: 174 and 98.
+static int match_max_scan(int nq, int chunk, int nchunks) {
+    const double scan = std::max(3.7, nq * 0.0049) * (chunk / kTile);
+    const double list = std::max(95.0, (double)nq * nchunks * (chunk / kTile) * 0.00067);
+    return std::max(3, (int)std::min(list / scan, (double)nchunks));
 }
 
 // ---------------------------------------------------------------------------- graph selection
@@ -921,20 +1050,37 @@ extern "C" fu_status fu_match_knn2(const float* query, int32_t nq, const float* 
     hipStream_t hs = (hipStream_t)s;
     const int chunk = match_chunk_len(nq, nt);
     const int nchunks = (nt + chunk - 1) / chunk;
-    float2* bound = nullptr;
-    if (nt > kScanAll) {
-        if (hipMallocAsync((void**)&bound, sizeof(float2) * (size_t)nchunks * nq, hs) != hipSuccess) {
-            (void)hipGetLastError();
-            return api_error(FU_ERR_NOMEM, "fu_match_knn2: %d partial lists", nchunks);
-        }
-        hipLaunchKernelGGL(k_match_bound, dim3((nq + 127) / 128 * 8, (nchunks + 7) / 8), dim3(256), 0, hs, query, nq, train, nt,
-                           chunk, bound);
+    const MatchForm form = match_form(nq, nt, nchunks);
+    const int max_scan = match_max_scan(nq, chunk, nchunks);
+    // every chunk's best two of every query (the bounds, read before any of them is written, lie in the
+    // same place), then the list
+    char* scratch = nullptr;
+    const size_t parts = sizeof(Best2) * (size_t)nchunks * nq, ints = form == kBounds ? 1 + (size_t)nq : 0;
+    if (form != kScan && hipMallocAsync((void**)&scratch, parts + sizeof(int) * ints, hs) != hipSuccess) {
+        (void)hipGetLastError();
+        return api_error(FU_ERR_NOMEM, "fu_match_knn2: %d partial lists", nchunks);
     }
-    hipLaunchKernelGGL(k_match_scan, dim3((nq + 3) / 4), dim3(256), 0, hs, query, nq, train, nt, chunk, nchunks, bound,
-                       idx, dist);
+    Best2* part = reinterpret_cast<Best2*>(scratch);
+    float2* bound = nullptr;
+    Todo todo{nullptr, nullptr};
+    if (form == kBounds) {
+        bound = reinterpret_cast<float2*>(scratch);
+        todo.n = reinterpret_cast<int*>(scratch + parts);
+        todo.list = todo.n + 1;
+        hipLaunchKernelGGL(k_match_bound, dim3((nq + 127) / 128 * 8, (nchunks + 7) / 8), dim3(256), 0, hs, query, nq, train, nt,
+                           chunk, bound, todo.n);
+    }
+    if (form != kAll)
+        hipLaunchKernelGGL(k_match_scan, dim3((nq + 3) / 4), dim3(256), 0, hs, query, nq, train, nt, chunk, nchunks, bound,
+                           max_scan, todo, idx, dist);
+    if (form == kAll || (form == kBounds && nchunks > max_scan)) {
+        hipLaunchKernelGGL(k_match_tile, dim3((unsigned)((nq + 255) / 256) * nchunks), dim3(256), 0, hs, query, nq, train, nt,
+                           chunk, nchunks, todo, part);
+        hipLaunchKernelGGL(k_match_merge, dim3((nq + 3) / 4), dim3(256), 0, hs, part, nq, nchunks, todo, idx, dist);
+    }
     hipError_t e = hipGetLastError();
-    if (bound) {
-        const hipError_t ef = hipFreeAsync(bound, hs);
+    if (scratch) {
+        const hipError_t ef = hipFreeAsync(scratch, hs);
         if (e == hipSuccess) e = ef;
     }
     if (e != hipSuccess) return api_error(FU_ERR_HIP, "fu_match_knn2: %s", hipGetErrorString(e));

@@ -50,6 +50,24 @@ def test_match_forms_exact(gpu, kind, nq, nt):
     assert np.array_equal(dist.cpu().numpy().view(np.uint32), do.view(np.uint32))
 
 
+@pytest.mark.parametrize("kind", ["unit", "few", "holes"])
+@pytest.mark.parametrize("nq,nt", [(8193, 600), (16385, 3), (16384, 128), (8193, 4096), (300, 4200), (40, 33100)])
+def test_match_dispatch_exact(gpu, kind, nq, nt):
+    """both sides of the dispatch's lines, and queries left to the list of those that have too many
+    chunks to scan: some of them, and more than a wave keeps the bounds of"""
+    print("match dispatch", kind, nq, nt, flush=True)
+    q, t = _descriptors("unit" if kind == "few" else kind, nq, nt)
+    if kind == "few":  # zeros in every chunk, and queries that are zero among others
+        t[::3] = 0
+        q[::7] = 0
+    idx, dist = A.match_knn2(torch.from_numpy(q).cuda(), torch.from_numpy(t).cuda())
+    some = np.unique(np.concatenate([np.arange(min(nq, 300)), np.arange(max(0, nq - 100), nq)]))
+    io, do = O.match_knn2(np.ascontiguousarray(q[some]), t)
+    assert np.array_equal(idx.cpu().numpy()[some], io)
+    assert np.array_equal(dist.cpu().numpy()[some].view(np.uint32), do.view(np.uint32))
+    assert int(idx.min()) >= -1 and int(idx.max()) < nt
+
+
 def _key_map(nk, max_keys, n_buckets, seed):
     rng = np.random.default_rng(seed)
     keys = np.zeros(nk, A.SURF_DTYPE)
