@@ -627,37 +627,52 @@ __global__ __launch_bounds__(kSelLanes) void k_select(SelArgs a) {
     if (tid == 0) a.n_selected[i] = count;
 }
 
-// launch: (ceil((max_sel - 1) / 4), lists) work-groups of 256 lanes.  The work-group that ends last
-// of a list's (counted in its n_refined, the marks written through to the memory that all XCDs
-// share) moves the marked pairs together.
+// launch: (work-groups per list, lists) of 256 lanes, a wave per pair: as many per list as it has pairs
+// in fours, up to kRefineGroups in all; beyond that, with kStage, about kStagedGroups, four per list at
+// least, whose waves take several pairs and have the list and its scores with the head in LDS (their
+// gathers from C meet in the caches, which more waves at once overrun).  200 lists of 1024 of 3000 pairs:
+// 962 us with a wave per pair, 842 with 4096 groups, now 690; 10 lists of 400: 73.
+// The work-group that ends last of a list's (counted in its n_refined, the marks written through to the
+// memory that all XCDs share) moves the marked pairs together.
+constexpr int kRefineGroups = 4096, kStagedGroups = 800;
 constexpr int kMark = (int)0x80000000u;  // pair indices are below 46340
+template <bool kStage>
 __global__ __launch_bounds__(256) void k_refine(SelArgs a) {
     __shared__ int last, wsum[4];
-    const int i = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    __shared__ int staged[kStage ? kMaxSelect : 1];
+    __shared__ float score[kStage ? kMaxSelect : 1];
+    const int i = blockIdx.y, x = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const int count = a.n_selected[i];
     if (count < 3) return;  // no PoseEstimate from fewer than three (:565)
-    const int groups = (count + 2) / 4;
-    if ((int)blockIdx.x >= groups) return;
+    const int groups = min((count + 2) / 4, (int)gridDim.x);
+    if (x >= groups) return;
     int* sel = a.refined + (size_t)i * a.max_sel;
     const float* Ch = a.C + (size_t)(sel[0] & ~kMark) * a.n;
+    if constexpr (kStage) {
+        for (int l = tid; l < count; l += 256) {
+            const int b = sel[l] & ~kMark;
+            staged[l] = b;
+            score[l] = Ch[b];
+        }
+        __syncthreads();
+    }
     // the t-th pair is kept unless a later one is nearly exclusive with it and scores higher
     // with the head (:567-582); the head (t = 0) is never kept
-    const int t = 1 + blockIdx.x * 4 + wid;
-    if (t < count) {
-        const int av = sel[t] & ~kMark;
-        const float ha = Ch[av];
+    for (int t = 1 + x * 4 + wid; t < count; t += groups * 4) {
+        const int av = kStage ? staged[t] : sel[t] & ~kMark;
+        const float ha = kStage ? score[t] : Ch[av];
         const float* Ca = a.C + (size_t)av * a.n;
         bool drop = false;
 #pragma unroll 4
         for (int l = t + 1 + lane; l < count; l += 64) {
-            const int b = sel[l] & ~kMark;
+            const int b = kStage ? staged[l] : sel[l] & ~kMark;
             const bool x = Ca[b] < 5e-3f || a.C[(size_t)b * a.n + av] < 5e-3f;
-            drop = drop || (Ch[b] > ha && x);
+            drop = drop || ((kStage ? score[l] : Ch[b]) > ha && x);
         }
         if (__ballot(drop) == 0ull && lane == 0)
             __hip_atomic_store(FU_G(int, sel + t), av | kMark, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the wave's mark is in place
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the wave's marks are in place
     __syncthreads();
     if (tid == 0)
         last = __hip_atomic_fetch_add(FU_G(int, a.n_refined + i), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == groups - 1;
@@ -1381,7 +1396,15 @@ extern "C" fu_status fu_select_subgraphs(const float* matrix, int32_t n, int32_t
     }
     const SelArgs a{matrix, order, n, max_select, min_score, n_selected, n_refined, refined};
     hipLaunchKernelGGL(k_select, dim3(n_lists), dim3(kSelLanes), 0, hs, a);
-    if (n > 0 && max_select > 1) hipLaunchKernelGGL(k_refine, dim3((max_select + 2) / 4, n_lists), dim3(256), 0, hs, a);
+    const int longest = std::min(max_select, n);
+    if (longest > 2) {  // no list of fewer is refined
+        const int fours = (longest + 2) / 4;
+        if ((long long)fours * n_lists <= kRefineGroups)
+            hipLaunchKernelGGL(k_refine<false>, dim3(fours, n_lists), dim3(256), 0, hs, a);
+        else
+            hipLaunchKernelGGL(k_refine<true>, dim3(std::min(fours, std::max(4, kStagedGroups / n_lists)), n_lists), dim3(256), 0,
+                               hs, a);
+    }
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return api_error(FU_ERR_HIP, "fu_select_subgraphs: %s", hipGetErrorString(e));
     return FU_OK;

@@ -144,3 +144,18 @@ def test_selection_forms(gpu, n, max_sel):
     assert np.array_equal(g[0], o[0])
     for a, b in zip(g[1], o[1]):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("n,max_sel,lists", [(1, 4, 3), (5, 1024, 4200), (70, 64, 300), (1100, 1024, 40), (300, 130, 125)])
+def test_selection_of_many_lists(gpu, n, max_sel, lists):
+    # more lists than a wave per pair is launched for: waves that take several pairs, lists that ranks end
+    rng = np.random.default_rng(n + lists)
+    C = (0.2 + 0.8 * rng.random((n, n))).astype(np.float32)
+    C[rng.random((n, n)) < 2.0 / n] = 0.0
+    print("select", n, max_sel, lists, flush=True)
+    g = A.select_subgraphs(torch.from_numpy(C).cuda(), lists, max_sel, 0.1)
+    o = O.graph_select(C, lists, max_sel, 0.1)
+    assert np.array_equal(g[0], o[0])
+    assert len(g[1]) == len(o[1]) == lists
+    for a, b in zip(g[1], o[1]):
+        assert np.array_equal(a, b)
