@@ -401,35 +401,42 @@ __global__ __launch_bounds__(256) void k_pyrdown_u8(const unsigned char* __restr
 // ComputeDerivativeImageKernel (Pyrdown.cu:210-236): 3x3 Sobel over the window clipped to
 // the image, the weight index counting down from 8 across the clipped window (at the border
 // the weights shift), float sums stored as shorts
-__constant__ int c_sobel_x[9] = {1, 0, -1, 2, 0, -2, 1, 0, -1};
-__constant__ int c_sobel_y[9] = {1, 2, 1, 0, 0, 0, -1, -2, -1};
+__constant__ float c_sobel_x[9] = {1, 0, -1, 2, 0, -2, 1, 0, -1};
+__constant__ float c_sobel_y[9] = {1, 2, 1, 0, 0, 0, -1, -2, -1};
 __device__ __forceinline__ void derivative_body(WG g, const unsigned char* __restrict__ img_, short* __restrict__ dx_,
                                                 short* __restrict__ dy_, int cols, int rows) {
     const int x = g.x * 16 + (threadIdx.x & 15);
     const int y = g.y * 16 + (threadIdx.x >> 4);
     if (x >= cols || y >= rows) return;
     const auto img = FU_G(const unsigned char, img_);
-    int a = 0, b = 0;  // the float sums are of small integers: exact
-    if (x >= 1 && y >= 1 && x + 2 < cols && y + 1 < rows) {
-        // the whole 3x3 window, a 4-byte load per row (its last byte not used)
+    float a = 0.f, b = 0.f;
+    if (x >= 1 && y >= 1 && x + 1 < cols && y + 1 < rows) {
+        // the whole 3x3 window: its nine loads issue together, the same products and sums in
+        // the same order as the clipped loop below (k = 8 .. 0)
+        constexpr float sx[9] = {1, 0, -1, 2, 0, -2, 1, 0, -1};
+        constexpr float sy[9] = {1, 2, 1, 0, 0, 0, -1, -2, -1};
         const auto p = img + (y - 1) * cols + (x - 1);
-        const unsigned r0 = load4(p), r1 = load4(p + cols), r2 = load4(p + 2 * cols);
-        auto at = [](unsigned r, int k) { return (int)((r >> (8 * k)) & 255u); };
-        a = (at(r0, 2) - at(r0, 0)) + 2 * (at(r1, 2) - at(r1, 0)) + (at(r2, 2) - at(r2, 0));
-        b = (at(r2, 0) + 2 * at(r2, 1) + at(r2, 2)) - (at(r0, 0) + 2 * at(r0, 1) + at(r0, 2));
+        float v[9];
+#pragma unroll
+        for (int q = 0; q < 9; ++q) v[q] = (float)p[(q / 3) * cols + q % 3];
+#pragma unroll
+        for (int q = 0; q < 9; ++q) {
+            a += v[q] * sx[8 - q];
+            b += v[q] * sy[8 - q];
+        }
     } else {
         int k = 8;
         for (int j = max(y - 1, 0); j <= min(y + 1, rows - 1); ++j) {
             for (int i = max(x - 1, 0); i <= min(x + 1, cols - 1); ++i) {
-                const int v = img[j * cols + i];
+                const float v = (float)img[j * cols + i];
                 a += v * c_sobel_x[k];
                 b += v * c_sobel_y[k];
                 --k;
             }
         }
     }
-    FU_G(short, dx_)[y * cols + x] = (short)a;
-    FU_G(short, dy_)[y * cols + x] = (short)b;
+    FU_G(short, dx_)[y * cols + x] = (short)f2i(a);
+    FU_G(short, dy_)[y * cols + x] = (short)f2i(b);
 }
 __global__ __launch_bounds__(256) void k_derivative(const unsigned char* __restrict__ img, short* __restrict__ dx,
                                                    short* __restrict__ dy, int cols, int rows) {
