@@ -107,10 +107,16 @@ extern "C" void fu_map_params_default(fu_map_params* p) {
     p->max_new_blocks = 1u << 18;
 }
 
-// cells per axis of the block grid: 2^7 (16 MB) covers a camera's surroundings (5 m at 5 mm
+// cells per axis of the block grid's first part: 2^7 (16 MB) covers a camera's surroundings (5 m at 5 mm
 // voxels) without two blocks in a cell; maps of few blocks take less
 static unsigned grid_bits(const fu_map_params* p) { return p->num_blocks > (1u << 14) ? 7 : p->num_blocks > (1u << 11) ? 6 : 5; }
-static size_t grid_cells(const fu_map_params* p) { return (size_t)1 << (3 * grid_bits(p)); }
+// cells of the second: as many (a cell and the tag give the block), or 8 for each block of the pool
+static size_t far_cells(const fu_map_params* p) {
+    size_t n = (size_t)1 << (3 * grid_bits(p));
+    while (n < 8ull * p->num_blocks) n <<= 1;
+    return n;
+}
+static size_t grid_cells(const fu_map_params* p) { return ((size_t)1 << (3 * grid_bits(p))) + far_cells(p); }
 
 static unsigned newset_size(const fu_map_params* p) {
     unsigned n = 1024;
@@ -188,6 +194,7 @@ extern "C" fu_status fu_map_create(const fu_map_params* p, fu_map** out) {
     v.num_blocks = p->num_blocks;
     v.newset_mask = ns - 1;
     v.grid_bits = grid_bits(p);
+    v.far_mask = (unsigned)(far_cells(p) - 1);
     v.bucket_mask = (p->num_buckets & (p->num_buckets - 1)) == 0 ? p->num_buckets - 1 : 0u;
     v.max_new = p->max_new_blocks;
     v.max_weight = p->max_weight;

@@ -74,8 +74,9 @@ struct MapView {
     unsigned long long* newkeys;  // [max_new]
     unsigned* newslot;          // [max_new]
     unsigned char* pool;        // voxel blocks
-    uint2* grid;                // block grid: (pool index, tag) by the low coordinate bits, see grid_find
-    unsigned grid_bits;         // 2^grid_bits cells per axis
+    uint2* grid;                // block grid: (pool index, tag) of a block in its cell, see find_block
+    unsigned grid_bits;         // 2^grid_bits cells per axis in its first part
+    unsigned far_mask;          // cells of its second part - 1
     unsigned bucket_mask;       // num_buckets - 1 when it is a power of two, else 0
     unsigned num_buckets, num_excess, num_blocks, newset_mask, max_new;
     unsigned max_weight;
@@ -167,15 +168,18 @@ FU_HD unsigned long long mix64(unsigned long long k) {
 }
 
 // ---- block grid --------------------------------------------------------------------------
-// A direct-mapped table of the allocated blocks by the low grid_bits of each block coordinate,
-// beside the hash table: a cell holds the pool index and the ten coordinate bits per axis above
-// those of the first block allocated in it (blocks are never freed between resets).  A lookup is
-// one 8-byte load: an empty cell proves that no block of its congruence class is allocated, an
-// equal tag gives the block, and only another block in the cell (one a whole grid away: 5 m at
-// 5 mm voxels and 2^7 cells) sends the lookup to the hash table, as do coordinates outside
-// +-2^(grid_bits + 9).  Neighbouring blocks along x share cache lines, and the index and tag are
-// shifts where the hash takes three 32-bit multiplications; the rays' and samples' lookups had
-// cost an occupancy bitmap load and then the hash entry's.
+// A direct-mapped table of the allocated blocks by the low grid_bits of each block coordinate, beside
+// the hash table: a cell holds the pool index and the ten coordinate bits per axis above those (the
+// block's period) of the first block allocated in it (blocks are never freed between resets).  A lookup
+// is one 8-byte load: an empty cell proves that no block of its congruence class is allocated and an
+// equal tag gives the block.  Surroundings of a period (5 m at 5 mm voxels and 2^7 cells) have a cell
+// for each of their blocks; of a wider map, floors and walls share theirs with what lies whole periods
+// away.  A block whose cell is taken goes to a second part, by the same bits folded with its period, 8
+// cells or more for each block of the pool, where the same holds; only one whose cell is taken there
+// too sends its lookup to the hash table, as do coordinates outside +-2^(grid_bits + 9).  Neighbouring
+// blocks along x share cache lines, and the index and tag are shifts where the hash takes three 32-bit
+// multiplications; the rays' and samples' lookups had cost an occupancy bitmap load and then the hash
+// entry's.
 constexpr unsigned kNoBlock = 0xFFFFFFFFu;  // pool index and tag of an empty cell
 FU_HD bool in_grid(const MapView& m, i3 b) {
     const unsigned half = 512u << m.grid_bits;
@@ -190,11 +194,21 @@ FU_HD unsigned grid_tag(const MapView& m, int c, int axis) {
 }
 FU_HD unsigned grid_index(const MapView& m, i3 b) { return grid_cell(m, b.x, 0) | grid_cell(m, b.y, 1) | grid_cell(m, b.z, 2); }
 FU_HD unsigned grid_tag3(const MapView& m, i3 b) { return grid_tag(m, b.x, 0) | grid_tag(m, b.y, 1) | grid_tag(m, b.z, 2); }
-// enters block bp (pool index heap) unless its cell is taken; atomic against other inserts
+// the parts of a coordinate's second cell, which is their sum modulo that part's cells; the factors are
+// multiples of a cache line's 16 cells
+FU_HD unsigned far_cell(const MapView& m, int c, int axis) {
+    return grid_cell(m, c, axis) + (((unsigned)c >> m.grid_bits) & 1023u) * (axis == 0 ? 0x9E3770u : axis == 1 ? 0x85EBD0u : 0xC2B2B0u);
+}
+FU_HD uint2* far_grid(const MapView& m) { return m.grid + (1u << (3 * m.grid_bits)); }
+FU_HD unsigned far_index(const MapView& m, i3 b) {
+    return (far_cell(m, b.x, 0) + far_cell(m, b.y, 1) + far_cell(m, b.z, 2)) & m.far_mask;
+}
+// enters block bp (pool index heap) unless its cells are taken; atomic against other inserts
 __device__ __forceinline__ void grid_insert(const MapView& m, i3 bp, unsigned heap) {
     if (!in_grid(m, bp)) return;
     const unsigned long long e = (unsigned long long)heap | ((unsigned long long)grid_tag3(m, bp) << 32);
-    atomicCAS(reinterpret_cast<unsigned long long*>(m.grid + grid_index(m, bp)), ~0ull, e);
+    if (atomicCAS(reinterpret_cast<unsigned long long*>(m.grid + grid_index(m, bp)), ~0ull, e) != ~0ull)
+        atomicCAS(reinterpret_cast<unsigned long long*>(far_grid(m) + far_index(m, bp)), ~0ull, e);
 }
 
 // heap index of block `bp` by the hash table, or -1 if it is not allocated
@@ -213,6 +227,8 @@ __device__ __forceinline__ int find_block(const MapView& m, i3 bp) {
     if (in_grid(m, bp)) {
         const uint2 e = FU_G(const uint2, m.grid)[grid_index(m, bp)];
         if (e.y == grid_tag3(m, bp) || e.x == kNoBlock) return (int)e.x;
+        const uint2 f = FU_G(const uint2, far_grid(m))[far_index(m, bp)];
+        if (f.y == grid_tag3(m, bp) || f.x == kNoBlock) return (int)f.x;
     }
     return hash_find(m, bp);
 }

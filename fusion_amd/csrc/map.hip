@@ -49,7 +49,7 @@ void launch_reset_map(const MapView& m, hipStream_t s) {
     hipLaunchKernelGGL(k_fill_u64, dim3(1024), dim3(256), 0, s, m.block_key, kEmptyKey, m.num_blocks);
     hipLaunchKernelGGL(k_fill_u64, dim3(1024), dim3(256), 0, s, m.newset, kEmptyKey, m.newset_mask + 1);
     hipLaunchKernelGGL(k_fill_u64, dim3(1024), dim3(256), 0, s, reinterpret_cast<unsigned long long*>(m.grid), ~0ull,
-                       1u << (3 * m.grid_bits));
+                       (1u << (3 * m.grid_bits)) + m.far_mask + 1);
     hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, s, m.ctr, (unsigned)C_COUNT);
 }
 
