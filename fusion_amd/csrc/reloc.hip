@@ -368,12 +368,21 @@ __device__ __forceinline__ void merge(Best2& b, const Best2& p) {
     if (p.i1 >= 0) push2(b, p.d1, p.i1);
 }
 
+// A chunk's best two as the merge reads them: the indices count from the chunk's first descriptor, 16 bits
+// each, kNone where there is none.  12 bytes: an allocation of 2 MB and more takes the stream's pool 45 us
+// longer, and 900 queries against 20,000 stay below with these.
+struct PartBest {
+    float d0, d1;
+    unsigned i;
+};
+constexpr int kNone = 0xFFFF;
+static_assert(kChunkMax <= kNone && sizeof(PartBest) >= sizeof(float2), "indices in a chunk; the bounds' place");
 // The best two of each query in each chunk, part[chunk * nq + query]; of the queries of the list
 // (todo.n not null), in its order.  Launch: a work-group per 256 queries and chunk, of a chunk one after
 // the other, or with a list, whose first groups alone may hold queries, of a group, so that all XCDs
 // have some.
 __global__ __launch_bounds__(256) void k_match_tile(const float* q, int nq, const float* t, int nt, int chunk, int nchunks,
-                                                    Todo todo, Best2* part) {
+                                                    Todo todo, PartBest* part) {
     __shared__ float tile[kTile * kDesc];
     const unsigned groups = (nq + 255) / 256, id = blockIdx.x;
     const int c = (int)(todo.n ? id % nchunks : id / groups), g = (int)(todo.n ? id / nchunks : id % groups);
@@ -403,14 +412,21 @@ __global__ __launch_bounds__(256) void k_match_tile(const float* q, int nq, cons
             if (d < b.d1) push2(b, d, base + r);  // indices rise within the chunk: d < d1 is the test
         }
     }
-    if (qi >= 0) part[(size_t)c * nq + at] = b;
+    if (qi >= 0)
+        part[(size_t)c * nq + at] = PartBest{b.d0, b.d1, (unsigned)(b.i0 >= 0 ? b.i0 - c0 : kNone) |
+                                                             (unsigned)(b.i1 >= 0 ? b.i1 - c0 : kNone) << 16};
 }
 // the chunks' best merged, a wave per query
-__global__ __launch_bounds__(256) void k_match_merge(const Best2* part, int nq, int nchunks, Todo todo, int* idx, float* dist) {
+__global__ __launch_bounds__(256) void k_match_merge(const PartBest* part, int nq, int chunk, int nchunks, Todo todo,
+                                                     int* idx, float* dist) {
     const int at = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (at >= (todo.n ? *todo.n : nq)) return;
     Best2 b{INFINITY, INFINITY, -1, -1};
-    for (int c = lane; c < nchunks; c += 64) merge(b, part[(size_t)c * nq + at]);
+    for (int c = lane; c < nchunks; c += 64) {
+        const PartBest p = part[(size_t)c * nq + at];
+        const int i0 = (int)(p.i & 0xFFFFu), i1 = (int)(p.i >> 16);
+        merge(b, Best2{p.d0, p.d1, i0 == kNone ? -1 : c * chunk + i0, i1 == kNone ? -1 : c * chunk + i1});
+    }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1)
         merge(b, Best2{__shfl_xor(b.d0, off), __shfl_xor(b.d1, off), __shfl_xor(b.i0, off), __shfl_xor(b.i1, off)});
@@ -1070,12 +1086,12 @@ extern "C" fu_status fu_match_knn2(const float* query, int32_t nq, const float* 
     // every chunk's best two of every query (the bounds, read before any of them is written, lie in the
     // same place), then the list
     char* scratch = nullptr;
-    const size_t parts = sizeof(Best2) * (size_t)nchunks * nq, ints = form == kBounds ? 1 + (size_t)nq : 0;
+    const size_t parts = sizeof(PartBest) * (size_t)nchunks * nq, ints = form == kBounds ? 1 + (size_t)nq : 0;
     if (form != kScan && hipMallocAsync((void**)&scratch, parts + sizeof(int) * ints, hs) != hipSuccess) {
         (void)hipGetLastError();
         return api_error(FU_ERR_NOMEM, "fu_match_knn2: %d partial lists", nchunks);
     }
-    Best2* part = reinterpret_cast<Best2*>(scratch);
+    PartBest* part = reinterpret_cast<PartBest*>(scratch);
     float2* bound = nullptr;
     Todo todo{nullptr, nullptr};
     if (form == kBounds) {
@@ -1091,7 +1107,7 @@ extern "C" fu_status fu_match_knn2(const float* query, int32_t nq, const float* 
     if (form == kAll || (form == kBounds && nchunks > max_scan)) {
         hipLaunchKernelGGL(k_match_tile, dim3((unsigned)((nq + 255) / 256) * nchunks), dim3(256), 0, hs, query, nq, train, nt,
                            chunk, nchunks, todo, part);
-        hipLaunchKernelGGL(k_match_merge, dim3((nq + 3) / 4), dim3(256), 0, hs, part, nq, nchunks, todo, idx, dist);
+        hipLaunchKernelGGL(k_match_merge, dim3((nq + 3) / 4), dim3(256), 0, hs, part, nq, chunk, nchunks, todo, idx, dist);
     }
     hipError_t e = hipGetLastError();
     if (scratch) {
