@@ -78,7 +78,7 @@ def _plane_maps(cols, rows, K, n=(0.1, -0.2, -1.0), c=-2.0, seed=0):
 
 def test_icp_step_sums_chunk_loop(gpu):
     """a frame of more pixels than 4096 work-groups of two pixels per lane cover (8.6M) takes
-    the per-lane chunk loop with compensated sums (k_icp<false>); its sums match FP64 and the
+    the per-lane chunk loop with compensated sums (k_icp_step<kLoop>); its sums match FP64 and the
     correspondence count is exact"""
     cols, rows = 4096, 2112
     K = (2000.0, 2000.0, cols / 2 - 0.5, rows / 2 - 0.5)
