@@ -634,8 +634,8 @@ def rooflines(st, sizes, nsess):
     # u8 weight/rgb layout), the visible id and block key (16 B), depth, normal and colour of
     # the frame read once (4 + 16 + 3 B per pixel)
     b_int = per_step * (nvis * 512 * 2 * 8 + nvis * 16 + px * (4 + 16 + 3))
-    # raycast: lower bound of W*H*32 B written (vertex + normal) plus each visible block's
-    # sdf and weight planes read once (8 B per voxel)
+    # raycast: W*H*32 B written (vertex + normal) plus each visible block's sdf and weight
+    # planes read once (8 B per voxel); counted whole, though rays read the voxels near the surface
     b_rc = per_step * (px * 32 + nvis * 512 * 8)
     # ICP: 52 B per pixel-iteration (current depth, from which the vertex is made, and normal, last
     # vertex+normal)

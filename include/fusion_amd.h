@@ -553,8 +553,8 @@ fu_status fu_system_get_stage_times(fu_system* sys, fu_stage_times* out);
 
 /* ---- batched ICP of many frame pairs ------------------------------------------------------
  * Tracker::ComputeSE3 (Tracking/Tracking.cc:296-409) for n trackers at once: levels coarse to
- * fine, every iteration one reduction launch and one solve launch covering up to
- * FU_MAX_BATCH trackers (larger n runs in groups).  Each tracker's pyramids have its own size
+ * fine, every iteration one launch covering up to FU_MAX_BATCH trackers (two where they have more
+ * than 4,096 chunks of 2,048 pixels; larger n runs in groups).  Each tracker's pyramids have its own size
  * (the tracker's cols x rows); K holds fx, fy, cx, cy of each pair's level 0.  Results are
  * those of fu_compute_se3 on each tracker alone (fu_tracker_result); asynchronous on `s`.
  * No reference counterpart for the batching itself. */
